@@ -44,7 +44,8 @@
 #define RL_SG_NF 32   // frequencies
 #define RL_SG_H 256   // hidden width
 #define RL_SG_OUT 2
-#define RL_SG_MAX_SPLIT 64  // split-K slices of the weight-gradient GEMMs (>= column-sum slices / 256 * 256)
+#define RL_SG_GROUP_RAYS 262144  // training rays drawn and marched in one launch (rl_surrogate_train)
+#define RL_SG_MAX_SPLIT 64  // slices of rows that the weight gradients are summed in
 #define RL_SG_NPARAM (RL_SG_H * RL_SG_F + RL_SG_H + 2 * (RL_SG_H * RL_SG_H + RL_SG_H) + RL_SG_OUT * RL_SG_H + RL_SG_OUT)
 
 typedef uint16_t bf16_t;
@@ -80,8 +81,8 @@ static_assert(SgLayout::N == RL_SG_NPARAM, "surrogate parameter layout");
 // ---------------------------------------------------------------------------
 // GEMM: C(m, n) = sum_k A(m, k) * B(k, n), bf16 operands, fp32 accumulation.
 // A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn] (any
-// transposition).  Epilogue: + bias[n], relu, zero where mask(m, n) <= 0 (a
-// bf16 matrix with the output's strides), then store fp32 and/or bf16.
+// transposition).  Epilogue: + bias[n], relu, then store fp32 and/or bf16.
+// Serves the per-layer forward pass (the heads) and the GEMM hooks.
 // Tile 64 x 64 per 256-thread workgroup, each wave 32 x 32 (2 x 2 MFMA tiles
 // of 16 x 16), k in steps of 32 through LDS.
 struct GemmArgs {
@@ -92,14 +93,9 @@ struct GemmArgs {
   int M, N, K;
   const float* bias;
   int relu;
-  const bf16_t* mask;
   float* C;       // optional fp32 output, C[m * scm + n * scn]
   bf16_t* Cb;     // optional bf16 output, same strides
   long long scm, scn;
-  // split-K (gridDim.z > 1): slice z sums k in [z * kchunk, (z + 1) * kchunk)
-  // and stores its fp32 partial at C + z * scz (no epilogue; see k_sg_reduce)
-  int kchunk;
-  long long scz;
 };
 
 typedef short sg_short4 __attribute__((ext_vector_type(4)));
@@ -111,25 +107,19 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const bool split = gridDim.z > 1;
-  const int kbeg = split ? (int)blockIdx.z * g.kchunk : 0;
-  const int kend = split ? min(g.K, kbeg + g.kchunk) : g.K;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   sg_float4 acc[2][2];
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) acc[i][j] = sg_float4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kbeg; k0 < kend; k0 += 32) {
+  for (int k0 = 0; k0 < g.K; k0 += 32) {
     // stage A (64 x 32) and B (32 x 64): 2048 elements each, 8 per thread.
-    // (Taking neighbouring m per thread when A is m-contiguous, as in the
-    // weight-gradient GEMMs, made training 6% slower: 0.967 vs 0.910 s; 4%
-    // slower when limited to the 256-row ones.)
     for (int e = tid; e < 64 * 32; e += 256) {
       int r = e >> 5, c = e & 31;
       int m = m0 + r, k = k0 + c;
-      As[r][c] = (m < g.M && k < kend) ? g.A[(long long)m * g.sam + (long long)k * g.sak] : (bf16_t)0;
+      As[r][c] = (m < g.M && k < g.K) ? g.A[(long long)m * g.sam + (long long)k * g.sak] : (bf16_t)0;
       int kr = e >> 6, nc = e & 63;
       int kk = k0 + kr, n = n0 + nc;
-      Bs[kr][nc] = (kk < kend && n < g.N) ? g.B[(long long)kk * g.sbk + (long long)n * g.sbn] : (bf16_t)0;
+      Bs[kr][nc] = (kk < g.K && n < g.N) ? g.B[(long long)kk * g.sbk + (long long)n * g.sbn] : (bf16_t)0;
     }
     __syncthreads();
     for (int ks = 0; ks < 32; ks += 16) {
@@ -158,14 +148,9 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
         int n = n0 + wn + j * 16 + (lane & 15);
         if (m >= g.M || n >= g.N) continue;
         float v = acc[i][j][q];
-        if (split) {
-          g.C[(long long)blockIdx.z * g.scz + (long long)m * g.scm + (long long)n * g.scn] = v;
-          continue;
-        }
         if (g.bias) v += g.bias[n];
         if (g.relu && v < 0.0f) v = 0.0f;
         long long o = (long long)m * g.scm + (long long)n * g.scn;
-        if (g.mask && !(bf2f(g.mask[o]) > 0.0f)) v = 0.0f;
         if (g.C) g.C[o] = v;
         if (g.Cb) g.Cb[o] = f2bf(v);
       }
@@ -416,86 +401,7 @@ __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ 
   }
 }
 
-// Output gradient and per-block loss partial sums.  out: n x 2 fp32.
-__global__ void k_sg_loss(const float* __restrict__ out, const float* __restrict__ target, float max_range,
-                          float inv_n, bf16_t* __restrict__ dout, float* __restrict__ grad_f32,
-                          float* __restrict__ partial, int n) {
-  __shared__ float red[256];
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.0f;
-  if (i < n) {
-    const float tau = 0.95f;
-    float pred = max_range * out[2 * i];
-    float e = pred - target[i];
-    float ae = fabsf(e);
-    float lr = ae <= 1.0f ? 0.5f * e * e : ae - 0.5f;
-    float ge = ae <= 1.0f ? e : (e > 0.0f ? 1.0f : -1.0f);
-    float lb0 = out[2 * i + 1];
-    float lb = lb0 > 20.0f ? 20.0f : (lb0 < -20.0f ? -20.0f : lb0);
-    float b = expf(lb);
-    float lq = ae > b ? tau * (ae - b) : (1.0f - tau) * (b - ae);
-    float gb = lb == lb0 ? (ae > b ? -tau : (1.0f - tau)) * b : 0.0f;
-    l = lr + 0.1f * lq;
-    float g0 = ge * max_range * inv_n, g1 = 0.1f * gb * inv_n;
-    dout[2 * i] = f2bf(g0);
-    dout[2 * i + 1] = f2bf(g1);
-    if (grad_f32) {
-      grad_f32[2 * i] = g0;
-      grad_f32[2 * i + 1] = g1;
-    }
-  }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0] * inv_n;
-}
-
-// Column sums of D (rows x cols, bf16 row-major) over row chunk blockIdx.y of
-// `chunk` rows: part[blockIdx.y * cols + c].  One thread per column.
-__global__ void k_sg_colsum(const bf16_t* __restrict__ D, int rows, int cols, int chunk,
-                            float* __restrict__ part) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  int r0 = blockIdx.y * chunk, r1 = min(rows, r0 + chunk);
-  float s = 0.0f;
-#pragma unroll 8
-  for (int r = r0; r < r1; ++r) s += bf2f(D[(size_t)r * cols + c]);  // loads issued ahead, sums in order
-  part[(size_t)blockIdx.y * cols + c] = s;
-}
-
-// dst[i] = sum over z of part[z * count + i], z in [0, slices), in order.
-__global__ void k_sg_reduce(const float* __restrict__ part, int slices, int count, float* __restrict__ dst) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  float s = 0.0f;
-#pragma unroll 8
-  for (int z = 0; z < slices; ++z) s += part[(size_t)z * count + i];  // loads issued ahead, sums in order
-  dst[i] = s;
-}
-
-// Adam on the flat parameter vector; writes the bf16 copy used by the GEMMs.
-__global__ void k_sg_adam(float* __restrict__ p, float* __restrict__ m1, float* __restrict__ m2,
-                          const float* __restrict__ g, bf16_t* __restrict__ pb, int n, float lr, float b1,
-                          float b2, float c1, float c2, float eps) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float gi = g[i];
-  float a = b1 * m1[i] + (1.0f - b1) * gi;
-  float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
-  m1[i] = a;
-  m2[i] = b;
-  float v = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
-  p[i] = v;
-  pb[i] = f2bf(v);
-}
-
-__global__ void k_sg_to_bf16(const float* __restrict__ p, bf16_t* __restrict__ pb, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) pb[i] = f2bf(p[i]);
-}
+#include "rl_surrogate_train.h"
 
 // Uniform free-space rays for training: cell drawn by a counter-based hash,
 // redrawn while occupied (at most 64 draws; the map must have free cells).
@@ -687,27 +593,30 @@ struct rl_surrogate {
   float* d_m2 = nullptr;
   float* d_g = nullptr;    // gradient
   bf16_t* d_pb = nullptr;  // bf16 parameters
+  bf16_t* d_pt = nullptr;  // W2 and W3 transposed (sg_store_bf16)
   float* d_freq = nullptr; // RL_SG_NF x 4
   long long adam_t = 0;
-  // activations for `cap` rays
+  // rays, outputs, poses and targets for `cap` rays
   int cap = 0;
-  bf16_t *d_x = nullptr, *d_a1 = nullptr, *d_a2 = nullptr, *d_a3 = nullptr, *d_do = nullptr;
-  bf16_t *d_dz_a = nullptr, *d_dz_b = nullptr;
-  float* d_out = nullptr;
-  float* d_partial = nullptr;
   float4* d_rays = nullptr;
+  float* d_out = nullptr;
   float* d_poses = nullptr;
   float* d_target = nullptr;
-  float* d_split = nullptr;  // split-K / column-sum partials
+  // training minibatches of up to `tcap` rays: transposed matrices, row-major
+  // features, gradient partials
+  int tcap = 0;
+  bf16_t *d_t = nullptr, *d_x = nullptr;
+  float *d_split = nullptr, *d_bsplit = nullptr;
+  float* d_partial = nullptr;  // `pcap` loss partials
+  size_t pcap = 0;
   unsigned* d_stats = nullptr;
 };
 
 namespace {
 
 void sg_free(rl_surrogate* s) {
-  void* ps[] = {s->d_p, s->d_m1, s->d_m2, s->d_g, s->d_pb, s->d_freq, s->d_x, s->d_a1, s->d_a2, s->d_a3,
-                s->d_do, s->d_dz_a, s->d_dz_b, s->d_out, s->d_partial, s->d_rays, s->d_poses, s->d_target,
-                s->d_split, s->d_stats};
+  void* ps[] = {s->d_p, s->d_m1, s->d_m2, s->d_g, s->d_pb, s->d_pt, s->d_freq, s->d_rays, s->d_out, s->d_poses,
+                s->d_target, s->d_t, s->d_x, s->d_split, s->d_bsplit, s->d_partial, s->d_stats};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
@@ -722,34 +631,48 @@ int sg_alloc(T** p, size_t count) {
   return RL_OK;
 }
 
-// Activation buffers for n rays.
+// Frees *p and allocates count elements.
+template <typename T>
+int sg_regrow(T** p, size_t count) {
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  return sg_alloc(p, count);
+}
+
+// Ray buffers for n rays.
 int sg_reserve(rl_surrogate* s, int n) {
   if (s->cap >= n) return RL_OK;
-  void* old[] = {s->d_x, s->d_a1, s->d_a2, s->d_a3, s->d_do, s->d_dz_a, s->d_dz_b, s->d_out, s->d_partial,
-                 s->d_rays, s->d_poses, s->d_target, s->d_split};
   HIP_TRY(hipStreamSynchronize(s->map->ctx->stream));
-  for (void* p : old)
-    if (p) (void)hipFree(p);
-  s->d_x = s->d_a1 = s->d_a2 = s->d_a3 = s->d_do = s->d_dz_a = s->d_dz_b = nullptr;
-  s->d_out = s->d_partial = s->d_poses = s->d_target = nullptr;
-  s->d_rays = nullptr;
-  s->d_split = nullptr;
   s->cap = 0;
   size_t c = (size_t)n;
-  TRY(sg_alloc(&s->d_x, c * RL_SG_F));
-  TRY(sg_alloc(&s->d_a1, c * RL_SG_H));
-  TRY(sg_alloc(&s->d_a2, c * RL_SG_H));
-  TRY(sg_alloc(&s->d_a3, c * RL_SG_H));
-  TRY(sg_alloc(&s->d_dz_a, c * RL_SG_H));
-  TRY(sg_alloc(&s->d_dz_b, c * RL_SG_H));
-  TRY(sg_alloc(&s->d_do, c * RL_SG_OUT));
-  TRY(sg_alloc(&s->d_out, c * RL_SG_OUT));
-  TRY(sg_alloc(&s->d_partial, c / 256 + 2));
-  TRY(sg_alloc(&s->d_rays, c));
-  TRY(sg_alloc(&s->d_poses, c * 3));
-  TRY(sg_alloc(&s->d_target, c));
-  TRY(sg_alloc(&s->d_split, (size_t)RL_SG_MAX_SPLIT * RL_SG_H * RL_SG_H));
+  TRY(sg_regrow(&s->d_rays, c));
+  TRY(sg_regrow(&s->d_out, c * RL_SG_OUT));
+  TRY(sg_regrow(&s->d_poses, c * 3));
+  TRY(sg_regrow(&s->d_target, c));
   s->cap = n;
+  return RL_OK;
+}
+
+// Training buffers for minibatches of n rays and `partials` loss partials.
+int sg_reserve_train(rl_surrogate* s, int n, size_t partials) {
+  if (s->tcap >= n && s->pcap >= partials) return RL_OK;
+  HIP_TRY(hipStreamSynchronize(s->map->ctx->stream));
+  if (s->tcap < n) {
+    s->tcap = 0;
+    const size_t ld = ((size_t)n + RL_SGT_ROWS - 1) / RL_SGT_ROWS * RL_SGT_ROWS;
+    // every minibatch of up to n rays is cut into at most this many slices
+    const size_t slices = std::min<size_t>(RL_SG_MAX_SPLIT, ((size_t)n + 1023) / 1024);
+    TRY(sg_regrow(&s->d_t, SgT::N * ld));
+    TRY(sg_regrow(&s->d_x, (size_t)n * RL_SG_F));
+    TRY(sg_regrow(&s->d_split, slices * RL_SG_NPARAM));
+    TRY(sg_regrow(&s->d_bsplit, (size_t)256 * RL_SGT_BIAS));
+    s->tcap = n;
+  }
+  if (s->pcap < partials) {
+    s->pcap = 0;
+    TRY(sg_regrow(&s->d_partial, partials));
+    s->pcap = partials;
+  }
   return RL_OK;
 }
 
@@ -757,7 +680,7 @@ int sg_reserve(rl_surrogate* s, int n) {
 // aligned rows, the output is dense row-major and nothing is masked.
 bool nt_ok(const GemmArgs& g) {
   return g.sak == 1 && g.sbk == 1 && g.sam == g.K && g.sbn == g.K && g.K % 32 == 0 && g.N % 128 == 0 &&
-         g.scn == 1 && g.scm == g.N && !g.mask && ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;
+         g.scn == 1 && g.scm == g.N && ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;
 }
 
 int sg_gemm(hipStream_t st, const GemmArgs& g) {
@@ -778,26 +701,29 @@ GemmArgs gemm_args() {
   return g;
 }
 
-// Forward pass of n rays already in d_rays: d_x -> d_a1..d_a3 -> d_out.
-int sg_forward(rl_surrogate* s, int n) {
+// Forward pass of n rays already in d_rays, layer by layer, into d_out: the
+// plain form that k_sg_infer is compared with (its buffers live for the call).
+int sg_forward_layers(rl_surrogate* s, int n) {
   rl_map* m = s->map;
   hipStream_t st = m->ctx->stream;
-  hipLaunchKernelGGL(k_sg_features, dim3(grid_for(n, 256)), dim3(256), 0, st, (const float4*)s->d_rays,
-                     (const float*)s->d_freq, 1.0f / (float)m->width, 1.0f / (float)m->height, s->d_x, n);
-  HIP_TRY(hipGetLastError());
-  const bf16_t* P = s->d_pb;
-  const bf16_t* in[4] = {s->d_x, s->d_a1, s->d_a2, s->d_a3};
-  bf16_t* outb[3] = {s->d_a1, s->d_a2, s->d_a3};
-  const int w_off[4] = {SgLayout::W1, SgLayout::W2, SgLayout::W3, SgLayout::W4};
-  const int b_off[4] = {SgLayout::B1, SgLayout::B2, SgLayout::B3, SgLayout::B4};
+  bf16_t* act[4] = {nullptr, nullptr, nullptr, nullptr};
   const int fin[4] = {RL_SG_F, RL_SG_H, RL_SG_H, RL_SG_H};
   const int fout[4] = {RL_SG_H, RL_SG_H, RL_SG_H, RL_SG_OUT};
-  for (int l = 0; l < 4; ++l) {
+  const int w_off[4] = {SgLayout::W1, SgLayout::W2, SgLayout::W3, SgLayout::W4};
+  const int b_off[4] = {SgLayout::B1, SgLayout::B2, SgLayout::B3, SgLayout::B4};
+  int rc = RL_OK;
+  for (int l = 0; l < 4 && rc == RL_OK; ++l) rc = sg_alloc(&act[l], (size_t)n * fin[l]);
+  if (rc == RL_OK) {
+    hipLaunchKernelGGL(k_sg_features, dim3(grid_for(n, 256)), dim3(256), 0, st, (const float4*)s->d_rays,
+                       (const float*)s->d_freq, 1.0f / (float)m->width, 1.0f / (float)m->height, act[0], n);
+    if (hipGetLastError() != hipSuccess) rc = fail(RL_ERR_HIP, "surrogate features launch failed");
+  }
+  for (int l = 0; l < 4 && rc == RL_OK; ++l) {
     GemmArgs g = gemm_args();
-    g.A = in[l];
+    g.A = act[l];
     g.sam = fin[l];
     g.sak = 1;
-    g.B = P + w_off[l];  // B(k = i, n = o) = W[o][i]
+    g.B = s->d_pb + w_off[l];  // B(k = i, n = o) = W[o][i]
     g.sbk = 1;
     g.sbn = fin[l];
     g.M = n;
@@ -808,16 +734,19 @@ int sg_forward(rl_surrogate* s, int n) {
     g.scm = fout[l];
     g.scn = 1;
     if (l < 3)
-      g.Cb = outb[l];
+      g.Cb = act[l + 1];
     else
       g.C = s->d_out;
-    TRY(sg_gemm(st, g));
+    rc = sg_gemm(st, g);
   }
-  return RL_OK;
+  if (rc == RL_OK && hipStreamSynchronize(st) != hipSuccess) rc = fail(RL_ERR_HIP, "surrogate layers failed");
+  for (bf16_t* a : act)
+    if (a) (void)hipFree(a);
+  return rc;
 }
 
 // Network outputs of n rays already in d_rays into d_out, one fused launch
-// (no intermediate activations in HBM); bitwise equal to sg_forward's d_out.
+// (no intermediate activations in HBM); bitwise equal to sg_forward_layers'.
 int sg_infer(rl_surrogate* s, int n) {
   rl_map* m = s->map;
   hipLaunchKernelGGL(k_sg_infer, dim3((unsigned)((n + RL_SG_TM - 1) / RL_SG_TM)), dim3(256), 0, m->ctx->stream,
@@ -827,94 +756,51 @@ int sg_infer(rl_surrogate* s, int n) {
   return RL_OK;
 }
 
-// Loss, gradient into d_g (fp32, layout of the parameters) for n rays with
-// targets in d_target.  grad_out (optional) receives d loss / d out (n x 2).
-int sg_backward(rl_surrogate* s, int n, float max_range, float* grad_out) {
+// Loss partials (one per RL_SGT_ROWS rays) into `partial` and the gradient's
+// partial sums for n rays, their gradient then formed by sg_update.  The
+// training buffers hold n rays.
+int sg_pass(rl_surrogate* s, const float4* rays, const float* target, int n, float max_range, float* partial,
+            bf16_t* x_rows) {
   rl_map* m = s->map;
   hipStream_t st = m->ctx->stream;
-  hipLaunchKernelGGL(k_sg_loss, dim3(grid_for(n, 256)), dim3(256), 0, st, (const float*)s->d_out,
-                     (const float*)s->d_target, max_range, 1.0f / (float)n, s->d_do, grad_out, s->d_partial, n);
+  const int blocks = (n + RL_SGT_ROWS - 1) / RL_SGT_ROWS, ld = blocks * RL_SGT_ROWS;
+  SgPass g;
+  g.rays = rays;
+  g.target = target;
+  g.freq = s->d_freq;
+  g.inv_w = 1.0f / (float)m->width;
+  g.inv_h = 1.0f / (float)m->height;
+  g.max_range = max_range;
+  g.inv_n = 1.0f / (float)n;
+  g.P = s->d_pb;
+  g.Pt = s->d_pt;
+  g.Pf = s->d_p;
+  g.T = s->d_t;
+  g.x_rows = x_rows;
+  g.partial = partial;
+  g.n = n;
+  g.ld = ld;
+  hipLaunchKernelGGL(k_sg_fwd_bwd, dim3(blocks), dim3(RL_SGT_THREADS), 0, st, g);
   HIP_TRY(hipGetLastError());
-  const bf16_t* P = s->d_pb;
-  // layer l: input act_in (n x fin), output grad dz (n x fout); W at w_off (fout x fin)
-  const bf16_t* acts[4] = {s->d_x, s->d_a1, s->d_a2, s->d_a3};
-  const int w_off[4] = {SgLayout::W1, SgLayout::W2, SgLayout::W3, SgLayout::W4};
-  const int b_off[4] = {SgLayout::B1, SgLayout::B2, SgLayout::B3, SgLayout::B4};
-  const int fin[4] = {RL_SG_F, RL_SG_H, RL_SG_H, RL_SG_H};
-  const int fout[4] = {RL_SG_H, RL_SG_H, RL_SG_H, RL_SG_OUT};
-  const bf16_t* dz = s->d_do;
-  bf16_t* bufs[2] = {s->d_dz_a, s->d_dz_b};
-  // split-K over the batch for the weight gradients: ~1024 rows per slice
-  const int splits = std::max(1, std::min(RL_SG_MAX_SPLIT, (n + 1023) / 1024));
-  const int kchunk = ((n + splits - 1) / splits + 31) / 32 * 32;
-  const int nz = (n + kchunk - 1) / kchunk;
-  // column sums over row chunks of >= 256 rows, at most 256 chunks
-  const int cchunk = std::max(256, (n + 255) / 256);
-  const int ncz = (n + cchunk - 1) / cchunk;
-  for (int l = 3; l >= 0; --l) {
-    // dW[o][i] = sum_b dz[b][o] act[b][i]
-    GemmArgs g = gemm_args();
-    g.A = dz;
-    g.sam = 1;
-    g.sak = fout[l];
-    g.B = acts[l];
-    g.sbk = fin[l];
-    g.sbn = 1;
-    g.M = fout[l];
-    g.N = fin[l];
-    g.K = n;
-    g.scm = fin[l];
-    g.scn = 1;
-    if (nz > 1) {
-      g.C = s->d_split;
-      g.kchunk = kchunk;
-      g.scz = (long long)fout[l] * fin[l];
-      dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, nz);
-      hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, st, g);
-      HIP_TRY(hipGetLastError());
-      hipLaunchKernelGGL(k_sg_reduce, dim3(grid_for(fout[l] * fin[l], 256)), dim3(256), 0, st,
-                         (const float*)s->d_split, nz, fout[l] * fin[l], s->d_g + w_off[l]);
-    } else {
-      g.C = s->d_g + w_off[l];
-      TRY(sg_gemm(st, g));
-    }
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_sg_colsum, dim3(grid_for(fout[l], 64), ncz), dim3(64), 0, st, dz, n, fout[l], cchunk,
-                       s->d_split);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_sg_reduce, dim3(grid_for(fout[l], 256)), dim3(256), 0, st, (const float*)s->d_split,
-                       ncz, fout[l], s->d_g + b_off[l]);
-    HIP_TRY(hipGetLastError());
-    if (l == 0) break;
-    // dz_prev[b][i] = (act[b][i] > 0) * sum_o dz[b][o] W[o][i]
-    bf16_t* nxt = bufs[l & 1];
-    GemmArgs h = gemm_args();
-    h.A = dz;
-    h.sam = fout[l];
-    h.sak = 1;
-    h.B = P + w_off[l];
-    h.sbk = fin[l];
-    h.sbn = 1;
-    h.M = n;
-    h.N = fin[l];
-    h.K = fout[l];
-    h.mask = acts[l];
-    h.Cb = nxt;
-    h.scm = fin[l];
-    h.scn = 1;
-    TRY(sg_gemm(st, h));
-    dz = nxt;
-  }
+  const SgSplit sp = sg_split(n);
+  const int gemm_blocks = 8 * ((sp.nz + 7) / 8) * RL_SGT_TILES;
+  hipLaunchKernelGGL(k_sg_wgrad, dim3(gemm_blocks + grid_for((long long)sp.ncz * RL_SGT_BIAS, 256)), dim3(256), 0, st,
+                     (const bf16_t*)s->d_t, n, ld, sp, gemm_blocks, s->d_split, s->d_bsplit);
+  HIP_TRY(hipGetLastError());
   return RL_OK;
 }
 
-int sg_adam(rl_surrogate* s, float lr) {
-  s->adam_t += 1;
-  const float b1 = 0.9f, b2 = 0.999f;
-  float c1 = (float)(1.0 - pow(0.9, (double)s->adam_t));
-  float c2 = (float)(1.0 - pow(0.999, (double)s->adam_t));
-  hipLaunchKernelGGL(k_sg_adam, dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, s->map->ctx->stream, s->d_p,
-                     s->d_m1, s->d_m2, (const float*)s->d_g, s->d_pb, RL_SG_NPARAM, lr, b1, b2, c1, c2, 1e-8f);
+// The gradient of the last sg_pass over n rays into d_g (SUM) and one Adam
+// step with d_g (ADAM).
+template <bool SUM, bool ADAM>
+int sg_update(rl_surrogate* s, int n, float lr) {
+  const SgSplit sp = sg_split(n);
+  if (ADAM) s->adam_t += 1;
+  const float c1 = (float)(1.0 - pow(0.9, (double)s->adam_t));
+  const float c2 = (float)(1.0 - pow(0.999, (double)s->adam_t));
+  hipLaunchKernelGGL((k_sg_update<SUM, ADAM>), dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, s->map->ctx->stream,
+                     (const float*)s->d_split, (const float*)s->d_bsplit, sp.nz, sp.ncz, s->d_g, s->d_p, s->d_m1, s->d_m2,
+                     s->d_pb, s->d_pt, lr, 0.9f, 0.999f, c1, c2, 1e-8f);
   HIP_TRY(hipGetLastError());
   return RL_OK;
 }
@@ -941,7 +827,8 @@ int rl_surrogate_create(rl_map* map, unsigned seed, rl_surrogate** out) {
   int rc = RL_OK;
   if ((rc = sg_alloc(&s->d_p, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_m1, RL_SG_NPARAM)) ||
       (rc = sg_alloc(&s->d_m2, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_g, RL_SG_NPARAM)) ||
-      (rc = sg_alloc(&s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_freq, RL_SG_NF * 4)) ||
+      (rc = sg_alloc(&s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_pt, 2 * RL_SG_H * RL_SG_H)) ||
+      (rc = sg_alloc(&s->d_freq, RL_SG_NF * 4)) ||
       (rc = sg_alloc(&s->d_stats, 5))) {
     sg_free(s);
     delete s;
@@ -983,7 +870,7 @@ int rl_surrogate_create(rl_map* map, unsigned seed, rl_surrogate** out) {
   if (e == hipSuccess) e = hipMemsetAsync(s->d_m2, 0, RL_SG_NPARAM * 4, st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_sg_to_bf16, dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, st, (const float*)s->d_p,
-                       s->d_pb, RL_SG_NPARAM);
+                       s->d_pb, s->d_pt, RL_SG_NPARAM);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1028,7 +915,7 @@ int rl_surrogate_set_params(rl_surrogate* s, const float* params, const float* f
   if (params) HIP_TRY(hipMemcpyAsync(s->d_p, params, RL_SG_NPARAM * 4, hipMemcpyHostToDevice, st));
   if (freq) HIP_TRY(hipMemcpyAsync(s->d_freq, freq, RL_SG_NF * 16, hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_sg_to_bf16, dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, st, (const float*)s->d_p,
-                     s->d_pb, RL_SG_NPARAM);
+                     s->d_pb, s->d_pt, RL_SG_NPARAM);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
@@ -1043,7 +930,7 @@ static int surrogate_forward(rl_surrogate* s, const float* rays4, int n, float* 
   TRY(sg_reserve(s, n));
   hipStream_t st = s->map->ctx->stream;
   HIP_TRY(hipMemcpyAsync(s->d_rays, rays4, (size_t)n * 16, hipMemcpyHostToDevice, st));
-  TRY(layers ? sg_forward(s, n) : sg_infer(s, n));
+  TRY(layers ? sg_forward_layers(s, n) : sg_infer(s, n));
   HIP_TRY(hipMemcpyAsync(out, s->d_out, (size_t)n * 8, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
@@ -1061,14 +948,15 @@ int rl_surrogate_gradient(rl_surrogate* s, float max_range, const float* rays4, 
   std::lock_guard<std::mutex> lk(s->map->ctx->mu);
   TRY(use_device(s->map->ctx));
   TRY(sg_reserve(s, n));
+  std::vector<float> part(grid_for(n, RL_SGT_ROWS));
+  TRY(sg_reserve_train(s, n, part.size()));
   hipStream_t st = s->map->ctx->stream;
   HIP_TRY(hipMemcpyAsync(s->d_rays, rays4, (size_t)n * 16, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(s->d_target, targets, (size_t)n * 4, hipMemcpyHostToDevice, st));
-  TRY(sg_forward(s, n));
-  TRY(sg_backward(s, n, max_range, nullptr));
+  TRY(sg_pass(s, s->d_rays, s->d_target, n, max_range, s->d_partial, features ? s->d_x : nullptr));
+  TRY((sg_update<true, false>(s, n, 0.0f)));
   if (grad) HIP_TRY(hipMemcpyAsync(grad, s->d_g, RL_SG_NPARAM * 4, hipMemcpyDeviceToHost, st));
   if (features) HIP_TRY(hipMemcpyAsync(features, s->d_x, (size_t)n * RL_SG_F * 2, hipMemcpyDeviceToHost, st));
-  std::vector<float> part(grid_for(n, 256));
   HIP_TRY(hipMemcpyAsync(part.data(), s->d_partial, part.size() * 4, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   if (loss) {
@@ -1085,7 +973,7 @@ int rl_surrogate_step(rl_surrogate* s, float lr) {
   CHECK_ARG(s && lr > 0.0f, "bad argument");
   std::lock_guard<std::mutex> lk(s->map->ctx->mu);
   TRY(use_device(s->map->ctx));
-  TRY(sg_adam(s, lr));
+  TRY((sg_update<false, true>(s, 1, lr)));
   HIP_TRY(hipStreamSynchronize(s->map->ctx->stream));
   return RL_OK;
 }
@@ -1100,25 +988,36 @@ int rl_surrogate_train(rl_surrogate* s, float max_range, long long n_pairs, int 
   rl_ctx* c = s->map->ctx;
   TRY(use_device(c));
   if (!s->map->d_edt) return fail(RL_ERR_STATE, "map has no distance transform");
-  TRY(sg_reserve(s, batch));
   hipStream_t st = c->stream;
   const long long steps = n_pairs / batch;
-  std::vector<float> part(grid_for(batch, 256));
-  for (long long k = 0; k < steps; ++k) {
-    hipLaunchKernelGGL(k_sg_sample, dim3(grid_for(batch, 256)), dim3(256), 0, st, s->map->dev(), c->trig, seed,
-                       k * (long long)batch, batch, s->d_poses, s->d_rays);
+  // The rays do not depend on the parameters: they are drawn and marched for
+  // several minibatches at once (a march is bound by its longest ray: 21 us for
+  // 16384 rays, 33 us for 262144), and the losses come back once per group.
+  const int group = (int)std::min<long long>(std::max<long long>(steps, 1), std::max(1, RL_SG_GROUP_RAYS / batch));
+  const int nb = grid_for(batch, RL_SGT_ROWS);
+  TRY(sg_reserve(s, group * batch));
+  TRY(sg_reserve_train(s, batch, (size_t)group * nb));
+  std::vector<float> part((size_t)group * nb);
+  for (long long k = 0; k < steps; k += group) {
+    const int cnt = (int)std::min<long long>(group, steps - k), n = cnt * batch;
+    hipLaunchKernelGGL(k_sg_sample, dim3(grid_for(n, 256)), dim3(256), 0, st, s->map->dev(), c->trig, seed,
+                       k * (long long)batch, n, s->d_poses, s->d_rays);
     HIP_TRY(hipGetLastError());
     TRY(launch_cast(s->map, RL_METHOD_RM, RL_FRAME_GRID, false, max_range, s->d_poses, nullptr, s->d_target,
-                    nullptr, batch, 0));
-    TRY(sg_forward(s, batch));
-    TRY(sg_backward(s, batch, max_range, nullptr));
-    TRY(sg_adam(s, lr));
+                    nullptr, n, 0));
+    for (int j = 0; j < cnt; ++j) {
+      TRY(sg_pass(s, s->d_rays + (size_t)j * batch, s->d_target + (size_t)j * batch, batch, max_range,
+                  s->d_partial + (size_t)j * nb, nullptr));
+      TRY((sg_update<true, true>(s, batch, lr)));
+    }
     if (loss_curve) {
-      HIP_TRY(hipMemcpyAsync(part.data(), s->d_partial, part.size() * 4, hipMemcpyDeviceToHost, st));
+      HIP_TRY(hipMemcpyAsync(part.data(), s->d_partial, (size_t)cnt * nb * 4, hipMemcpyDeviceToHost, st));
       HIP_TRY(hipStreamSynchronize(st));
-      double t = 0;
-      for (float v : part) t += v;
-      loss_curve[k] = (float)t;
+      for (int j = 0; j < cnt; ++j) {
+        double t = 0;
+        for (int b = 0; b < nb; ++b) t += part[(size_t)j * nb + b];
+        loss_curve[k + j] = (float)t;
+      }
     }
   }
   HIP_TRY(hipStreamSynchronize(st));

@@ -390,3 +390,24 @@ def test_surrogate_rejects_bad_arguments(ctx):
         sg.train(10.0, n_pairs=100, batch=16)  # batch below 64
     with pytest.raises(ValueError):
         sg.set_params(np.zeros(5, np.float32))
+
+
+@pytest.mark.parametrize("n", [1, 65, 1056, 70001])
+def test_gradient_row_cuts_vs_cpu(ctx, n):
+    """Gradients where the rows' cuts end unevenly: one ray, a workgroup of one
+    ray, two slices of 544 rows (not a multiple of the 64-row stage), and 64
+    slices with bias chunks that start off the 8-row loads."""
+    R = 120.0
+    img, g, rays = _map_and_rays(n)
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    sg = rl.Surrogate(dm, seed=3)
+    p, _ = sg.params()
+    _, _, feat = sg.gradient(R, rays, np.zeros(n, np.float32))
+    x = S.bf16_to_f64(feat)
+    t = _targets_for_both_regimes(p, x, R, n)
+    loss, grad, _ = sg.gradient(R, rays, t)
+    l16, g16, _ = S.loss_and_grad(p, x, t, R, emulate_bf16=True)
+    assert abs(loss - l16) <= 1e-4 * abs(l16)
+    for w, b, o, i in S.LAYERS:
+        for sl in (slice(w, w + o * i), slice(b, b + o)):
+            assert _rel(grad[sl], g16[sl]) <= 1e-2 and _cos(grad[sl], g16[sl]) >= 0.9999
