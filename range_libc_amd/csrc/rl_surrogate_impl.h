@@ -78,6 +78,25 @@ struct SgLayout {
 };
 static_assert(SgLayout::N == RL_SG_NPARAM, "surrogate parameter layout");
 
+// The hidden layers' bf16 weights (and W2, W3 transposed, for the data
+// gradients) in the order the 16x16x32 instruction takes them: for each 16 rows
+// and 32 k, lane l's eight values (row l & 15, k = 8 (l >> 4) .. + 7) follow those
+// of lane l - 1, so a fragment load of a wave is 1 KB of whole cache lines.  Read
+// from the row-major matrix it touched 16 half lines, and the loads' rate bounded
+// the layers (a 256 x 256 layer's fragments of one workgroup: 7000 cycles, 1300 so).
+struct SgFrag {
+  static constexpr int W1 = 0;
+  static constexpr int W2 = W1 + RL_SG_H * RL_SG_F;
+  static constexpr int W3 = W2 + RL_SG_H * RL_SG_H;
+  static constexpr int W2T = W3 + RL_SG_H * RL_SG_H;
+  static constexpr int W3T = W2T + RL_SG_H * RL_SG_H;
+  static constexpr int N = W3T + RL_SG_H * RL_SG_H;
+  // place of element (row, k) of a matrix with K columns
+  __host__ __device__ static constexpr int at(int row, int k, int K) {
+    return (((row >> 4) * (K >> 5) + (k >> 5)) * 64 + (row & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // GEMM: C(m, n) = sum_k A(m, k) * B(k, n), bf16 operands, fp32 accumulation.
 // A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn] (any
@@ -285,8 +304,8 @@ __global__ void k_sg_bf16_check(unsigned long long* __restrict__ bad) {
 }
 
 // One hidden layer: act (64 x K) -> act (64 x 256), wave w computing columns
-// 64w .. 64w + 63.  W is the bf16 layer matrix [256][K] (K-contiguous), sb the
-// layer's biases in LDS.  b0 holds the wave's fragments of the first k step,
+// 64w .. 64w + 63.  W is the layer's matrix in SgFrag order, sb the layer's
+// biases in LDS.  b0 holds the wave's fragments of the first k step,
 // loaded before the layer starts; the layer loads those of the next layer (Wn,
 // KN columns; KN = 0: none) before its own epilogue, so that no layer starts
 // with an L2 round trip.
@@ -307,7 +326,7 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
     sg_bf16x8 b[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      b[j] = s == 0 ? b0[j] : *(const sg_bf16x8*)(W + (size_t)(nw + j * 16 + r16) * K + s * 32 + kq);
+      b[j] = s == 0 ? b0[j] : *(const sg_bf16x8*)(W + (((wave * 4 + j) * KS + s) * 64 + lane) * 8);
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
       const sg_bf16x8 a = *(const sg_bf16x8*)(act + (i * 16 + r16) * RL_SG_ACT_PAD + s * 32 + kq);
@@ -317,7 +336,7 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
   }
   if (KN) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) b0[j] = *(const sg_bf16x8*)(Wn + (size_t)(nw + j * 16 + r16) * KN + kq);
+    for (int j = 0; j < 4; ++j) b0[j] = *(const sg_bf16x8*)(Wn + ((wave * 4 + j) * (KN / 32) * 64 + lane) * 8);
   }
   __syncthreads();  // every wave has read the layer's input before it is overwritten
 #pragma unroll
@@ -336,13 +355,15 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
   __syncthreads();
 }
 
-// rays: n x (x0, y0, sin h, cos h); P / Pf: the bf16 / fp32 parameter vectors;
+// rays: n x (x0, y0, sin h, cos h); P / Pf: the bf16 / fp32 parameter vectors, F
+// the weights in SgFrag order;
 // out: n x 2 fp32.  Launched with ceil(n / 64) workgroups of 256 threads.
 // Register use is held to 128 so that four waves share each SIMD (measured on
 // 240,000 rays: 3 waves, 144 registers, 5% slower).
 __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ rays, const float* __restrict__ freq,
                                                   float inv_w, float inv_h, const bf16_t* __restrict__ P,
-                                                  const float* __restrict__ Pf, float* __restrict__ out, int n) {
+                                                  const bf16_t* __restrict__ F, const float* __restrict__ Pf,
+                                                  float* __restrict__ out, int n) {
   __shared__ __align__(16) bf16_t act[RL_SG_TM * RL_SG_ACT_PAD];
   __shared__ float sbias[3 * RL_SG_H + RL_SG_OUT];         // b1, b2, b3, b4
   __shared__ __align__(16) bf16_t sw4[RL_SG_OUT * RL_SG_H];  // W4
@@ -351,8 +372,7 @@ __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ 
   sg_bf16x8 b0[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    b0[j] = *(const sg_bf16x8*)(P + SgLayout::W1 + (size_t)(wave * 64 + j * 16 + (lane & 15)) * RL_SG_F +
-                                (lane >> 4) * 8);
+    b0[j] = *(const sg_bf16x8*)(F + SgFrag::W1 + ((wave * 4 + j) * (RL_SG_F / 32) * 64 + lane) * 8);
   sbias[tid] = Pf[SgLayout::B1 + tid];
   sbias[RL_SG_H + tid] = Pf[SgLayout::B2 + tid];
   sbias[2 * RL_SG_H + tid] = Pf[SgLayout::B3 + tid];
@@ -374,9 +394,9 @@ __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ 
     act[r * RL_SG_ACT_PAD + RL_SG_NF + j] = c;
   }
   __syncthreads();
-  sg_hidden_layer<RL_SG_F, RL_SG_H>(act, P + SgLayout::W1, sbias, P + SgLayout::W2, b0, wave, lane);
-  sg_hidden_layer<RL_SG_H, RL_SG_H>(act, P + SgLayout::W2, sbias + RL_SG_H, P + SgLayout::W3, b0, wave, lane);
-  sg_hidden_layer<RL_SG_H, 0>(act, P + SgLayout::W3, sbias + 2 * RL_SG_H, nullptr, b0, wave, lane);
+  sg_hidden_layer<RL_SG_F, RL_SG_H>(act, F + SgFrag::W1, sbias, F + SgFrag::W2, b0, wave, lane);
+  sg_hidden_layer<RL_SG_H, RL_SG_H>(act, F + SgFrag::W2, sbias + RL_SG_H, F + SgFrag::W3, b0, wave, lane);
+  sg_hidden_layer<RL_SG_H, 0>(act, F + SgFrag::W3, sbias + 2 * RL_SG_H, nullptr, b0, wave, lane);
   // heads: wave w takes rows 16w .. 16w + 15 (RL_SG_TM / 64 tiles of 16 rows
   // per wave); columns 0 and 1 of one 16-wide tile
   const int col = lane & 15, kb = 4 * (lane >> 4);
@@ -593,7 +613,7 @@ struct rl_surrogate {
   float* d_m2 = nullptr;
   float* d_g = nullptr;    // gradient
   bf16_t* d_pb = nullptr;  // bf16 parameters
-  bf16_t* d_pt = nullptr;  // W2 and W3 transposed (sg_store_bf16)
+  bf16_t* d_pf = nullptr;  // weights as matrix operands (SgFrag)
   float* d_freq = nullptr; // RL_SG_NF x 4
   long long adam_t = 0;
   // rays, outputs, poses and targets for `cap` rays
@@ -602,10 +622,9 @@ struct rl_surrogate {
   float* d_out = nullptr;
   float* d_poses = nullptr;
   float* d_target = nullptr;
-  // training minibatches of up to `tcap` rays: transposed matrices, row-major
-  // features, gradient partials
+  // training minibatches of up to `tcap` rays: matrices (SgT), gradient partials
   int tcap = 0;
-  bf16_t *d_t = nullptr, *d_x = nullptr;
+  bf16_t* d_t = nullptr;
   float *d_split = nullptr, *d_bsplit = nullptr;
   float* d_partial = nullptr;  // `pcap` loss partials
   size_t pcap = 0;
@@ -615,8 +634,8 @@ struct rl_surrogate {
 namespace {
 
 void sg_free(rl_surrogate* s) {
-  void* ps[] = {s->d_p, s->d_m1, s->d_m2, s->d_g, s->d_pb, s->d_pt, s->d_freq, s->d_rays, s->d_out, s->d_poses,
-                s->d_target, s->d_t, s->d_x, s->d_split, s->d_bsplit, s->d_partial, s->d_stats};
+  void* ps[] = {s->d_p, s->d_m1, s->d_m2, s->d_g, s->d_pb, s->d_pf, s->d_freq, s->d_rays, s->d_out, s->d_poses,
+                s->d_target, s->d_t, s->d_split, s->d_bsplit, s->d_partial, s->d_stats};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
@@ -659,12 +678,11 @@ int sg_reserve_train(rl_surrogate* s, int n, size_t partials) {
   HIP_TRY(hipStreamSynchronize(s->map->ctx->stream));
   if (s->tcap < n) {
     s->tcap = 0;
-    const size_t ld = ((size_t)n + RL_SGT_ROWS - 1) / RL_SGT_ROWS * RL_SGT_ROWS;
+    const size_t ld = ((size_t)n + 63) / 64 * 64;
     // every minibatch of up to n rays is cut into at most this many slices
     const size_t slices = std::min<size_t>(RL_SG_MAX_SPLIT, ((size_t)n + 1023) / 1024);
     TRY(sg_regrow(&s->d_t, SgT::N * ld));
-    TRY(sg_regrow(&s->d_x, (size_t)n * RL_SG_F));
-    TRY(sg_regrow(&s->d_split, slices * RL_SG_NPARAM));
+    TRY(sg_regrow(&s->d_split, slices * RL_SGT_PART));
     TRY(sg_regrow(&s->d_bsplit, (size_t)256 * RL_SGT_BIAS));
     s->tcap = n;
   }
@@ -751,19 +769,19 @@ int sg_infer(rl_surrogate* s, int n) {
   rl_map* m = s->map;
   hipLaunchKernelGGL(k_sg_infer, dim3((unsigned)((n + RL_SG_TM - 1) / RL_SG_TM)), dim3(256), 0, m->ctx->stream,
                      (const float4*)s->d_rays, (const float*)s->d_freq, 1.0f / (float)m->width,
-                     1.0f / (float)m->height, (const bf16_t*)s->d_pb, (const float*)s->d_p, s->d_out, n);
+                     1.0f / (float)m->height, (const bf16_t*)s->d_pb, (const bf16_t*)s->d_pf, (const float*)s->d_p,
+                     s->d_out, n);
   HIP_TRY(hipGetLastError());
   return RL_OK;
 }
 
 // Loss partials (one per RL_SGT_ROWS rays) into `partial` and the gradient's
-// partial sums for n rays, their gradient then formed by sg_update.  The
+// partial sums for n rays (the features are the first matrix of d_t), their gradient then formed by sg_update.  The
 // training buffers hold n rays.
-int sg_pass(rl_surrogate* s, const float4* rays, const float* target, int n, float max_range, float* partial,
-            bf16_t* x_rows) {
+int sg_pass(rl_surrogate* s, const float4* rays, const float* target, int n, float max_range, float* partial) {
   rl_map* m = s->map;
   hipStream_t st = m->ctx->stream;
-  const int blocks = (n + RL_SGT_ROWS - 1) / RL_SGT_ROWS, ld = blocks * RL_SGT_ROWS;
+  const int ld = (n + 63) / 64 * 64;
   SgPass g;
   g.rays = rays;
   g.target = target;
@@ -773,19 +791,18 @@ int sg_pass(rl_surrogate* s, const float4* rays, const float* target, int n, flo
   g.max_range = max_range;
   g.inv_n = 1.0f / (float)n;
   g.P = s->d_pb;
-  g.Pt = s->d_pt;
+  g.F = s->d_pf;
   g.Pf = s->d_p;
   g.T = s->d_t;
-  g.x_rows = x_rows;
   g.partial = partial;
   g.n = n;
   g.ld = ld;
-  hipLaunchKernelGGL(k_sg_fwd_bwd, dim3(blocks), dim3(RL_SGT_THREADS), 0, st, g);
+  hipLaunchKernelGGL(k_sg_fwd_bwd, dim3(ld / RL_SGT_ROWS), dim3(RL_SGT_THREADS), 0, st, g);
   HIP_TRY(hipGetLastError());
   const SgSplit sp = sg_split(n);
-  const int gemm_blocks = 8 * ((sp.nz + 7) / 8) * RL_SGT_TILES;
-  hipLaunchKernelGGL(k_sg_wgrad, dim3(gemm_blocks + grid_for((long long)sp.ncz * RL_SGT_BIAS, 256)), dim3(256), 0, st,
-                     (const bf16_t*)s->d_t, n, ld, sp, gemm_blocks, s->d_split, s->d_bsplit);
+  const int bias_blocks = (grid_for((long long)sp.ncz * RL_SGT_BIAS, 256) + 7) / 8 * 8;
+  hipLaunchKernelGGL(k_sg_wgrad, dim3(bias_blocks + 8 * ((sp.nz + 7) / 8) * RL_SGT_TILES), dim3(256), 0, st,
+                     (const bf16_t*)s->d_t, n, ld, sp, bias_blocks, s->d_split, s->d_bsplit);
   HIP_TRY(hipGetLastError());
   return RL_OK;
 }
@@ -800,7 +817,7 @@ int sg_update(rl_surrogate* s, int n, float lr) {
   const float c2 = (float)(1.0 - pow(0.999, (double)s->adam_t));
   hipLaunchKernelGGL((k_sg_update<SUM, ADAM>), dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, s->map->ctx->stream,
                      (const float*)s->d_split, (const float*)s->d_bsplit, sp.nz, sp.ncz, s->d_g, s->d_p, s->d_m1, s->d_m2,
-                     s->d_pb, s->d_pt, lr, 0.9f, 0.999f, c1, c2, 1e-8f);
+                     s->d_pb, s->d_pf, lr, 0.9f, 0.999f, c1, c2, 1e-8f);
   HIP_TRY(hipGetLastError());
   return RL_OK;
 }
@@ -827,7 +844,7 @@ int rl_surrogate_create(rl_map* map, unsigned seed, rl_surrogate** out) {
   int rc = RL_OK;
   if ((rc = sg_alloc(&s->d_p, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_m1, RL_SG_NPARAM)) ||
       (rc = sg_alloc(&s->d_m2, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_g, RL_SG_NPARAM)) ||
-      (rc = sg_alloc(&s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_pt, 2 * RL_SG_H * RL_SG_H)) ||
+      (rc = sg_alloc(&s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_pf, SgFrag::N)) ||
       (rc = sg_alloc(&s->d_freq, RL_SG_NF * 4)) ||
       (rc = sg_alloc(&s->d_stats, 5))) {
     sg_free(s);
@@ -870,7 +887,7 @@ int rl_surrogate_create(rl_map* map, unsigned seed, rl_surrogate** out) {
   if (e == hipSuccess) e = hipMemsetAsync(s->d_m2, 0, RL_SG_NPARAM * 4, st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_sg_to_bf16, dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, st, (const float*)s->d_p,
-                       s->d_pb, s->d_pt, RL_SG_NPARAM);
+                       s->d_pb, s->d_pf, RL_SG_NPARAM);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -915,7 +932,7 @@ int rl_surrogate_set_params(rl_surrogate* s, const float* params, const float* f
   if (params) HIP_TRY(hipMemcpyAsync(s->d_p, params, RL_SG_NPARAM * 4, hipMemcpyHostToDevice, st));
   if (freq) HIP_TRY(hipMemcpyAsync(s->d_freq, freq, RL_SG_NF * 16, hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_sg_to_bf16, dim3(grid_for(RL_SG_NPARAM, 256)), dim3(256), 0, st, (const float*)s->d_p,
-                     s->d_pb, s->d_pt, RL_SG_NPARAM);
+                     s->d_pb, s->d_pf, RL_SG_NPARAM);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
@@ -948,15 +965,15 @@ int rl_surrogate_gradient(rl_surrogate* s, float max_range, const float* rays4, 
   std::lock_guard<std::mutex> lk(s->map->ctx->mu);
   TRY(use_device(s->map->ctx));
   TRY(sg_reserve(s, n));
-  std::vector<float> part(grid_for(n, RL_SGT_ROWS));
+  std::vector<float> part((size_t)(n + 63) / 64 * 64 / RL_SGT_ROWS);
   TRY(sg_reserve_train(s, n, part.size()));
   hipStream_t st = s->map->ctx->stream;
   HIP_TRY(hipMemcpyAsync(s->d_rays, rays4, (size_t)n * 16, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(s->d_target, targets, (size_t)n * 4, hipMemcpyHostToDevice, st));
-  TRY(sg_pass(s, s->d_rays, s->d_target, n, max_range, s->d_partial, features ? s->d_x : nullptr));
+  TRY(sg_pass(s, s->d_rays, s->d_target, n, max_range, s->d_partial));
   TRY((sg_update<true, false>(s, n, 0.0f)));
   if (grad) HIP_TRY(hipMemcpyAsync(grad, s->d_g, RL_SG_NPARAM * 4, hipMemcpyDeviceToHost, st));
-  if (features) HIP_TRY(hipMemcpyAsync(features, s->d_x, (size_t)n * RL_SG_F * 2, hipMemcpyDeviceToHost, st));
+  if (features) HIP_TRY(hipMemcpyAsync(features, s->d_t, (size_t)n * RL_SG_F * 2, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipMemcpyAsync(part.data(), s->d_partial, part.size() * 4, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   if (loss) {
@@ -994,7 +1011,7 @@ int rl_surrogate_train(rl_surrogate* s, float max_range, long long n_pairs, int 
   // several minibatches at once (a march is bound by its longest ray: 21 us for
   // 16384 rays, 33 us for 262144), and the losses come back once per group.
   const int group = (int)std::min<long long>(std::max<long long>(steps, 1), std::max(1, RL_SG_GROUP_RAYS / batch));
-  const int nb = grid_for(batch, RL_SGT_ROWS);
+  const int nb = (batch + 63) / 64 * 64 / RL_SGT_ROWS;
   TRY(sg_reserve(s, group * batch));
   TRY(sg_reserve_train(s, batch, (size_t)group * nb));
   std::vector<float> part((size_t)group * nb);
@@ -1007,7 +1024,7 @@ int rl_surrogate_train(rl_surrogate* s, float max_range, long long n_pairs, int 
                     nullptr, n, 0));
     for (int j = 0; j < cnt; ++j) {
       TRY(sg_pass(s, s->d_rays + (size_t)j * batch, s->d_target + (size_t)j * batch, batch, max_range,
-                  s->d_partial + (size_t)j * nb, nullptr));
+                  s->d_partial + (size_t)j * nb));
       TRY((sg_update<true, true>(s, batch, lr)));
     }
     if (loss_curve) {
