@@ -277,9 +277,8 @@ __global__ void k_sg_features(const float4* __restrict__ rays, const float* __re
 // bf16 tile, rewritten in place by each layer).  The outputs are bitwise those
 // of k_sg_features followed by the per-layer GEMMs: the same feature
 // expression, the same matrix instructions over k in the same ascending order
-// from zero accumulators (16x16x32 for the hidden layers as in
-// k_gemm_bf16_nt, 16x16x16 for the heads as in k_gemm_bf16), the same bias /
-// relu / bf16 epilogue.  Each row's outputs depend on that row alone, so the
+// from zero accumulators (16x16x32, whose bits are those of the two 16x16x16
+// instructions of k_gemm_bf16), the same bias / relu / bf16 epilogue.  Each row's outputs depend on that row alone, so the
 // rows past n (zero features) are computed and never stored.
 #define RL_SG_TM 64
 #define RL_SG_ACT_PAD (RL_SG_H + 8)  // row stride in elements: 16-byte reads of 16 rows spread over the banks
@@ -301,6 +300,19 @@ __global__ void k_sg_bf16_check(unsigned long long* __restrict__ bad) {
     local += f2bf_hw(f) != f2bf(f) ? 1u : 0u;
   }
   if (local) atomicAdd(bad, local);
+}
+
+// Two floats rounded to bf16 (nearest even), v0 in the low half.
+__device__ __forceinline__ unsigned sg_pack2(float v0, float v1) {
+  return (unsigned)__builtin_bit_cast(bf16_t, (__bf16)v0) | ((unsigned)__builtin_bit_cast(bf16_t, (__bf16)v1) << 16);
+}
+
+// relu of two bf16: negative values have their sign bit set, so the signed
+// 16-bit maximum with 0 is relu (a NaN of the matrix instructions is positive
+// and stays).
+__device__ __forceinline__ unsigned sg_relu2(unsigned v) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(s2, v), s2{0, 0}));
 }
 
 // One hidden layer: act (64 x K) -> act (64 x 256), wave w computing columns
@@ -331,7 +343,7 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
     for (int i = 0; i < RT; ++i) {
       const sg_bf16x8 a = *(const sg_bf16x8*)(act + (i * 16 + r16) * RL_SG_ACT_PAD + s * 32 + kq);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, acc[i][j], 0, 0, 0);
     }
   }
   if (KN) {
@@ -339,18 +351,17 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
     for (int j = 0; j < 4; ++j) b0[j] = *(const sg_bf16x8*)(Wn + ((wave * 4 + j) * (KN / 32) * 64 + lane) * 8);
   }
   __syncthreads();  // every wave has read the layer's input before it is overwritten
+  // the weights are the first operand: lane l holds row l & 15 of a tile and its
+  // columns 4 (l >> 4) .. + 3, packed and stored together
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int n = nw + j * 16 + r16;
-    const float bb = sb[n];
+    const int c = nw + j * 16 + 4 * (lane >> 4);
+    const sg_float4 bb = *(const sg_float4*)(sb + c);
 #pragma unroll
     for (int i = 0; i < RT; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v = acc[i][j][q] + bb;
-        v = v < 0.0f ? 0.0f : v;
-        act[(i * 16 + 4 * (lane >> 4) + q) * RL_SG_ACT_PAD + n] = f2bf_hw(v);
-      }
+      *(uint2*)(act + (i * 16 + r16) * RL_SG_ACT_PAD + c) =
+          make_uint2(sg_relu2(sg_pack2(acc[i][j][0] + bb[0], acc[i][j][1] + bb[1])),
+                     sg_relu2(sg_pack2(acc[i][j][2] + bb[2], acc[i][j][3] + bb[3])));
   }
   __syncthreads();
 }
@@ -358,14 +369,16 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
 // rays: n x (x0, y0, sin h, cos h); P / Pf: the bf16 / fp32 parameter vectors, F
 // the weights in SgFrag order;
 // out: n x 2 fp32.  Launched with ceil(n / 64) workgroups of 256 threads.
-// Register use is held to 128 so that four waves share each SIMD (measured on
-// 240,000 rays: 3 waves, 144 registers, 5% slower).
+// Register use is held to 128 so that four waves share each SIMD (three: 91 us
+// for 240,000 rays, four: 81; 128 rays per workgroup: 107).  81 us are 0.88
+// PFLOP/s; a 8192^3 bf16 product reaches 1.19 on this card.  Without the weight
+// loads it takes 72 us, without the features 78.
 __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ rays, const float* __restrict__ freq,
                                                   float inv_w, float inv_h, const bf16_t* __restrict__ P,
                                                   const bf16_t* __restrict__ F, const float* __restrict__ Pf,
                                                   float* __restrict__ out, int n) {
   __shared__ __align__(16) bf16_t act[RL_SG_TM * RL_SG_ACT_PAD];
-  __shared__ float sbias[3 * RL_SG_H + RL_SG_OUT];         // b1, b2, b3, b4
+  __shared__ __align__(16) float sbias[3 * RL_SG_H + RL_SG_OUT];  // b1, b2, b3, b4
   __shared__ __align__(16) bf16_t sw4[RL_SG_OUT * RL_SG_H];  // W4
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int r0 = blockIdx.x * RL_SG_TM;
@@ -379,19 +392,23 @@ __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ 
   if (tid < RL_SG_OUT) sbias[3 * RL_SG_H + tid] = Pf[SgLayout::B4 + tid];
   sw4[tid] = P[SgLayout::W4 + tid];
   sw4[RL_SG_H + tid] = P[SgLayout::W4 + RL_SG_H + tid];
-  for (int e = tid; e < RL_SG_TM * RL_SG_NF; e += 256) {
-    const int r = e / RL_SG_NF, j = e - r * RL_SG_NF;
-    bf16_t s = 0, c = 0;
-    if (r0 + r < n) {
-      const float4 rr = rays[r0 + r];
-      const float v0 = rr.x * inv_w, v1 = rr.y * inv_h, v2 = rr.z, v3 = rr.w;
-      const float p = 6.283185307179586f * (freq[4 * j] * v0 + freq[4 * j + 1] * v1 + freq[4 * j + 2] * v2 +
-                                            freq[4 * j + 3] * v3);
-      s = f2bf(sinf(p));
-      c = f2bf(cosf(p));
+  {  // a thread's rows all take frequency tid % 32
+    const int j = tid & (RL_SG_NF - 1);
+    const float4 f = ((const float4*)freq)[j];
+#pragma unroll 2
+    for (int r = tid / RL_SG_NF; r < RL_SG_TM; r += 256 / RL_SG_NF) {
+      unsigned sc = 0;
+      if (r0 + r < n) {
+        const float4 rr = rays[r0 + r];
+        const float v0 = rr.x * inv_w, v1 = rr.y * inv_h, v2 = rr.z, v3 = rr.w;
+        const float p = 6.283185307179586f * (f.x * v0 + f.y * v1 + f.z * v2 + f.w * v3);
+        float s, c;
+        sincosf(p, &s, &c);
+        sc = (unsigned)f2bf_hw(s) | ((unsigned)f2bf_hw(c) << 16);
+      }
+      act[r * RL_SG_ACT_PAD + j] = (bf16_t)sc;
+      act[r * RL_SG_ACT_PAD + RL_SG_NF + j] = (bf16_t)(sc >> 16);
     }
-    act[r * RL_SG_ACT_PAD + j] = s;
-    act[r * RL_SG_ACT_PAD + RL_SG_NF + j] = c;
   }
   __syncthreads();
   sg_hidden_layer<RL_SG_F, RL_SG_H>(act, F + SgFrag::W1, sbias, F + SgFrag::W2, b0, wave, lane);
@@ -405,10 +422,11 @@ __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ 
     const int rt = (wave * (RL_SG_TM / 64) + t) * 16;
     sg_float4 acc = sg_float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < RL_SG_H; k += 16) {
-      const sg_short4 a = *(const sg_short4*)(act + (rt + col) * RL_SG_ACT_PAD + k + kb);
-      const sg_short4 b = col < RL_SG_OUT ? *(const sg_short4*)(sw4 + col * RL_SG_H + k + kb) : sg_short4{0, 0, 0, 0};
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    for (int k = 0; k < RL_SG_H; k += 32) {
+      const sg_bf16x8 a = *(const sg_bf16x8*)(act + (rt + col) * RL_SG_ACT_PAD + k + 2 * kb);
+      sg_bf16x8 b{};
+      if (col < RL_SG_OUT) b = *(const sg_bf16x8*)(sw4 + col * RL_SG_H + k + 2 * kb);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
     }
     if (col < RL_SG_OUT) {
       const float bb = sbias[3 * RL_SG_H + col];
@@ -485,14 +503,53 @@ __global__ void k_sg_rays_from_particles(MapDev m, TrigDev trig, const float* __
 #define RL_SG_CERT_STEP 8.0f  // largest gap between certificate samples (cells)
 #define RL_SG_PROBES 4
 #define RL_SG_PROBE_READS 64  // reads per probe before the ray is rejected
-__global__ __launch_bounds__(256) void k_sg_checked_march(MapDev m, float max_range,
+// Distances of N cells, d[j] that of cell(j, &px, &py) where it returns true,
+// else 0, all reads in flight together.  IDX8: from the compact map and its
+// tabulated distances in LDS (a code of 0 stands for any distance that ends a
+// march; escaped cells are read from the fp32 map), so the reads fall in a
+// quarter of the fp32 map's lines.
+template <bool IDX8, int N, class Cell>
+__device__ __forceinline__ void sg_dist_n(const MapDev& m, const float* dist, float (&d)[N], Cell cell) {
+  int px[N], py[N];
+  bool in[N];
+  unsigned c[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    in[j] = cell(j, &px[j], &py[j]);
+    if (IDX8)
+      c[j] = rl::idx8_code<false>(m, rl::Box{nullptr, 0, 0}, (unsigned)px[j], (unsigned)py[j]);  // off the map: any
+    else
+      d[j] = in[j] ? rl::glb(m.edt)[(size_t)px[j] * (unsigned)m.height + py[j]] : 0.0f;
+  }
+  if (!IDX8) return;
+  bool esc = false;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    d[j] = rl::lds(dist)[c[j]];
+    d[j] = in[j] ? d[j] : 0.0f;
+    esc |= in[j] & (c[j] == RL_IDX8_ESCAPE);
+  }
+  if (esc)
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (in[j] && c[j] == RL_IDX8_ESCAPE) d[j] = rl::glb(m.edt)[(size_t)px[j] * (unsigned)m.height + py[j]];
+}
+
+// One ray per lane.  240,000 rays are 3.7 waves per SIMD: registers are held to
+// 128 so that they are all resident (224 registers, with the distances read
+// from the fp32 map one after the other: 63 us; 38 so).
+template <bool IDX8>
+__global__ __launch_bounds__(256, 4) void k_sg_checked_march(MapDev m, float max_range,
                                                           const float4* __restrict__ rays,
                                                           const float* __restrict__ out, float bound_max,
                                                           float* __restrict__ ranges, float scale,
                                                           unsigned* __restrict__ stats, int n) {
-  __shared__ float lut[RL_LUT_SIZE];
+  __shared__ float lut[RL_LUT_SIZE], dist[RL_LUT_SIZE];
   __shared__ unsigned cnt[5];
-  for (int i = threadIdx.x; i < RL_LUT_SIZE; i += blockDim.x) lut[i] = m.steps[i];
+  for (int i = threadIdx.x; i < RL_LUT_SIZE; i += blockDim.x) {
+    lut[i] = m.steps[i];
+    dist[i] = m.steps[i - RL_LUT_SIZE];  // the distances stand before their steps (rl_ctx::d_lut)
+  }
   if (threadIdx.x < 5) cnt[threadIdx.x] = 0u;
   __syncthreads();
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -517,18 +574,20 @@ __global__ __launch_bounds__(256) void k_sg_checked_march(MapDev m, float max_ra
       const int nc = t0 > 0.0f ? (int)ceilf(t0 / RL_SG_CERT_STEP) : 0;
       const float gap = nc > 0 ? t0 / (float)nc : 0.0f;
       float dprev = 0.0f;
-      for (int k0 = 0; k0 <= nc; k0 += 16) {  // 16 independent reads in flight per round
+      // 16 independent reads in flight per round; the statistics count every sample,
+      // the rounds after the first that fails need no reading
+      reads += nc + 1;
+      rounds += nc / 16 + 1;
+      for (int k0 = 0; ok && k0 <= nc; k0 += 16) {
         float d[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        sg_dist_n<IDX8, 16>(m, dist, d, [&](int j, int* px, int* py) {
           const int k = k0 + j;
           const float tk = gap * (float)k;
           const float fx = x0 + dx * tk, fy = y0 + dy * tk;
-          const int px = (int)fx, py = (int)fy;
-          d[j] = 0.0f;  // off the map or in (-1, 0), where truncation is not floor: no certificate
-          if (k <= nc && fx >= 0.0f && fy >= 0.0f && (unsigned)px < W && (unsigned)py < H)
-            d[j] = rl::glb(m.edt)[(size_t)px * H + py];
-        }
+          *px = (int)fx, *py = (int)fy;
+          // off the map or in (-1, 0), where truncation is not floor: 0, no certificate
+          return k <= nc && fx >= 0.0f && fy >= 0.0f && (unsigned)*px < W && (unsigned)*py < H;
+        });
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int k = k0 + j;
@@ -536,10 +595,8 @@ __global__ __launch_bounds__(256) void k_sg_checked_march(MapDev m, float max_ra
           if (k <= nc) {
             if (!(d[j] > 0.0f) || (k > 0 && !(cover >= gap + 0.01f))) ok = false;
             dprev = d[j];
-            ++reads;
           }
         }
-        ++rounds;
       }
       // 2. probes from t0 at RL_SG_PROBES phases, marched side by side
       if (ok) {
@@ -553,27 +610,30 @@ __global__ __launch_bounds__(256) void k_sg_checked_march(MapDev m, float max_ra
         }
         for (int step = 0; step < RL_SG_PROBE_READS; ++step) {
           bool any = false;
-#pragma unroll
-          for (int k = 0; k < RL_SG_PROBES; ++k) {
+          float d[RL_SG_PROBES];
+          sg_dist_n<IDX8, RL_SG_PROBES>(m, dist, d, [&](int k, int* px, int* py) {
             // a probe past its window (r + b + 2), max_range or the map ends
             // without a hit (1)
-            const int px = (int)(x0 + dx * tp[k]), py = (int)(y0 + dy * tp[k]);
-            const bool inb = (unsigned)px < W && (unsigned)py < H;
+            *px = (int)(x0 + dx * tp[k]), *py = (int)(y0 + dy * tp[k]);
+            const bool inb = (unsigned)*px < W && (unsigned)*py < H;
             if (ep[k] == 0 && (!(tp[k] < max_range) || tp[k] > t_end || !inb)) ep[k] = 1;
+            return ep[k] == 0;
+          });
+#pragma unroll
+          for (int k = 0; k < RL_SG_PROBES; ++k)
             if (ep[k] == 0) {
-              const float d = rl::glb(m.edt)[(size_t)px * H + py];
               ++reads;
               any = true;
-              if (d <= 0.0f) {
+              if (d[k] <= 0.0f) {
+                const int px = (int)(x0 + dx * tp[k]), py = (int)(y0 + dy * tp[k]);
                 const float xd = (float)px - x0, yd = (float)py - y0;
                 rp[k] = __builtin_sqrtf(xd * xd + yd * yd);
                 ep[k] = 2;
               } else {
-                const float st = d * 0.999f;
+                const float st = d[k] * 0.999f;
                 tp[k] += (st < 1.0f) ? 1.0f : st;
               }
             }
-          }
           if (!any) break;
           ++rounds;
         }
@@ -586,7 +646,7 @@ __global__ __launch_bounds__(256) void k_sg_checked_march(MapDev m, float max_ra
     }
     if (result < 0.0f) {
       int c = 0;
-      result = (m.idx8 && rl::fast_march_ok(x0, y0, max_range))
+      result = (IDX8 && rl::fast_march_ok(x0, y0, max_range))
                    ? rl::rm_march_idx8<true>(m, lut, rl::Box{nullptr, 0, 0}, max_range, x0, y0, dx, dy, &c)
                    : rl::rm_march<true>(m.edt, m.width, m.height, max_range, x0, y0, dx, dy, &c);
       reads += c;
@@ -1067,9 +1127,9 @@ int rl_surrogate_calc_range_angles_dev(rl_surrogate* s, float max_range, const f
                      d_angles, N, M, s->d_rays);
   HIP_TRY(hipGetLastError());
   TRY(sg_infer(s, n));
-  hipLaunchKernelGGL(k_sg_checked_march, dim3(grid_for(n, 256)), dim3(256), 0, st, md, max_range,
-                     (const float4*)s->d_rays, (const float*)s->d_out, bound_max, d_ranges, md.world.scale,
-                     s->d_stats, n);
+  hipLaunchKernelGGL(md.idx8 ? k_sg_checked_march<true> : k_sg_checked_march<false>, dim3(grid_for(n, 256)), dim3(256),
+                     0, st, md, max_range, (const float4*)s->d_rays, (const float*)s->d_out, bound_max, d_ranges,
+                     md.world.scale, s->d_stats, n);
   HIP_TRY(hipGetLastError());
   if (stats) {
     HIP_TRY(hipMemcpyAsync(stats, s->d_stats, 5 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
