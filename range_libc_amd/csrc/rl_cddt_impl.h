@@ -36,41 +36,51 @@ __global__ void k_cddt_consts(TrigDev trig, int td, int W, int H, float m2pi_div
   trans[a] = (float)(t > 0.0 ? t : 0.0);  // std::max(0.0, t)
 }
 
-// 2. Edge cells, compacted into `list` (one atomic per wave).
-__global__ void k_cddt_edges(const uint8_t* __restrict__ occ, int W, int H, int* __restrict__ list,
-                             unsigned* __restrict__ n_out) {
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;  // W * H < 2^31 (checked by the caller)
-  bool e = false;
-  if (i < (unsigned)W * (unsigned)H) {
-    const int x = (int)(i / (unsigned)H), y = (int)(i - (unsigned)x * (unsigned)H);
-    if (occ[i]) {
-      const int dx[8] = {1, -1, 0, 0, 1, -1, 1, -1}, dy[8] = {0, 0, 1, -1, 1, 1, -1, -1};
-      for (int k = 0; k < 8; ++k) {
-        const int cx = x + dx[k], cy = y + dy[k];
-        if (0 <= cx && 0 <= cy && cx < W && cy < H && !occ[(size_t)cx * H + cy]) {
-          e = true;
-          break;
-        }
-      }
-    }
-  }
-  const unsigned long long mask = __ballot(e);
+// 2. Edge cells as (x << 16) | y (sides are below 65536), in any order.  A
+// workgroup gathers the edge cells of 4096 in LDS and takes their place in the
+// list with one atomic: with one per wave, 65,536 atomics on one address took
+// 0.65 ms for a 2048^2 map; 0.04 so.
+#define RL_CDDT_EDGE_ITEMS 16
+__global__ __launch_bounds__(256) void k_cddt_edges(const uint8_t* __restrict__ occ, int W, int H,
+                                                    unsigned* __restrict__ list, unsigned* __restrict__ n_out) {
+  __shared__ unsigned found[256 * RL_CDDT_EDGE_ITEMS];
+  __shared__ unsigned cnt, base;
+  if (threadIdx.x == 0) cnt = 0;
+  __syncthreads();
+  const unsigned n = (unsigned)W * (unsigned)H;  // < 2^31 (checked by the caller)
+  const unsigned first = blockIdx.x * (256 * RL_CDDT_EDGE_ITEMS) + threadIdx.x;
   const int lane = threadIdx.x & 63;
-  unsigned base = 0;
-  if (lane == 0 && mask) base = atomicAdd(n_out, (unsigned)__popcll(mask));
-  base = __shfl(base, 0);
-  if (e) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = (int)i;
+  for (int k = 0; k < RL_CDDT_EDGE_ITEMS; ++k) {
+    const unsigned i = first + (unsigned)k * 256u;
+    bool e = false;
+    int x = 0, y = 0;
+    if (i < n && occ[i]) {
+      x = (int)(i / (unsigned)H), y = (int)(i - (unsigned)x * (unsigned)H);
+      const uint8_t* c = occ + i;
+      const bool l = x > 0, r = x + 1 < W, d = y > 0, u = y + 1 < H;
+      e = (r && !c[H]) || (l && !*(c - H)) || (u && !c[1]) || (d && !*(c - 1)) || (r && u && !c[H + 1]) ||
+          (l && u && !*(c - H + 1)) || (r && d && !c[H - 1]) || (l && d && !*(c - H - 1));
+    }
+    const unsigned long long m = __ballot(e);
+    unsigned at = 0;
+    if (lane == 0 && m) at = atomicAdd(&cnt, (unsigned)__popcll(m));
+    at = __shfl(at, 0);
+    if (e) found[at + __popcll(m & ((1ull << lane) - 1ull))] = ((unsigned)x << 16) | (unsigned)y;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) base = atomicAdd(n_out, cnt);
+  __syncthreads();
+  for (unsigned i = threadIdx.x; i < cnt; i += 256) list[base + i] = found[i];
 }
 
-// Footprint of edge cell `cell` (x * H + y) at angle a (RangeLib.h:1096-1115):
-// the projected centre and the bins [lower, upper] it is stored in.
+// Footprint of an edge cell at angle a (RangeLib.h:1096-1115): the projected
+// centre and the bins [lower, upper] it is stored in.
 struct CddtProj {
   float cx;
   int lower, upper;
 };
-__device__ __forceinline__ CddtProj cddt_project(int cell, int H, float cs, float sn, float tr) {
-  const int x = cell / H, y = cell - (cell / H) * H;
-  const float px = (float)(x + 0.5), py = (float)(y + 0.5);
+__device__ __forceinline__ CddtProj cddt_project(unsigned cell, float cs, float sn, float tr) {
+  const float px = (float)(cell >> 16) + 0.5f, py = (float)(cell & 0xffffu) + 0.5f;  // exact
   const float half = (float)((double)(fabsf(sn) + fabsf(cs)) / 2.0);
   CddtProj p;
   p.cx = px * cs - py * sn;
@@ -80,15 +90,69 @@ __device__ __forceinline__ CddtProj cddt_project(int cell, int H, float cs, floa
   return p;
 }
 
-// 3. Counting (fill == false) or filling (fill == true) pass; one thread per
-// (edge cell, angle): angle a0 + blockIdx.y, edge cells along blockIdx.x (the
-// edge list holds runs of neighbouring cells, one run per wave of
-// k_cddt_edges), so a wave's lanes mostly project nearby cells under one angle.
+// 3. Counting (FILL == false) and filling (FILL == true) passes over the (edge
+// cell, angle) pairs.  A workgroup takes one angle and one of G chunks of the
+// edge list and counts into the angle's bins in LDS (up to RL_CDDT_LDS_BINS of
+// them): the first pass stores the chunk's counts, k_cddt_chunks turns them into
+// each chunk's offsets in the bins, and the second pass starts its LDS cursors
+// there.  All chunks of an angle run on one XCD (workgroup b is on XCD b mod 8),
+// so an angle's entries, about 1 MB at 2048^2, are put together in its L2.
+// 2048^2 corridor map, 54 headings, 32.9 M entries: 1.00 + 1.19 ms with an atomic
+// on a 64-bit counter in memory per entry and pass; 0.05 + 0.27 so.
 // Bins outside [0, width) are skipped (the reference would write outside its
 // table; it does not happen for maps whose edge cells project inside the
 // rotated bounding box, which the translation and width are built to cover).
+#define RL_CDDT_LDS_BINS 16384  // 64 KB: maps of up to about 11,500 cells a side
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_cddt_scatter(const int* __restrict__ edges, int n_edges, int a0, int H,
+__global__ __launch_bounds__(256) void k_cddt_hist(const unsigned* __restrict__ edges, int n_edges, int nang, int G,
+                                                   const int* __restrict__ width, const float* __restrict__ trans,
+                                                   const float* __restrict__ cosv, const float* __restrict__ sinv,
+                                                   const long long* __restrict__ bin_off,
+                                                   const long long* __restrict__ start, unsigned* __restrict__ chunks,
+                                                   long long nb, float* __restrict__ vals) {
+  extern __shared__ unsigned bins[];
+  const int k = (int)(blockIdx.x >> 3);
+  const int a = (int)(blockIdx.x & 7) + 8 * (k / G), g = k % G;
+  if (a >= nang) return;  // the same in every thread
+  const int w = width[a];
+  const long long off = bin_off[a];
+  unsigned* mine = chunks + (size_t)g * (size_t)nb + off;
+  for (int b = threadIdx.x; b < w; b += 256) bins[b] = FILL ? (unsigned)start[off + b] + mine[b] : 0u;
+  __syncthreads();
+  const float cs = cosv[a], sn = sinv[a], tr = trans[a];
+  const int per = (n_edges + G - 1) / G, e0 = g * per, e1 = min(n_edges, e0 + per);
+  for (int e = e0 + (int)threadIdx.x; e < e1; e += 256) {
+    const CddtProj p = cddt_project(edges[e], cs, sn, tr);
+    for (int b = p.lower; b <= p.upper; ++b) {
+      if (b < 0 || b >= w) continue;
+      const unsigned pos = atomicAdd(&bins[b], 1u);
+      if (FILL) vals[pos] = p.cx;
+    }
+  }
+  if (FILL) return;
+  __syncthreads();
+  for (int b = threadIdx.x; b < w; b += 256) mine[b] = bins[b];
+}
+
+// Per bin (the first nba of nb): the chunks' counts become their offsets in the
+// bin, their sum the bin's count.
+__global__ __launch_bounds__(256) void k_cddt_chunks(unsigned* __restrict__ chunks, int G, long long nb,
+                                                     unsigned long long* __restrict__ counts, long long nba) {
+  const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nba) return;
+  unsigned s = 0;
+  for (int g = 0; g < G; ++g) {
+    const unsigned c = chunks[(size_t)g * (size_t)nb + b];
+    chunks[(size_t)g * (size_t)nb + b] = s;
+    s += c;
+  }
+  counts[b] = s;
+}
+
+// The same passes for maps whose angles have more bins than LDS holds: one
+// thread per (edge cell, angle a0 + blockIdx.y), counting in memory.
+template <bool FILL>
+__global__ __launch_bounds__(256) void k_cddt_scatter(const unsigned* __restrict__ edges, int n_edges, int a0,
                                                       const int* __restrict__ width, const float* __restrict__ trans,
                                                       const float* __restrict__ cosv, const float* __restrict__ sinv,
                                                       const long long* __restrict__ bin_off,
@@ -97,7 +161,7 @@ __global__ __launch_bounds__(256) void k_cddt_scatter(const int* __restrict__ ed
   const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (e >= n_edges) return;
   const int a = a0 + (int)blockIdx.y;
-  const CddtProj p = cddt_project(edges[e], H, cosv[a], sinv[a], trans[a]);
+  const CddtProj p = cddt_project(edges[e], cosv[a], sinv[a], trans[a]);
   for (int b = p.lower; b <= p.upper; ++b) {
     if (b < 0 || b >= width[a]) continue;
     const unsigned long long pos = atomicAdd(&counter[bin_off[a] + b], 1ull);
@@ -105,68 +169,160 @@ __global__ __launch_bounds__(256) void k_cddt_scatter(const int* __restrict__ ed
   }
 }
 
-// 4./5. Per bin: count the entries kept (COPY == false) or copy them to their
-// new place (COPY == true).  mode 0 keeps the first of each run of equal
-// values (after sorting), mode 1 keeps the entries marked used.
+// 4./5. One wave per bin: count the entries kept (COPY == false) or copy them to
+// their new place (COPY == true).  mode 0 keeps the first of each run of equal
+// values (after sorting), mode 1 keeps the entries marked used.  Lanes take
+// consecutive entries, so a bin's loads are whole lines (one thread per bin read
+// 4 bytes of a line at a time: 0.47 and 0.95 ms on the 2048^2 corridor map with 108
+// headings; 0.07 and 0.08 ms so).
 template <bool COPY>
-__global__ void k_cddt_compact(long long nb, const long long* __restrict__ start, const float* __restrict__ vals,
-                               const uint8_t* __restrict__ used, int mode,
-                               const long long* __restrict__ new_start, long long* __restrict__ kept,
-                               float* __restrict__ out) {
-  const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_cddt_compact(long long nb, const long long* __restrict__ start,
+                                                      const float* __restrict__ vals, const uint8_t* __restrict__ used,
+                                                      int mode, const long long* __restrict__ new_start,
+                                                      long long* __restrict__ kept, float* __restrict__ out) {
+  const long long b = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (b >= nb) return;
   const long long s = start[b], e = start[b + 1];
-  long long o = COPY ? new_start[b] : 0, k = 0;
-  for (long long j = s; j < e; ++j) {
-    const bool keep = mode == 0 ? (j == s || vals[j] != vals[j - 1]) : used[j] != 0;
-    if (!keep) continue;
-    if (COPY) out[o++] = vals[j];
-    ++k;
+  long long o = COPY ? new_start[b] : 0;
+  for (long long j0 = s; j0 < e; j0 += 64) {
+    const long long j = j0 + lane;
+    bool keep = false;
+    float v = 0.0f;
+    if (j < e) {
+      v = vals[j];
+      keep = mode == 0 ? (j == s || v != vals[j - 1]) : used[j] != 0;
+    }
+    const unsigned long long m = __ballot(keep);
+    if (COPY && keep) out[o + __popcll(m & ((1ull << lane) - 1ull))] = v;
+    o += __popcll(m);
   }
-  if (!COPY) kept[b] = k;
+  if (!COPY && lane == 0) kept[b] = o;
 }
 
-// 5. Prune marks (RangeLib.h:1172-1275), one thread per (cell, angle): angle
-// a = blockIdx.y, cells x-major along blockIdx.x, so the lanes of a wave are
-// neighbouring cells of one column under one angle and look up neighbouring
-// bins.  Where the reference's linear search leaves its index unset (no entry
-// at or beyond the cell), the lower_bound value is taken, as its binary search.
-// W * H < 2^31 (checked when the tables are built).
-__global__ __launch_bounds__(256) void k_cddt_prune_mark(const uint8_t* __restrict__ occ, int W, int H, float max_range,
+// 5. Prune marks (RangeLib.h:1172-1275).  In the reference every free cell looks
+// up its bin under every angle and marks the entries around it: the first entry
+// at or beyond its projection and the one before (where the reference's linear
+// search leaves its index unset, the lower_bound value is taken, as its binary
+// search; past the last entry that entry is marked whatever max_range is).  So
+// entry i is used exactly when a free cell of the bin's strip projects into
+// (v[i - 1], v[i]] or (v[i], v[i + 1]] (unbounded at the ends), and one such cell
+// per interval is enough: a lane takes an interval and walks the cells of the
+// strip that can project into it until it finds a free one.  The walk's bounds
+// are real geometry with a margin far above float rounding; a cell counts only
+// if its own float projection (the reference's expressions) falls in the bin and
+// the interval.  2048^2 corridor map, 108 headings: one lookup
+// (binary search) per cell and angle, 226 M of them, took 4.65 ms; 0.46 so
+// (0.96 with every lane walking its interval to the end).
+// One wave per bin, angle blockIdx.y; used[i] of every entry is written, and the
+// bin's number of used entries.
+__global__ __launch_bounds__(256) void k_cddt_prune_mark(const uint8_t* __restrict__ occ, int W, int H,
                                                          const int* __restrict__ width, const float* __restrict__ trans,
                                                          const float* __restrict__ cosv, const float* __restrict__ sinv,
                                                          const long long* __restrict__ bin_off,
                                                          const long long* __restrict__ start,
                                                          const float* __restrict__ vals, uint8_t* __restrict__ used,
-                                                         int a0) {
-  const unsigned cell = blockIdx.x * blockDim.x + threadIdx.x;
-  if (cell >= (unsigned)W * (unsigned)H) return;
-  if (occ[cell]) return;  // (every exit below leaves no mark, so the order of the tests is free)
+                                                         long long* __restrict__ kept, int a0) {
   const int a = a0 + (int)blockIdx.y;
-  const int x = (int)(cell / (unsigned)H), y = (int)(cell - (unsigned)x * (unsigned)H);
-  const float fx = (float)(0.5 + x), fy = (float)(0.5 + y);
-  const float cs = cosv[a], sn = sinv[a];
-  const float lx = fx * cs - fy * sn;
-  const float ly = (fx * sn + fy * cs) + trans[a];
-  const unsigned li = (unsigned)rl::trunc_x86(ly);
+  const unsigned li = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (li >= (unsigned)width[a]) return;
   const long long b = bin_off[a] + li, s = start[b];
   const int n = (int)(start[b + 1] - s);  // fewer than 2^31 entries in all (checked at build)
-  const float* v = vals + s;
-  uint8_t* u = used + s;
-  const int high = n - 1;
-  if (high == -1) return;
-  if (v[high] < lx && lx - v[high] < max_range) {
-    u[high] = 1;
+  if (n == 0) {
+    if (lane == 0) kept[b] = 0;
     return;
   }
-  int lo = 0, hi = n;  // lower_bound
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (v[mid] < lx) lo = mid + 1; else hi = mid;
+  const float* v = vals + s;
+  const float cs = cosv[a], sn = sinv[a], tr = trans[a];
+  // a cell centre (fx, fy) is at lx = fx cs - fy sn along the strip and l = fx sn +
+  // fy cs across it, l in [l0, l1) up to rounding; fx = lx cs + l sn, fy = l cs - lx sn
+  const float mg = 0.05f + 4.0e-6f * (float)(W + H);
+  // (bin 0 also takes the projections that truncate to it from (-1, 0))
+  const float l0 = (li ? (float)li : -1.0f) - tr - mg, l1 = (float)li - tr + 1.0f + mg;
+  // p: the axis along which the strip advances fastest, q the other; np, nq their
+  // sizes.  l = fp * kp + fq * kq with |kq| >= 0.7
+  const bool along_x = fabsf(cs) >= fabsf(sn);
+  const float kp = along_x ? sn : cs, kq = along_x ? cs : sn;
+  const int np = along_x ? W : H, nq = along_x ? H : W;
+  const float inv_kq = 1.0f / kq;
+  // positions p for which the strip crosses the map: fp in [0, np], fp * kp = l - fq * kq
+  float pmin = 0.0f, pmax = (float)np;
+  if (fabsf(kp) > 1.0e-3f) {
+    const float e = (float)nq * kq;
+    const float u = l0 - fmaxf(e, 0.0f), w = l1 - fminf(e, 0.0f);
+    const float r0 = u / kp, r1 = w / kp;
+    pmin = fmaxf(pmin, fminf(r0, r1) - 1.0f);
+    pmax = fminf(pmax, fmaxf(r0, r1) + 1.0f);
   }
-  if (lo < n) u[lo] = 1;
-  if (lo >= 1) u[lo - 1] = 1;
+  // lx's part of fp: along x fp = lx cs + l sn, along y fp = -lx sn + l cs
+  const float kx = along_x ? cs : -sn, kl = along_x ? sn : cs;
+  const float lmin = fminf(l0 * kl, l1 * kl) - mg, lmax = fmaxf(l0 * kl, l1 * kl) + mg;
+  // whether a free cell at position p of the strip projects into (lo, hi]
+  auto column = [&](int p, float lo, float hi) {
+    const float fp = (float)p + 0.5f;
+    const float c0 = (l0 - fp * kp) * inv_kq, c1 = (l1 - fp * kp) * inv_kq;
+    const int q0 = max(0, (int)ceilf(fminf(c0, c1) - 0.5f)), q1 = min(nq - 1, (int)floorf(fmaxf(c0, c1) - 0.5f));
+    for (int q = q0; q <= q1; ++q) {
+      const int x = along_x ? p : q, y = along_x ? q : p;
+      const float fx = (float)x + 0.5f, fy = (float)y + 0.5f;  // (exact, as the reference's 0.5 + x in double)
+      const float lx = fx * cs - fy * sn;
+      const float ly = (fx * sn + fy * cs) + tr;
+      if (lx > lo && lx <= hi && (unsigned)rl::trunc_x86(ly) == li && !occ[(size_t)x * (unsigned)H + (unsigned)y])
+        return true;
+    }
+    return false;
+  };
+  // orders a wave's LDS accesses
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  __shared__ int sel[4][8];
+  int* slot = sel[threadIdx.x >> 6];
+  long long cnt = 0;
+  // 64 intervals a round, the last of them again the first of the next round:
+  // entry i is used by intervals i and i + 1
+  for (int i0 = 0; i0 < n; i0 += 63) {
+    const int i = i0 + lane;
+    bool found = false;
+    int p = 0, p1 = -1;
+    float lo = 0.0f, hi = 0.0f;
+    if (i <= n) {
+      lo = i > 0 ? v[i - 1] : -FLT_MAX, hi = i < n ? v[i] : FLT_MAX;
+      const float g0 = lo * kx, g1 = hi * kx;
+      const float f0 = fmaxf(pmin, fminf(g0, g1) + lmin), f1 = fminf(pmax, fmaxf(g0, g1) + lmax);
+      p = max(0, (int)ceilf(f0 - 0.5f)), p1 = min(np - 1, (int)floorf(f1 - 0.5f));
+      for (int k = 0; k < 2 && p <= p1 && !found; ++k, ++p) found = column(p, lo, hi);
+    }
+    // the few lanes that are left cross a wall or a solid block: eight of them at a
+    // time are helped by eight lanes each, which take the next eight positions
+    for (;;) {  // the same in every lane
+      const bool left = !found && p <= p1;
+      const unsigned long long lm = __ballot(left);
+      if (!lm) break;
+      const int rank = __popcll(lm & ((1ull << lane) - 1ull)), grp = lane >> 3;
+      if (left && rank < 8) slot[rank] = lane;
+      wave_sync();
+      const int owner = grp < __popcll(lm) ? slot[grp] : lane;
+      wave_sync();  // read before the next round's writes
+      const float olo = __shfl(lo, owner), ohi = __shfl(hi, owner);
+      const int op = __shfl(p, owner) + (lane & 7), op1 = __shfl(p1, owner);
+      const bool hit = grp < __popcll(lm) && op <= op1 && column(op, olo, ohi);
+      const unsigned long long hm = __ballot(hit);
+      if (left && rank < 8) {
+        found = (hm >> (8 * rank)) & 0xffull;
+        p += 8;
+      }
+    }
+    const unsigned long long f = __ballot(found);
+    const unsigned long long u = (f | (f >> 1)) & 0x7fffffffffffffffull;  // entries i0 .. i0 + 62
+    const bool mine = lane < 63 && i < n;
+    if (mine) used[s + i] = (uint8_t)((u >> lane) & 1ull);
+    cnt += __popcll(u & __ballot(mine));
+  }
+  if (lane == 0) kept[b] = cnt;
 }
 
 // RangeMethod::calc_range_many_radial_optimized (RangeLib.h:616-676), one
@@ -260,26 +416,20 @@ int scan_counts(hipStream_t st, const unsigned long long* counts, long long* out
   return exclusive_sum_u64(st, counts, (unsigned long long*)out, n + 1);
 }
 
-// Keeps the entries selected by `mode` (see k_cddt_compact): new start and values.
-int cddt_compact(rl_map* m, int mode, const uint8_t* used) {
+// Keeps the entries selected by `mode` (see k_cddt_compact): new start and
+// values.  kept: the bins' numbers of entries to keep (nb + 1, the last 0).
+int cddt_compact(rl_map* m, int mode, const uint8_t* used, const DevBuf& kept) {
   hipStream_t st = m->ctx->stream;
   const long long nb = m->cddt_nb;
-  DevBuf kept, nstart, nvals;
-  TRY(kept.alloc((size_t)(nb + 1) * sizeof(unsigned long long)));
+  DevBuf nstart, nvals;
   TRY(nstart.alloc((size_t)(nb + 1) * sizeof(long long)));
-  HIP_TRY(hipMemsetAsync(kept.p, 0, (size_t)(nb + 1) * sizeof(unsigned long long), st));
-  const unsigned g = (unsigned)grid_for(nb, 256);
-  hipLaunchKernelGGL(k_cddt_compact<false>, dim3(g), dim3(256), 0, st, nb, (const long long*)m->cddt_start,
-                     (const float*)m->cddt_vals, used, mode, (const long long*)nullptr, kept.as<long long>(),
-                     (float*)nullptr);
-  HIP_TRY(hipGetLastError());
   TRY(scan_counts(st, kept.as<unsigned long long>(), nstart.as<long long>(), nb));
   long long total = 0;
   HIP_TRY(hipMemcpy(&total, nstart.as<long long>() + nb, sizeof(long long), hipMemcpyDeviceToHost));
   TRY(nvals.alloc((size_t)total * sizeof(float)));
-  hipLaunchKernelGGL(k_cddt_compact<true>, dim3(g), dim3(256), 0, st, nb, (const long long*)m->cddt_start,
-                     (const float*)m->cddt_vals, used, mode, (const long long*)nstart.p, (long long*)nullptr,
-                     nvals.as<float>());
+  hipLaunchKernelGGL(k_cddt_compact<true>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
+                     (const long long*)m->cddt_start, (const float*)m->cddt_vals, used, mode, (const long long*)nstart.p,
+                     (long long*)nullptr, nvals.as<float>());
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
   (void)hipFree(m->cddt_start);
@@ -288,6 +438,14 @@ int cddt_compact(rl_map* m, int mode, const uint8_t* used) {
   m->cddt_vals = nvals.as<float>();
   nstart.p = nvals.p = nullptr;
   m->cddt_nv = total;
+  return RL_OK;
+}
+
+// nb + 1 zeroed counts.
+int cddt_counts(rl_map* m, DevBuf* kept) {
+  const size_t bytes = (size_t)(m->cddt_nb + 1) * sizeof(unsigned long long);
+  TRY(kept->alloc(bytes));
+  HIP_TRY(hipMemsetAsync(kept->p, 0, bytes, m->ctx->stream));
   return RL_OK;
 }
 
@@ -322,41 +480,61 @@ int cddt_build_locked(rl_map* m, int td) {
   // edge cells
   const long long N = (long long)W * H;
   DevBuf edges, n_edges;
-  TRY(edges.alloc((size_t)N * sizeof(int)));
+  TRY(edges.alloc((size_t)N * sizeof(unsigned)));
   TRY(n_edges.alloc(sizeof(unsigned)));
   HIP_TRY(hipMemsetAsync(n_edges.p, 0, sizeof(unsigned), st));
-  hipLaunchKernelGGL(k_cddt_edges, dim3(grid_for(N, 256)), dim3(256), 0, st, (const uint8_t*)m->d_occ, W, H,
-                     edges.as<int>(), n_edges.as<unsigned>());
+  hipLaunchKernelGGL(k_cddt_edges, dim3(grid_for(N, 256 * RL_CDDT_EDGE_ITEMS)), dim3(256), 0, st,
+                     (const uint8_t*)m->d_occ, W, H, edges.as<unsigned>(), n_edges.as<unsigned>());
   HIP_TRY(hipGetLastError());
   unsigned ne = 0;
   HIP_TRY(hipMemcpyAsync(&ne, n_edges.p, sizeof(unsigned), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  // count, scan, fill
-  DevBuf counter;
-  TRY(counter.alloc((size_t)(nb + 1) * sizeof(unsigned long long)));
-  HIP_TRY(hipMemsetAsync(counter.p, 0, (size_t)(nb + 1) * sizeof(unsigned long long), st));
-  const long long pairs = (long long)ne * nang;
-  if (pairs > 0) {
-    for (int a0 = 0; a0 < nang; a0 += 65535) {  // grid rows: at most 65535 angles per launch
-      hipLaunchKernelGGL(k_cddt_scatter<false>, dim3(grid_for(ne, 256), (unsigned)std::min(65535, nang - a0)),
-                         dim3(256), 0, st, (const int*)edges.p, (int)ne, a0, H, (const int*)m->cddt_width,
-                         (const float*)m->cddt_trans, (const float*)m->cddt_cos, (const float*)m->cddt_sin,
-                         (const long long*)m->cddt_bin_off, counter.as<unsigned long long>(), (float*)nullptr);
-      HIP_TRY(hipGetLastError());
-    }
+  // count, scan, fill.  In LDS where an angle's bins fit; about 1024 workgroups,
+  // each of at least 2048 edge cells and at most 32 chunks of an angle
+  DevBuf counter, chunks;
+  TRY(cddt_counts(m, &counter));
+  const int max_width = *std::max_element(widths.begin(), widths.end());
+  const bool in_lds = max_width <= RL_CDDT_LDS_BINS;
+  const int G = std::max(1, std::min(std::min(32, 1024 / nang + 1), (int)(ne / 2048u)));
+  const unsigned hist_grid = 8u * (unsigned)((nang + 7) / 8) * (unsigned)G;
+  const unsigned hist_lds = (unsigned)max_width * sizeof(unsigned);
+  if (ne && in_lds) {
+    const long long nba = off[nang];  // the bins of the angles that hold entries
+    TRY(chunks.alloc((size_t)G * (size_t)nb * sizeof(unsigned)));
+    hipLaunchKernelGGL(k_cddt_hist<false>, dim3(hist_grid), dim3(256), hist_lds, st, (const unsigned*)edges.p, (int)ne,
+                       nang, G, (const int*)m->cddt_width, (const float*)m->cddt_trans, (const float*)m->cddt_cos,
+                       (const float*)m->cddt_sin, (const long long*)m->cddt_bin_off, (const long long*)nullptr,
+                       chunks.as<unsigned>(), nb, (float*)nullptr);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_cddt_chunks, dim3((unsigned)grid_for(nba, 256)), dim3(256), 0, st, chunks.as<unsigned>(), G, nb,
+                       counter.as<unsigned long long>(), nba);
+    HIP_TRY(hipGetLastError());
+  }
+  for (int a0 = 0; ne && !in_lds && a0 < nang; a0 += 65535) {  // grid rows: at most 65535 angles per launch
+    hipLaunchKernelGGL(k_cddt_scatter<false>, dim3(grid_for(ne, 256), (unsigned)std::min(65535, nang - a0)), dim3(256),
+                       0, st, (const unsigned*)edges.p, (int)ne, a0, (const int*)m->cddt_width,
+                       (const float*)m->cddt_trans, (const float*)m->cddt_cos, (const float*)m->cddt_sin,
+                       (const long long*)m->cddt_bin_off, counter.as<unsigned long long>(), (float*)nullptr);
+    HIP_TRY(hipGetLastError());
   }
   HIP_TRY(hipMalloc(&m->cddt_start, (size_t)(nb + 1) * sizeof(long long)));
   TRY(scan_counts(st, counter.as<unsigned long long>(), m->cddt_start, nb));
   long long total = 0;
   HIP_TRY(hipMemcpy(&total, m->cddt_start + nb, sizeof(long long), hipMemcpyDeviceToHost));
   if (total > 0x7fffffffLL) return fail(RL_ERR_ARG, "CDDT: %lld table entries exceed 2^31", total);
-  HIP_TRY(hipMemcpy(counter.p, m->cddt_start, (size_t)(nb + 1) * sizeof(long long), hipMemcpyDeviceToDevice));
   DevBuf raw;
   TRY(raw.alloc((size_t)total * sizeof(float)));
-  if (pairs > 0) {
-    for (int a0 = 0; a0 < nang; a0 += 65535) {  // grid rows: at most 65535 angles per launch
-      hipLaunchKernelGGL(k_cddt_scatter<true>, dim3(grid_for(ne, 256), (unsigned)std::min(65535, nang - a0)),
-                         dim3(256), 0, st, (const int*)edges.p, (int)ne, a0, H, (const int*)m->cddt_width,
+  if (ne && in_lds) {
+    hipLaunchKernelGGL(k_cddt_hist<true>, dim3(hist_grid), dim3(256), hist_lds, st, (const unsigned*)edges.p, (int)ne,
+                       nang, G, (const int*)m->cddt_width, (const float*)m->cddt_trans, (const float*)m->cddt_cos,
+                       (const float*)m->cddt_sin, (const long long*)m->cddt_bin_off, (const long long*)m->cddt_start,
+                       chunks.as<unsigned>(), nb, raw.as<float>());
+    HIP_TRY(hipGetLastError());
+  } else if (ne) {
+    HIP_TRY(hipMemcpy(counter.p, m->cddt_start, (size_t)(nb + 1) * sizeof(long long), hipMemcpyDeviceToDevice));
+    for (int a0 = 0; a0 < nang; a0 += 65535) {
+      hipLaunchKernelGGL(k_cddt_scatter<true>, dim3(grid_for(ne, 256), (unsigned)std::min(65535, nang - a0)), dim3(256),
+                         0, st, (const unsigned*)edges.p, (int)ne, a0, (const int*)m->cddt_width,
                          (const float*)m->cddt_trans, (const float*)m->cddt_cos, (const float*)m->cddt_sin,
                          (const long long*)m->cddt_bin_off, counter.as<unsigned long long>(), raw.as<float>());
       HIP_TRY(hipGetLastError());
@@ -367,25 +545,34 @@ int cddt_build_locked(rl_map* m, int td) {
   if (total > 0) TRY(segmented_sort_f32(st, raw.as<float>(), m->cddt_vals, m->cddt_start, nb));
   m->cddt_nv = total;
   // drop duplicates
-  return cddt_compact(m, 0, nullptr);
+  DevBuf kept;
+  TRY(cddt_counts(m, &kept));
+  hipLaunchKernelGGL(k_cddt_compact<false>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
+                     (const long long*)m->cddt_start, (const float*)m->cddt_vals, (const uint8_t*)nullptr, 0,
+                     (const long long*)nullptr, kept.as<long long>(), (float*)nullptr);
+  HIP_TRY(hipGetLastError());
+  return cddt_compact(m, 0, nullptr, kept);
 }
 
-int cddt_prune_locked(rl_map* m, float max_range) {
+// CDDTCast::prune: max_range does not change which entries stay (k_cddt_prune_mark).
+int cddt_prune_locked(rl_map* m) {
   hipStream_t st = m->ctx->stream;
   const int W = m->width, H = m->height;
-  DevBuf used;
+  DevBuf used, kept;
   TRY(used.alloc((size_t)m->cddt_nv + 1));
-  HIP_TRY(hipMemsetAsync(used.p, 0, (size_t)m->cddt_nv + 1, st));
-  const long long cells = (long long)W * H;
-  for (int a0 = 0; cells > 0 && a0 < m->cddt_nang; a0 += 65535) {  // grid rows: at most 65535 angles per launch
+  TRY(cddt_counts(m, &kept));
+  // widths are at most |W sin| + |H cos| rounded up
+  const int max_width = (int)ceil(sqrt((double)W * W + (double)H * H)) + 1;
+  for (int a0 = 0; a0 < m->cddt_nang; a0 += 65535) {  // grid rows: at most 65535 angles per launch
     const int na = std::min(65535, m->cddt_nang - a0);
-    hipLaunchKernelGGL(k_cddt_prune_mark, dim3(grid_for(cells, 256), (unsigned)na), dim3(256), 0, st,
-                       (const uint8_t*)m->d_occ, W, H, max_range, (const int*)m->cddt_width, (const float*)m->cddt_trans,
+    hipLaunchKernelGGL(k_cddt_prune_mark, dim3((unsigned)grid_for(max_width, 4), (unsigned)na), dim3(256), 0, st,
+                       (const uint8_t*)m->d_occ, W, H, (const int*)m->cddt_width, (const float*)m->cddt_trans,
                        (const float*)m->cddt_cos, (const float*)m->cddt_sin, (const long long*)m->cddt_bin_off,
-                       (const long long*)m->cddt_start, (const float*)m->cddt_vals, used.as<uint8_t>(), a0);
+                       (const long long*)m->cddt_start, (const float*)m->cddt_vals, used.as<uint8_t>(),
+                       kept.as<long long>(), a0);
     HIP_TRY(hipGetLastError());
   }
-  return cddt_compact(m, 1, used.as<uint8_t>());
+  return cddt_compact(m, 1, used.as<uint8_t>(), kept);
 }
 
 template <int METHOD>
@@ -477,7 +664,7 @@ int rl_map_build_cddt(rl_map* m, int theta_disc) {
   return RL_OK;
 }
 
-int rl_map_prune_cddt(rl_map* m, float max_range) {
+int rl_map_prune_cddt(rl_map* m, float /*max_range*/) {
   CHECK_ARG(m, "map is NULL");
   rl_ctx* c = m->ctx;
   std::lock_guard<std::mutex> lk(c->mu);
@@ -485,7 +672,7 @@ int rl_map_prune_cddt(rl_map* m, float max_range) {
   if (!m->cddt_vals) return fail(RL_ERR_STATE, "no CDDT tables (call rl_map_build_cddt first)");
   HIP_TRY(hipStreamSynchronize(c->stream));
   m->gen.fetch_add(1);
-  return cddt_prune_locked(m, max_range);
+  return cddt_prune_locked(m);
 }
 
 int rl_map_get_cddt(rl_map* m, int* theta_disc, long long* nbins, long long* nvals, int* widths, float* trans,

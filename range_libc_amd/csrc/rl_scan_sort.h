@@ -10,8 +10,8 @@
 //
 // Sort: floats are sorted by their order-preserving unsigned keys (sign bit
 // set: all bits inverted; clear: sign bit set), the order of a radix sort of
-// float bit patterns (-0 before +0).  Segments of up to 256 keys are sorted by
-// one wave each in LDS, up to 2048 by a 256-thread workgroup, up to 16384 by a
+// float bit patterns (-0 before +0).  Segments of up to 512 keys are sorted by
+// one wave each in registers, up to 2048 by a 256-thread workgroup in LDS, up to 16384 by a
 // 1024-thread workgroup (64 KiB of LDS), all with bitonic networks over the
 // segment padded to a power of two with the largest key; longer segments
 // (maps far above 4096 cells a side) are sorted in global memory, one
@@ -131,21 +131,9 @@ __device__ __forceinline__ float sort_key_value(unsigned k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-struct WaveSync {
-  __device__ void operator()() const {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-};
-struct BlockSync {
-  __device__ void operator()() const { __syncthreads(); }
-};
-
-// Ascending bitonic sort of s[0..P), P a power of two >= 2, by threads
-// tid = 0..nt-1; sync() orders consecutive stages.
-template <class Sync>
-__device__ __forceinline__ void bitonic_lds(unsigned* s, int P, int tid, int nt, Sync sync) {
+// Ascending bitonic sort of s[0..P) in LDS, P a power of two >= 2, by the
+// workgroup's threads tid = 0..nt-1.
+__device__ __forceinline__ void bitonic_lds(unsigned* s, int P, int tid, int nt) {
   for (int k = 2; k <= P; k <<= 1)
     for (int j = k >> 1; j > 0; j >>= 1) {
       for (int i = tid; i < (P >> 1); i += nt) {
@@ -156,7 +144,7 @@ __device__ __forceinline__ void bitonic_lds(unsigned* s, int P, int tid, int nt,
           s[b] = x;
         }
       }
-      sync();
+      __syncthreads();
     }
 }
 
@@ -166,30 +154,76 @@ __device__ __forceinline__ int pow2_at_least(long long n) {
   return p;
 }
 
-#define RL_SORT_WAVE_MAX 256
+#define RL_SORT_WAVE_MAX 512
 #define RL_SORT_MID_MAX 2048
 #define RL_SORT_BIG_MAX 16384
 
+// Ascending bitonic sort of 64 E keys by one wave, key e of lane l being element
+// l E + e: stages between elements of one lane are min / max of its registers,
+// stages between lanes one exchange per register.
+template <int E>
+__device__ __forceinline__ void bitonic_regs(unsigned (&r)[E], int lane) {
+#pragma unroll
+  for (int k = 2; k <= 64 * E; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      if (j >= E) {
+        // elements l E + e and (l ^ d) E + e; ascending where bit k of the element
+        // is clear (k > j >= E: a bit of the lane, or none when k is all of them)
+        const int d = j / E;
+        const bool keep_min = ((lane & d) == 0) == ((lane & (k / E)) == 0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const unsigned o = (unsigned)__shfl_xor((int)r[e], d);
+          r[e] = keep_min ? min(r[e], o) : max(r[e], o);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          if (e & j) continue;
+          const bool up = k < E ? (e & k) == 0 : (lane & (k / E)) == 0;
+          const unsigned lo = min(r[e], r[e | j]), hi = max(r[e], r[e | j]);
+          r[e] = up ? lo : hi;
+          r[e | j] = up ? hi : lo;
+        }
+      }
+    }
+  }
+}
+
+template <int E>
+__device__ __forceinline__ void sort_wave(const float* __restrict__ in, float* __restrict__ out, int n, int lane) {
+  unsigned r[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {  // (any order will do: the loads take consecutive elements)
+    const int i = e * 64 + lane;
+    r[e] = i < n ? sort_key(in[i]) : 0xffffffffu;
+  }
+  bitonic_regs<E>(r, lane);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (lane * E + e < n) out[lane * E + e] = sort_key_value(r[e]);
+}
+
 // Segments of at most RL_SORT_WAVE_MAX keys, one wave each (4 per workgroup);
-// longer segments are left to the other kernels.
+// longer segments are left to the other kernels.  32.9 M keys in 140,000
+// segments of up to 512: 204 us (a wave sorting at most 256 in LDS, workgroups
+// the others: 120 + 490 us).
 __global__ void __launch_bounds__(256) k_seg_sort_wave(const float* __restrict__ in, float* __restrict__ out,
                                                        const long long* __restrict__ start, long long nseg) {
-  __shared__ unsigned sh[4][RL_SORT_WAVE_MAX];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const long long seg = (long long)blockIdx.x * 4 + w;
-  if (seg >= nseg) return;  // no workgroup barrier below: a finished wave may leave
+  if (seg >= nseg) return;
   const long long b = start[seg], n = start[seg + 1] - b;
   if (n > RL_SORT_WAVE_MAX || n <= 0) return;
-  if (n == 1) {
-    if (lane == 0) out[b] = in[b];
-    return;
-  }
-  const int P = pow2_at_least(n);
-  unsigned* s = sh[w];
-  for (int i = lane; i < P; i += 64) s[i] = (i < n) ? sort_key(in[b + i]) : 0xffffffffu;
-  WaveSync()();
-  bitonic_lds(s, P, lane, 64, WaveSync());
-  for (int i = lane; i < n; i += 64) out[b + i] = sort_key_value(s[i]);
+  if (n <= 64)
+    sort_wave<1>(in + b, out + b, (int)n, lane);
+  else if (n <= 128)
+    sort_wave<2>(in + b, out + b, (int)n, lane);
+  else if (n <= 256)
+    sort_wave<4>(in + b, out + b, (int)n, lane);
+  else
+    sort_wave<8>(in + b, out + b, (int)n, lane);
 }
 
 // One workgroup of NT threads per listed segment (at most MAXN keys).
@@ -203,7 +237,7 @@ __global__ void __launch_bounds__(NT) k_seg_sort_block(const float* __restrict__
   const int P = pow2_at_least(n);
   for (int i = threadIdx.x; i < P; i += NT) s[i] = (i < n) ? sort_key(in[b + i]) : 0xffffffffu;
   __syncthreads();
-  bitonic_lds(s, P, threadIdx.x, NT, BlockSync());
+  bitonic_lds(s, P, threadIdx.x, NT);
   for (int i = threadIdx.x; i < n; i += NT) out[b + i] = sort_key_value(s[i]);
 }
 

@@ -191,3 +191,42 @@ def test_radial_optimized_golden_and_dev(ctx, golden, name):
     rm.calc_range_many_radial_optimized(rl.RL_METHOD_RM, R, ins[:50], out, 50, 60, -3 * math.pi / 4, 3 * math.pi / 4)
     assert_bits_equal(out, O.Oracle(img, R, "rm").calc_range_many_radial_optimized(ins[:50], 60, -3 * math.pi / 4,
                                                                                     3 * math.pi / 4), "rm pairs")
+
+
+def _cddt_map(name):
+    if name == "solid":  # blocks far thicker than a wall, and free cells inside one
+        img = np.ones((150, 101), np.uint8)
+        img[10:40, 5:90] = 0
+        img[90:92, 50:52] = 0
+        return img
+    if name == "open":  # a few lone cells, no walls: strips that leave the map free
+        img = np.zeros((97, 160), np.uint8)
+        img[3, 4] = img[50, 80] = img[51, 80] = img[96, 159] = 1
+        return img
+    if name == "free":
+        return np.zeros((40, 33), np.uint8)
+    if name == "full":
+        return np.ones((33, 40), np.uint8)
+    if name == "line":
+        return (np.arange(70)[None, :] % 9 == 0).astype(np.uint8)
+    if name == "noise":
+        return (np.random.default_rng(5).random((130, 77)) < 0.3).astype(np.uint8)
+    return W.corridor_map(300, seed=12)[:211, :300]
+
+
+@pytest.mark.parametrize("td", [1, 2, 7, 108, 361])
+@pytest.mark.parametrize("name", ["solid", "open", "free", "full", "line", "noise", "corridor"])
+def test_cddt_tables_equal_oracle(ctx, name, td):
+    """Whole tables, full and pruned, against the oracle: bins with one entry and
+    with many, strips without entries, intervals without and with free cells,
+    headings along the axes, at 45 degrees and in between."""
+    img = _cddt_map(name)
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    dm.build_cddt(td)
+    for prune in (False, True):
+        if prune:
+            dm.prune_cddt(50.0)
+        got, want = dm.cddt_tables(), O.Oracle(img, 50.0, "cddt", theta_disc=td, prune=prune).cddt_tables()
+        assert np.array_equal(got["widths"], want["widths"])
+        assert np.array_equal(got["start"], want["start"]), "pruned" if prune else "full"
+        assert_bits_equal(got["vals"], want["vals"], "pruned" if prune else "full")
