@@ -36,6 +36,49 @@ __global__ void k_cddt_consts(TrigDev trig, int td, int W, int H, float m2pi_div
   trans[a] = (float)(t > 0.0 ? t : 0.0);  // std::max(0.0, t)
 }
 
+// Bin offsets of the angles (one workgroup of 1024): exclusive sums of the
+// widths, and the build's sizes into pinned memory.
+struct CddtSizes {
+  long long nb, nba;  // bins of all angles, of the first nang
+  unsigned ne;        // edge cells
+  int max_width;
+};
+__global__ __launch_bounds__(1024) void k_cddt_offsets(const int* __restrict__ width, int td, int nang,
+                                                       const unsigned* __restrict__ n_edges, long long* __restrict__ off,
+                                                       CddtSizes* __restrict__ out) {
+  __shared__ long long sum[1024];
+  __shared__ int top[1024];
+  const int t = threadIdx.x, per = (td + 1023) / 1024;
+  const int a0 = min(td, t * per), a1 = min(td, a0 + per);
+  long long s = 0;
+  int mw = 0;
+  for (int a = a0; a < a1; ++a) s += width[a], mw = max(mw, width[a]);
+  sum[t] = s;
+  top[t] = mw;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {  // inclusive sums and maxima
+    const long long o = t >= d ? sum[t - d] : 0;
+    const int q = t >= d ? top[t - d] : 0;
+    __syncthreads();
+    sum[t] += o;
+    top[t] = max(top[t], q);
+    __syncthreads();
+  }
+  long long run = sum[t] - s;
+  for (int a = a0; a < a1; ++a) {
+    off[a] = run;
+    if (a == nang) out->nba = run;
+    run += width[a];
+  }
+  if (t == 1023) {
+    off[td] = sum[t];
+    out->nb = sum[t];
+    out->ne = *n_edges;
+    out->max_width = top[t];
+    if (nang == td) out->nba = sum[t];
+  }
+}
+
 // 2. Edge cells as (x << 16) | y (sides are below 65536), in any order.  A
 // workgroup gathers the edge cells of 4096 in LDS and takes their place in the
 // list with one atomic: with one per wave, 65,536 atomics on one address took
@@ -378,15 +421,21 @@ __global__ __launch_bounds__(256) void k_radial(MapDev m, TrigDev trig, float ma
 
 namespace {
 
+// A build's scratch from the context's pool, given back when the build's scope
+// ends (after waiting for what it launched).
 struct DevBuf {
+  rl_ctx* c;
   void* p = nullptr;
+  explicit DevBuf(rl_ctx* ctx) : c(ctx) {}
+  DevBuf(const DevBuf&) = delete;
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (!p) return;
+    (void)hipStreamSynchronize(c->stream);
+    c->pool.release(p, true);
   }
   int alloc(size_t bytes) {
-    if (hipMalloc(&p, bytes ? bytes : 16) != hipSuccess) {
+    if (c->pool.alloc(&p, bytes) != hipSuccess) {
       (void)hipGetLastError();
-      p = nullptr;
       return fail(RL_ERR_NOMEM, "CDDT: device allocation of %zu bytes failed", bytes);
     }
     return RL_OK;
@@ -401,8 +450,7 @@ struct DevBuf {
 
 void cddt_free(rl_map* m) {
   void* ps[] = {m->cddt_width, m->cddt_trans, m->cddt_cos, m->cddt_sin, m->cddt_bin_off, m->cddt_start, m->cddt_vals};
-  for (void* p : ps)
-    if (p) (void)hipFree(p);
+  for (void* p : ps) m->ctx->pool.release(p, false);
   m->cddt_width = nullptr;
   m->cddt_trans = m->cddt_cos = m->cddt_sin = m->cddt_vals = nullptr;
   m->cddt_bin_off = m->cddt_start = nullptr;
@@ -410,30 +458,47 @@ void cddt_free(rl_map* m) {
   m->cddt_nb = m->cddt_nv = 0;
 }
 
-// Exclusive scan of counts[0..n) into out[0..n] (out[n] = total), on the stream.
-int scan_counts(hipStream_t st, const unsigned long long* counts, long long* out, long long n) {
-  // the scan writes n + 1 values: counts is read with a trailing zero
-  return exclusive_sum_u64(st, counts, (unsigned long long*)out, n + 1);
+// Table buffer from the pool.
+template <class T>
+int cddt_table(rl_map* m, T** p, size_t count) {
+  if (m->ctx->pool.alloc(p, count * sizeof(T)) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(RL_ERR_NOMEM, "CDDT: device allocation of %zu bytes failed", count * sizeof(T));
+  }
+  return RL_OK;
+}
+
+// A 64-bit value of the device, after the stream's work so far (through the
+// context's pinned block: its mutex is held).
+int cddt_read(rl_map* m, const long long* d, long long* out) {
+  long long* h;
+  TRY(m->ctx->pinned((void**)&h));
+  HIP_TRY(hipMemcpyAsync(h, d, sizeof(long long), hipMemcpyDeviceToHost, m->ctx->stream));
+  HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+  *out = *h;
+  return RL_OK;
 }
 
 // Keeps the entries selected by `mode` (see k_cddt_compact): new start and
 // values.  kept: the bins' numbers of entries to keep (nb + 1, the last 0).
 int cddt_compact(rl_map* m, int mode, const uint8_t* used, const DevBuf& kept) {
-  hipStream_t st = m->ctx->stream;
+  rl_ctx* c = m->ctx;
+  hipStream_t st = c->stream;
   const long long nb = m->cddt_nb;
-  DevBuf nstart, nvals;
+  DevBuf tiles(c), nstart(c), nvals(c);  // (the new tables leave through .p)
   TRY(nstart.alloc((size_t)(nb + 1) * sizeof(long long)));
-  TRY(scan_counts(st, kept.as<unsigned long long>(), nstart.as<long long>(), nb));
+  // the scan writes n + 1 values: its input has a trailing zero
+  TRY(exclusive_sum_u64(st, kept.as<unsigned long long>(), nstart.as<unsigned long long>(), nb + 1, &tiles));
   long long total = 0;
-  HIP_TRY(hipMemcpy(&total, nstart.as<long long>() + nb, sizeof(long long), hipMemcpyDeviceToHost));
+  TRY(cddt_read(m, nstart.as<long long>() + nb, &total));
   TRY(nvals.alloc((size_t)total * sizeof(float)));
   hipLaunchKernelGGL(k_cddt_compact<true>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
                      (const long long*)m->cddt_start, (const float*)m->cddt_vals, used, mode, (const long long*)nstart.p,
                      (long long*)nullptr, nvals.as<float>());
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
-  (void)hipFree(m->cddt_start);
-  (void)hipFree(m->cddt_vals);
+  c->pool.release(m->cddt_start, false);
+  c->pool.release(m->cddt_vals, false);
   m->cddt_start = nstart.as<long long>();
   m->cddt_vals = nvals.as<float>();
   nstart.p = nvals.p = nullptr;
@@ -461,45 +526,42 @@ int cddt_build_locked(rl_map* m, int td) {
   m->cddt_nang = nang;
   m->cddt_td_div_2pi = (float)((double)td / 6.28318530718);          // RangeLib.h:976
   const float m2pi_div_td = (float)(6.28318530718 / (double)(float)td);  // :977
-  HIP_TRY(hipMalloc(&m->cddt_width, td * sizeof(int)));
-  HIP_TRY(hipMalloc(&m->cddt_trans, td * sizeof(float)));
-  HIP_TRY(hipMalloc(&m->cddt_cos, td * sizeof(float)));
-  HIP_TRY(hipMalloc(&m->cddt_sin, td * sizeof(float)));
-  HIP_TRY(hipMalloc(&m->cddt_bin_off, (td + 1) * sizeof(long long)));
+  TRY(cddt_table(m, &m->cddt_width, (size_t)td));
+  TRY(cddt_table(m, &m->cddt_trans, (size_t)td));
+  TRY(cddt_table(m, &m->cddt_cos, (size_t)td));
+  TRY(cddt_table(m, &m->cddt_sin, (size_t)td));
+  TRY(cddt_table(m, &m->cddt_bin_off, (size_t)td + 1));
   hipLaunchKernelGGL(k_cddt_consts, dim3(grid_for(td, 64)), dim3(64), 0, st, c->trig, td, W, H, m2pi_div_td,
                      m->cddt_width, m->cddt_trans, m->cddt_cos, m->cddt_sin);
   HIP_TRY(hipGetLastError());
-  std::vector<int> widths(td);
-  HIP_TRY(hipMemcpyAsync(widths.data(), m->cddt_width, td * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  std::vector<long long> off(td + 1, 0);
-  for (int a = 0; a < td; ++a) off[a + 1] = off[a] + widths[a];
-  const long long nb = off[td];
-  m->cddt_nb = nb;
-  HIP_TRY(hipMemcpy(m->cddt_bin_off, off.data(), (td + 1) * sizeof(long long), hipMemcpyHostToDevice));
   // edge cells
   const long long N = (long long)W * H;
-  DevBuf edges, n_edges;
+  DevBuf edges(c), n_edges(c);
   TRY(edges.alloc((size_t)N * sizeof(unsigned)));
   TRY(n_edges.alloc(sizeof(unsigned)));
   HIP_TRY(hipMemsetAsync(n_edges.p, 0, sizeof(unsigned), st));
   hipLaunchKernelGGL(k_cddt_edges, dim3(grid_for(N, 256 * RL_CDDT_EDGE_ITEMS)), dim3(256), 0, st,
                      (const uint8_t*)m->d_occ, W, H, edges.as<unsigned>(), n_edges.as<unsigned>());
   HIP_TRY(hipGetLastError());
-  unsigned ne = 0;
-  HIP_TRY(hipMemcpyAsync(&ne, n_edges.p, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+  CddtSizes* sz;
+  TRY(c->pinned((void**)&sz));
+  hipLaunchKernelGGL(k_cddt_offsets, dim3(1), dim3(1024), 0, st, (const int*)m->cddt_width, td, nang,
+                     (const unsigned*)n_edges.p, m->cddt_bin_off, sz);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
+  const long long nb = sz->nb, nba = sz->nba;
+  const unsigned ne = sz->ne;
+  const int max_width = sz->max_width;
+  m->cddt_nb = nb;
   // count, scan, fill.  In LDS where an angle's bins fit; about 1024 workgroups,
   // each of at least 2048 edge cells and at most 32 chunks of an angle
-  DevBuf counter, chunks;
+  DevBuf counter(c), chunks(c), tiles(c), raw(c), kept(c), lists(c);
   TRY(cddt_counts(m, &counter));
-  const int max_width = *std::max_element(widths.begin(), widths.end());
   const bool in_lds = max_width <= RL_CDDT_LDS_BINS;
   const int G = std::max(1, std::min(std::min(32, 1024 / nang + 1), (int)(ne / 2048u)));
   const unsigned hist_grid = 8u * (unsigned)((nang + 7) / 8) * (unsigned)G;
   const unsigned hist_lds = (unsigned)max_width * sizeof(unsigned);
   if (ne && in_lds) {
-    const long long nba = off[nang];  // the bins of the angles that hold entries
     TRY(chunks.alloc((size_t)G * (size_t)nb * sizeof(unsigned)));
     hipLaunchKernelGGL(k_cddt_hist<false>, dim3(hist_grid), dim3(256), hist_lds, st, (const unsigned*)edges.p, (int)ne,
                        nang, G, (const int*)m->cddt_width, (const float*)m->cddt_trans, (const float*)m->cddt_cos,
@@ -517,12 +579,11 @@ int cddt_build_locked(rl_map* m, int td) {
                        (const long long*)m->cddt_bin_off, counter.as<unsigned long long>(), (float*)nullptr);
     HIP_TRY(hipGetLastError());
   }
-  HIP_TRY(hipMalloc(&m->cddt_start, (size_t)(nb + 1) * sizeof(long long)));
-  TRY(scan_counts(st, counter.as<unsigned long long>(), m->cddt_start, nb));
+  TRY(cddt_table(m, &m->cddt_start, (size_t)nb + 1));
+  TRY(exclusive_sum_u64(st, counter.as<unsigned long long>(), (unsigned long long*)m->cddt_start, nb + 1, &tiles));
   long long total = 0;
-  HIP_TRY(hipMemcpy(&total, m->cddt_start + nb, sizeof(long long), hipMemcpyDeviceToHost));
+  TRY(cddt_read(m, m->cddt_start + nb, &total));
   if (total > 0x7fffffffLL) return fail(RL_ERR_ARG, "CDDT: %lld table entries exceed 2^31", total);
-  DevBuf raw;
   TRY(raw.alloc((size_t)total * sizeof(float)));
   if (ne && in_lds) {
     hipLaunchKernelGGL(k_cddt_hist<true>, dim3(hist_grid), dim3(256), hist_lds, st, (const unsigned*)edges.p, (int)ne,
@@ -531,7 +592,7 @@ int cddt_build_locked(rl_map* m, int td) {
                        chunks.as<unsigned>(), nb, raw.as<float>());
     HIP_TRY(hipGetLastError());
   } else if (ne) {
-    HIP_TRY(hipMemcpy(counter.p, m->cddt_start, (size_t)(nb + 1) * sizeof(long long), hipMemcpyDeviceToDevice));
+    HIP_TRY(hipMemcpyAsync(counter.p, m->cddt_start, (size_t)(nb + 1) * sizeof(long long), hipMemcpyDeviceToDevice, st));
     for (int a0 = 0; a0 < nang; a0 += 65535) {
       hipLaunchKernelGGL(k_cddt_scatter<true>, dim3(grid_for(ne, 256), (unsigned)std::min(65535, nang - a0)), dim3(256),
                          0, st, (const unsigned*)edges.p, (int)ne, a0, (const int*)m->cddt_width,
@@ -541,11 +602,10 @@ int cddt_build_locked(rl_map* m, int td) {
     }
   }
   // sort each bin
-  HIP_TRY(hipMalloc(&m->cddt_vals, (size_t)(total ? total : 1) * sizeof(float)));
-  if (total > 0) TRY(segmented_sort_f32(st, raw.as<float>(), m->cddt_vals, m->cddt_start, nb));
+  TRY(cddt_table(m, &m->cddt_vals, (size_t)total));
+  if (total > 0) TRY(segmented_sort_f32(st, raw.as<float>(), m->cddt_vals, m->cddt_start, nb, &lists));
   m->cddt_nv = total;
   // drop duplicates
-  DevBuf kept;
   TRY(cddt_counts(m, &kept));
   hipLaunchKernelGGL(k_cddt_compact<false>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
                      (const long long*)m->cddt_start, (const float*)m->cddt_vals, (const uint8_t*)nullptr, 0,
@@ -558,7 +618,7 @@ int cddt_build_locked(rl_map* m, int td) {
 int cddt_prune_locked(rl_map* m) {
   hipStream_t st = m->ctx->stream;
   const int W = m->width, H = m->height;
-  DevBuf used, kept;
+  DevBuf used(m->ctx), kept(m->ctx);
   TRY(used.alloc((size_t)m->cddt_nv + 1));
   TRY(cddt_counts(m, &kept));
   // widths are at most |W sin| + |H cos| rounded up
@@ -700,14 +760,20 @@ int rl_debug_exclusive_sum_dev(rl_ctx* c, const unsigned long long* in, unsigned
   CHECK_ARG(c && (n <= 0 || (in && out)), "bad argument");
   std::lock_guard<std::mutex> lk(c->mu);
   TRY(use_device(c));
-  return exclusive_sum_u64(c->stream, in, out, n);
+  DevBuf tiles(c);
+  TRY(exclusive_sum_u64(c->stream, in, out, n, &tiles));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return RL_OK;
 }
 
 int rl_debug_segmented_sort_dev(rl_ctx* c, const float* in, float* out, const long long* start, long long nseg) {
   CHECK_ARG(c && (nseg <= 0 || (in && out && start)), "bad argument");
   std::lock_guard<std::mutex> lk(c->mu);
   TRY(use_device(c));
-  return segmented_sort_f32(c->stream, in, out, start, nseg);
+  DevBuf lists(c);
+  TRY(segmented_sort_f32(c->stream, in, out, start, nseg, &lists));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return RL_OK;
 }
 
 }  // extern "C"

@@ -26,6 +26,7 @@
 #include <atomic>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/rangelib_hip.h"
@@ -180,14 +181,14 @@ __global__ __launch_bounds__(64) void k_edt_envelope(const float* __restrict__ f
 //
 // The search from x stops at the first distance d with d^2 >= best: every
 // candidate beyond it is at least d^2.  Rows whose inputs break the condition
-// are marked in slow[y] (every row's mark is written) and left to
-// k_edt_envelope.  LDS holds the rows x-major, s[x * EDT_RB + r], the order
+// are marked in slow[y] (every row's mark is written) and in *any_slow, and
+// left to k_edt_envelope.  LDS holds the rows x-major, s[x * EDT_RB + r], the order
 // they sit in global memory, so loads, searches and stores are unit-stride
 // across the lanes.
 constexpr int EDT_RB = 4;
 __global__ __launch_bounds__(256) void k_edt_rows(const float* __restrict__ g,
                                                   float* __restrict__ D, int W, int H,
-                                                  int* __restrict__ slow, int do_sqrt) {
+                                                  int* __restrict__ slow, int* __restrict__ any_slow, int do_sqrt) {
   extern __shared__ float s_g[];
   __shared__ int s_bad[EDT_RB], s_fin[EDT_RB];
   const int y0 = blockIdx.x * EDT_RB;
@@ -215,7 +216,10 @@ __global__ __launch_bounds__(256) void k_edt_rows(const float* __restrict__ g,
     s_g[c] = v;
   }
   __syncthreads();
-  if (t < EDT_RB && y0 + t < H) slow[y0 + t] = s_bad[t];
+  if (t < EDT_RB && y0 + t < H) {
+    slow[y0 + t] = s_bad[t];
+    if (s_bad[t]) *any_slow = 1;
+  }
   for (int c = t; c < n; c += 256) {
     const int r = c % EDT_RB, x = c / EDT_RB, y = y0 + r;
     if (y >= H || s_bad[r]) continue;
@@ -1050,7 +1054,90 @@ int segment_size(int m) {
 
 #define RL_PINNED_BYTES (512u << 10)  // host-pointer calls whose parts fit run zero-copy (rl_ctx::pinned)
 
+// Device blocks of maps, tables and their builds, kept for the next one when they
+// are let go: hipFree of a block above 16 MB takes 0.22 ms and up (0.9 ms seen
+// for the next hipMalloc after it), and replacing a 2048^2 map spent 0.6 of its
+// 1.04 ms there.  Blocks below RL_POOL_MIN go to the allocator directly (under a
+// microsecond).  At most RL_POOL_BYTES are kept idle, and given back with the
+// context.  A block that other streams may still be reading (a map's buffers:
+// their addresses are handed out) is reused only after the device was waited
+// for, as hipFree would have.
+#define RL_POOL_MIN (1u << 20)
+#define RL_POOL_BYTES (512u << 20)  // the buffers of a CDDT build of a 2048^2 map are 0.4 GB
+struct DevPool {
+  struct Block {
+    void* p;
+    size_t cap;
+    bool idle;  // no work uses it any more
+  };
+  std::mutex mu;
+  std::vector<Block> kept;
+  std::unordered_map<void*, size_t> live;  // capacities of the blocks handed out
+  size_t held = 0;
+
+  template <class T>
+  hipError_t alloc(T** out, size_t bytes) {
+    *out = nullptr;
+    if (bytes < RL_POOL_MIN) return hipMalloc((void**)out, bytes ? bytes : 16);
+    const size_t cap = (bytes + (2u << 20) - 1) & ~(size_t)((2u << 20) - 1);
+    std::lock_guard<std::mutex> lk(mu);
+    size_t best = kept.size();
+    for (size_t i = 0; i < kept.size(); ++i)
+      if (kept[i].cap >= cap && kept[i].cap <= cap + cap / 4 && (best == kept.size() || kept[i].cap < kept[best].cap))
+        best = i;
+    if (best < kept.size() && !kept[best].idle) {
+      if (hipDeviceSynchronize() == hipSuccess)
+        for (Block& b : kept) b.idle = true;
+      else
+        best = kept.size(), (void)hipGetLastError();
+    }
+    if (best < kept.size()) {
+      const Block b = kept[best];
+      kept.erase(kept.begin() + (long)best);
+      held -= b.cap;
+      live[b.p] = b.cap;
+      *out = (T*)b.p;
+      return hipSuccess;
+    }
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, cap);
+    if (e != hipSuccess && !kept.empty()) {  // out of memory with blocks kept: give them back first
+      (void)hipGetLastError();
+      drop();
+      e = hipMalloc(&p, cap);
+    }
+    if (e != hipSuccess) return e;
+    live[p] = cap;
+    *out = (T*)p;
+    return hipSuccess;
+  }
+
+  // idle: the caller has waited for all work that uses the block
+  void release(void* p, bool idle) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu);
+    const auto it = live.find(p);
+    if (it != live.end()) {
+      const size_t cap = it->second;
+      live.erase(it);
+      if (held + cap <= RL_POOL_BYTES) {
+        kept.push_back(Block{p, cap, idle});
+        held += cap;
+        return;
+      }
+    }
+    (void)hipFree(p);
+  }
+
+  void drop() {  // mu held, or the last user
+    for (const Block& b : kept) (void)hipFree(b.p);
+    kept.clear();
+    held = 0;
+  }
+};
+
 struct rl_ctx {
+  DevPool pool;
   int device = 0;
   hipStream_t own_stream = nullptr;
   hipStream_t stream = nullptr;
@@ -1333,15 +1420,13 @@ int build_compact(rl_map* m, unsigned flags) {
   m->nby = (H + 7) / 8;
   const size_t nbytes = (size_t)((W + 7) / 8) * (size_t)m->nby * 64;
   if (nbytes > 0xFFFFFFFFull) return RL_OK;  // 32-bit offsets only: such maps march the fp32 map
-  if (hipMalloc(&m->d_idx8, nbytes) != hipSuccess) {
+  if (!m->d_idx8 && c->pool.alloc(&m->d_idx8, nbytes) != hipSuccess) {
     (void)hipGetLastError();
-    m->d_idx8 = nullptr;
     return fail(RL_ERR_NOMEM, "device allocation of the %zu-byte compact map failed", nbytes);
   }
   hipLaunchKernelGGL(k_build_idx8, dim3(grid_for((long long)nbytes, 256)), dim3(256), 0, c->stream,
                      (const float*)m->d_edt, (const float*)c->d_lut, m->d_idx8, W, H, m->nby, nbytes);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(RL_ERR_HIP, "compact map build: %s", hipGetErrorString(e));
   return RL_OK;
 }
@@ -1354,9 +1439,8 @@ int build_bits(rl_map* m) {
   const int ntx = (m->width + 7) / 8, nty = (m->height + 7) / 8;
   const size_t nbytes = (size_t)ntx * nty * 16;
   if (nbytes + 16 > 0xFFFFFFFFull) return RL_OK;
-  if (hipMalloc(&m->d_bits, nbytes + 16) != hipSuccess) {
+  if (c->pool.alloc(&m->d_bits, nbytes + 16) != hipSuccess) {
     (void)hipGetLastError();
-    m->d_bits = nullptr;
     return fail(RL_ERR_NOMEM, "device allocation of the %zu-byte occupancy bitmap failed", nbytes + 16);
   }
   m->bits_bytes = (unsigned)nbytes;
@@ -1366,35 +1450,54 @@ int build_bits(rl_map* m) {
                        (const uint8_t*)m->d_occ, (unsigned long long*)m->d_bits, m->width, m->height, ntx, nty);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return fail(RL_ERR_HIP, "occupancy bitmap build: %s", hipGetErrorString(e));
   return RL_OK;
 }
 
+// Distance transform of m->d_occ into m->d_edt, with the compact map and the
+// occupancy bitmap, waited for.  The envelope's stacks (12 bytes a cell) are
+// allocated only when a row needs them.
 int build_edt(rl_map* m, unsigned flags) {
   rl_ctx* c = m->ctx;
   const int W = m->width, H = m->height;
   const size_t N = (size_t)W * H;
+  const bool cols = H <= 4096 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY);
+  // the row search needs EDT_RB rows of the map in LDS (plus its flags) within 64 KiB
+  const bool search = (size_t)EDT_RB * W * sizeof(float) + 64 <= 65536 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY);
   float* g = nullptr;
-  int* v = nullptr;
+  int *v = nullptr, *slow = nullptr;  // slow[y]: row y is left to the envelope
   double* z = nullptr;
+  int* any_slow;  // in pinned memory, written by the kernel where a row is
+  TRY(c->pinned((void**)&any_slow));
+  *any_slow = 0;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   int rc = RL_OK;
+  auto oom = [&] {
+    (void)hipGetLastError();
+    rc = fail(RL_ERR_NOMEM, "device allocation for the %dx%d distance transform failed", W, H);
+  };
+  auto stacks = [&] {
+    return c->pool.alloc(&v, N * sizeof(int)) == hipSuccess &&
+           c->pool.alloc(&z, (N + (size_t)W + (size_t)H) * sizeof(double)) == hipSuccess;
+  };
+  auto rows_envelope = [&](const int* only) {
+    hipLaunchKernelGGL(k_edt_envelope, dim3(grid_for(H, 64)), dim3(64), 0, c->stream, (const float*)g, m->d_edt, H, W,
+                       (long long)H, 1LL, v, z, 1, only);
+  };
   do {
-    if (hipMalloc(&g, N * sizeof(float)) != hipSuccess ||
-        hipMalloc(&v, (N + (size_t)H) * sizeof(int)) != hipSuccess ||
-        hipMalloc(&z, (N + (size_t)W + (size_t)H) * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      rc = fail(RL_ERR_NOMEM, "device allocation for the %dx%d distance transform failed", W, H);
+    if (c->pool.alloc(&g, N * sizeof(float)) != hipSuccess || hipMalloc(&slow, (size_t)H * sizeof(int)) != hipSuccess ||
+        (!(cols && search) && !stacks())) {
+      oom();
       break;
     }
-    if (hipEventRecord(e0, c->stream) != hipSuccess) {
-      rc = fail(RL_ERR_HIP, "hipEventRecord failed");
+    hipError_t e = hipEventRecord(e0, c->stream);
+    if (e != hipSuccess) {
+      rc = fail(RL_ERR_HIP, "distance transform: %s", hipGetErrorString(e));
       break;
     }
-    if (H <= 4096 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY)) {
+    if (cols) {
       hipLaunchKernelGGL(k_edt_cols, dim3(W), dim3(256), 0, c->stream, m->d_occ, g, H);
     } else {
       hipLaunchKernelGGL(k_edt_init, dim3(grid_for((long long)N, 256)), dim3(256), 0, c->stream,
@@ -1405,30 +1508,35 @@ int build_edt(rl_map* m, unsigned flags) {
     }
     // Pass 2: the bounded search where it is exact, the lower envelope on the
     // rows it marks (or on every row when the envelope is asked for).
-    const int* rows = nullptr;
-    // the row search needs EDT_RB rows of the map in LDS (plus its flags) within 64 KiB
-    if ((size_t)EDT_RB * W * sizeof(float) + 64 <= 65536 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY)) {
-      int* slow = v + N;
+    if (search)
       hipLaunchKernelGGL(k_edt_rows, dim3((H + EDT_RB - 1) / EDT_RB), dim3(256),
                          (size_t)EDT_RB * W * sizeof(float), c->stream, (const float*)g,
-                         m->d_edt, W, H, slow, 1);
-      rows = slow;
-    }
-    hipLaunchKernelGGL(k_edt_envelope, dim3(grid_for(H, 64)), dim3(64), 0, c->stream,
-                       (const float*)g, m->d_edt, H, W, (long long)H, 1LL, v, z, 1, rows);
-    hipError_t e = hipGetLastError();
+                         m->d_edt, W, H, slow, any_slow, 1);
+    else
+      rows_envelope(nullptr);
+    e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
+    if (e == hipSuccess && (rc = build_compact(m, flags)) == RL_OK) rc = build_bits(m);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
-      rc = fail(RL_ERR_HIP, "distance transform: %s", hipGetErrorString(e));
-      break;
+    if (e == hipSuccess && rc == RL_OK && *(volatile int*)any_slow) {
+      if (!v && !stacks()) {
+        oom();
+        break;
+      }
+      rows_envelope(slow);
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
+      if (e == hipSuccess) rc = build_compact(m, flags);
+      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     }
-    (void)hipEventElapsedTime(&m->edt_ms, e0, e1);
-    rc = build_compact(m, flags);
+    if (e != hipSuccess) rc = fail(RL_ERR_HIP, "distance transform: %s", hipGetErrorString(e));
+    if (rc == RL_OK) (void)hipEventElapsedTime(&m->edt_ms, e0, e1);
   } while (0);
-  if (g) (void)hipFree(g);
-  if (v) (void)hipFree(v);
-  if (z) (void)hipFree(z);
+  (void)hipStreamSynchronize(c->stream);
+  c->pool.release(g, true);
+  c->pool.release(v, true);
+  c->pool.release(z, true);
+  if (slow) (void)hipFree(slow);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return rc;
@@ -1599,6 +1707,7 @@ int rl_destroy(rl_ctx* c) {
   if (c->refs.fetch_sub(1) != 1) return RL_OK;  // maps or batches still hold it
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
+  c->pool.drop();
   for (int i = 0; i < 6; ++i)
     if (c->stage[i]) (void)hipFree(c->stage[i]);
   if (c->pin) (void)hipHostFree(c->pin);
@@ -1639,7 +1748,7 @@ int rl_map_create_ex(rl_ctx* c, const uint8_t* occ, int width, int height, unsig
   m->height = height;
   set_world(m, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f);  // RangeLibc.pyx:174-180
   const size_t N = (size_t)width * height;
-  if (hipMalloc(&m->d_occ, N) != hipSuccess || hipMalloc(&m->d_edt, N * sizeof(float)) != hipSuccess) {
+  if (c->pool.alloc(&m->d_occ, N) != hipSuccess || c->pool.alloc(&m->d_edt, N * sizeof(float)) != hipSuccess) {
     (void)hipGetLastError();
     rl_map_destroy(m);
     return fail(RL_ERR_NOMEM, "device allocation for a %dx%d map failed", width, height);
@@ -1648,8 +1757,7 @@ int rl_map_create_ex(rl_ctx* c, const uint8_t* occ, int width, int height, unsig
     rl_map_destroy(m);
     return fail(RL_ERR_HIP, "occupancy upload failed");
   }
-  int rc = build_edt(m, flags);
-  if (rc == RL_OK) rc = build_bits(m);
+  const int rc = build_edt(m, flags);
   if (rc != RL_OK) {
     std::string msg = g_err;
     rl_map_destroy(m);
@@ -1673,14 +1781,15 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
   if (!m->d_edt) return fail(RL_ERR_STATE, "map has no distance transform");
   const long long total = (long long)m->width * m->height * theta_disc;
   m->gen.fetch_add(1);
-  if (m->d_glt) {
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipFree(m->d_glt));
+  // a rebuilt table of the same size takes its predecessor's place, once nothing
+  // reads that any more
+  if (m->d_glt) HIP_TRY(hipDeviceSynchronize());
+  if (m->d_glt && (long long)m->width * m->height * m->glt_td != total) {
+    c->pool.release(m->d_glt, true);
     m->d_glt = nullptr;
   }
-  if (hipMalloc(&m->d_glt, (size_t)total * sizeof(uint16_t)) != hipSuccess) {
+  if (!m->d_glt && c->pool.alloc(&m->d_glt, (size_t)total * sizeof(uint16_t)) != hipSuccess) {
     (void)hipGetLastError();
-    m->d_glt = nullptr;
     return fail(RL_ERR_NOMEM, "device allocation of the %lld-entry GiantLUTCast table failed", total);
   }
   // RangeLib.h:1783-1786 (int / double, double / float, float / int, int / float)
@@ -1724,7 +1833,7 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (e != hipSuccess) {
-    (void)hipFree(m->d_glt);
+    c->pool.release(m->d_glt, false);
     m->d_glt = nullptr;
     return fail(RL_ERR_HIP, "GiantLUTCast build: %s", hipGetErrorString(e));
   }
@@ -1763,7 +1872,7 @@ int rl_map_create_from_edt(rl_ctx* c, const uint8_t* occ, const float* edt, int 
   m->height = height;
   set_world(m, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f);
   const size_t N = (size_t)width * height;
-  if (hipMalloc(&m->d_occ, N) != hipSuccess || hipMalloc(&m->d_edt, N * sizeof(float)) != hipSuccess) {
+  if (c->pool.alloc(&m->d_occ, N) != hipSuccess || c->pool.alloc(&m->d_edt, N * sizeof(float)) != hipSuccess) {
     (void)hipGetLastError();
     rl_map_destroy(m);
     return fail(RL_ERR_NOMEM, "device allocation for a %dx%d map failed", width, height);
@@ -1792,19 +1901,11 @@ int rl_map_destroy(rl_map* m) {
   rl_ctx* c = m->ctx;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  if (m->d_occ) (void)hipFree(m->d_occ);
-  if (m->d_edt) (void)hipFree(m->d_edt);
-  if (m->d_idx8) (void)hipFree(m->d_idx8);
-  if (m->d_bits) (void)hipFree(m->d_bits);
   if (m->d_sched) (void)hipFree(m->d_sched);
   if (m->d_table) (void)hipFree(m->d_table);
-  if (m->d_glt) (void)hipFree(m->d_glt);
-  {
-    void* ps[] = {m->cddt_width, m->cddt_trans, m->cddt_cos, m->cddt_sin, m->cddt_vals, m->cddt_bin_off,
-                  m->cddt_start};
-    for (void* p : ps)
-      if (p) (void)hipFree(p);
-  }
+  void* ps[] = {m->d_occ, m->d_edt, m->d_idx8, m->d_bits, m->d_glt, m->cddt_width, m->cddt_trans, m->cddt_cos,
+                m->cddt_sin, m->cddt_vals, m->cddt_bin_off, m->cddt_start};
+  for (void* p : ps) c->pool.release(p, false);
   delete m;
   return rl_destroy(c);  // drops the map's reference
 }

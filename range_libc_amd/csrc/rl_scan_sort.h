@@ -106,20 +106,20 @@ __global__ void __launch_bounds__(RL_SCAN_BLOCK) k_scan_out(const unsigned long 
   }
 }
 
-// out[i] = in[0] + ... + in[i - 1] for i < n, on the stream (returns after it ran).
-int exclusive_sum_u64(hipStream_t st, const unsigned long long* in, unsigned long long* out, long long n) {
+// out[i] = in[0] + ... + in[i - 1] for i < n, on the stream; `tiles` is scratch
+// for one call.
+int exclusive_sum_u64(hipStream_t st, const unsigned long long* in, unsigned long long* out, long long n,
+                      DevBuf* tiles) {
   if (n <= 0) return RL_OK;
   const long long nt = (n + RL_SCAN_TILE - 1) / RL_SCAN_TILE;
   if (nt > 0x7fffffffLL) return fail(RL_ERR_ARG, "scan: %lld items is too many", n);
-  DevBuf tiles;
-  TRY(tiles.alloc((size_t)nt * sizeof(unsigned long long)));
+  TRY(tiles->alloc((size_t)nt * sizeof(unsigned long long)));
   hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)nt), dim3(RL_SCAN_BLOCK), 0, st, in, n,
-                     tiles.as<unsigned long long>());
-  hipLaunchKernelGGL(k_scan_spine, dim3(1), dim3(RL_SCAN_BLOCK), 0, st, tiles.as<unsigned long long>(), nt);
+                     tiles->as<unsigned long long>());
+  hipLaunchKernelGGL(k_scan_spine, dim3(1), dim3(RL_SCAN_BLOCK), 0, st, tiles->as<unsigned long long>(), nt);
   hipLaunchKernelGGL(k_scan_out, dim3((unsigned)nt), dim3(RL_SCAN_BLOCK), 0, st, in, n,
-                     (const unsigned long long*)tiles.p, out);
+                     (const unsigned long long*)tiles->p, out);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
 }
 
@@ -226,19 +226,23 @@ __global__ void __launch_bounds__(256) k_seg_sort_wave(const float* __restrict__
     sort_wave<8>(in + b, out + b, (int)n, lane);
 }
 
-// One workgroup of NT threads per listed segment (at most MAXN keys).
+// Workgroups of NT threads over the listed segments (at most MAXN keys each).
 template <int NT, int MAXN>
 __global__ void __launch_bounds__(NT) k_seg_sort_block(const float* __restrict__ in, float* __restrict__ out,
                                                        const long long* __restrict__ start,
-                                                       const unsigned* __restrict__ list) {
+                                                       const unsigned* __restrict__ list,
+                                                       const unsigned* __restrict__ count) {
   __shared__ unsigned s[MAXN];
-  const long long seg = list[blockIdx.x];
-  const long long b = start[seg], n = start[seg + 1] - b;
-  const int P = pow2_at_least(n);
-  for (int i = threadIdx.x; i < P; i += NT) s[i] = (i < n) ? sort_key(in[b + i]) : 0xffffffffu;
-  __syncthreads();
-  bitonic_lds(s, P, threadIdx.x, NT);
-  for (int i = threadIdx.x; i < n; i += NT) out[b + i] = sort_key_value(s[i]);
+  for (unsigned l = blockIdx.x; l < *count; l += gridDim.x) {  // the same in every thread
+    const long long seg = list[l];
+    const long long b = start[seg], n = start[seg + 1] - b;
+    const int P = pow2_at_least(n);
+    for (int i = threadIdx.x; i < P; i += NT) s[i] = (i < n) ? sort_key(in[b + i]) : 0xffffffffu;
+    __syncthreads();
+    bitonic_lds(s, P, threadIdx.x, NT);
+    for (int i = threadIdx.x; i < n; i += NT) out[b + i] = sort_key_value(s[i]);
+    __syncthreads();  // stored before the next segment is loaded
+  }
 }
 
 // Lists the segments longer than RL_SORT_WAVE_MAX by size class: class 0
@@ -283,39 +287,40 @@ __global__ void k_sort_global_store(const unsigned* __restrict__ keys, float* __
 }
 
 // out[start[s] .. start[s + 1]) = in[start[s] .. start[s + 1]) sorted ascending,
-// for every segment s < nseg (start on the device, nseg + 1 entries, nseg < 2^32).
-int segmented_sort_f32(hipStream_t st, const float* in, float* out, const long long* start, long long nseg) {
+// for every segment s < nseg (start on the device, nseg + 1 entries, nseg < 2^32);
+// `lists` is scratch for one call.  Waits for the stream only to learn whether
+// a segment is left to the global-memory sort.
+int segmented_sort_f32(hipStream_t st, const float* in, float* out, const long long* start, long long nseg,
+                       DevBuf* lists) {
   if (nseg <= 0) return RL_OK;
   if (nseg >= 0xffffffffLL) return fail(RL_ERR_ARG, "sort: %lld segments is too many", nseg);
   hipLaunchKernelGGL(k_seg_sort_wave, dim3((unsigned)((nseg + 3) / 4)), dim3(256), 0, st, in, out, start, nseg);
-  DevBuf lists, counts;
-  TRY(lists.alloc((size_t)nseg * 3 * sizeof(unsigned)));
-  TRY(counts.alloc(4 * sizeof(unsigned)));
-  HIP_TRY(hipMemsetAsync(counts.p, 0, 4 * sizeof(unsigned), st));
-  hipLaunchKernelGGL(k_seg_classify, dim3((unsigned)((nseg + 255) / 256)), dim3(256), 0, st, start, nseg,
-                     lists.as<unsigned>(), counts.as<unsigned>());
+  TRY(lists->alloc((4 + (size_t)nseg * 3) * sizeof(unsigned)));
+  unsigned* counts = lists->as<unsigned>();  // 4, then the three lists
+  const unsigned* L = counts + 4;
+  HIP_TRY(hipMemsetAsync(counts, 0, 4 * sizeof(unsigned), st));
+  hipLaunchKernelGGL(k_seg_classify, dim3((unsigned)((nseg + 255) / 256)), dim3(256), 0, st, start, nseg, counts + 4,
+                     counts);
+  hipLaunchKernelGGL((k_seg_sort_block<256, RL_SORT_MID_MAX>), dim3((unsigned)std::min<long long>(nseg, 1024)), dim3(256),
+                     0, st, in, out, start, L, (const unsigned*)counts);
+  hipLaunchKernelGGL((k_seg_sort_block<1024, RL_SORT_BIG_MAX>), dim3((unsigned)std::min<long long>(nseg, 512)), dim3(1024),
+                     0, st, in, out, start, L + nseg, (const unsigned*)counts + 1);
   HIP_TRY(hipGetLastError());
-  unsigned cnt[4] = {0, 0, 0, 0};
-  HIP_TRY(hipMemcpyAsync(cnt, counts.p, sizeof(cnt), hipMemcpyDeviceToHost, st));
+  unsigned* cnt;
+  TRY(lists->c->pinned((void**)&cnt));
+  HIP_TRY(hipMemcpyAsync(cnt, counts, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  const unsigned* L = lists.as<unsigned>();
-  if (cnt[0])
-    hipLaunchKernelGGL((k_seg_sort_block<256, RL_SORT_MID_MAX>), dim3(cnt[0]), dim3(256), 0, st, in, out, start, L);
-  if (cnt[1])
-    hipLaunchKernelGGL((k_seg_sort_block<1024, RL_SORT_BIG_MAX>), dim3(cnt[1]), dim3(1024), 0, st, in, out, start,
-                       L + nseg);
-  HIP_TRY(hipGetLastError());
   if (cnt[2]) {
     std::vector<unsigned> big(cnt[2]);
     std::vector<long long> se(2);
-    HIP_TRY(hipMemcpyAsync(big.data(), L + 2 * nseg, cnt[2] * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(big.data(), L + 2 * nseg, big.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     for (unsigned s : big) {
       HIP_TRY(hipMemcpy(se.data(), start + s, 2 * sizeof(long long), hipMemcpyDeviceToHost));
       const long long b = se[0], n = se[1] - se[0];
       long long P = 2;
       while (P < n) P <<= 1;
-      DevBuf keys;
+      DevBuf keys(lists->c);
       TRY(keys.alloc((size_t)P * sizeof(unsigned)));
       const unsigned gp = (unsigned)((P + 255) / 256), gh = (unsigned)((P / 2 + 255) / 256);
       hipLaunchKernelGGL(k_sort_global_load, dim3(gp), dim3(256), 0, st, in + b, keys.as<unsigned>(), n, P);
@@ -325,9 +330,7 @@ int segmented_sort_f32(hipStream_t st, const float* in, float* out, const long l
       hipLaunchKernelGGL(k_sort_global_store, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                          (const unsigned*)keys.p, out + b, n);
       HIP_TRY(hipGetLastError());
-      HIP_TRY(hipStreamSynchronize(st));
     }
   }
-  HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
 }

@@ -566,3 +566,34 @@ def test_dependent_load_probe(ctx):
         i = int(nxt[i])
     assert int(out[1].item()) == i
     assert int(out[0].item()) > 0 and tick_ns > 0
+
+
+def test_map_buffers_reused(ctx):
+    """Maps let go and made again take each other's device blocks, also while a
+    launch on another stream still reads the map that went: every range is that
+    of the map it was cast on."""
+    torch = _torch()
+    imgs = [W.rect_disk_map(1100, seed=s)[:1000] for s in (1, 2, 3)]
+    q = W.grid_poses(imgs[0], 200000, seed=4)
+    d = torch.from_numpy(q).cuda()
+    want = [O.Oracle(im, 300.0, "rm").calc_range_many(q[:3000]) for im in imgs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = []
+    try:
+        for k in range(6):
+            s = streams[k & 1]
+            s.wait_stream(torch.cuda.current_stream())
+            ctx.set_stream(s.cuda_stream)
+            dm = rl.DeviceMap(ctx, O.xmajor(imgs[k % 3]))
+            out = torch.zeros(q.shape[0], dtype=torch.float32, device="cuda")
+            torch.cuda.synchronize()
+            for _ in range(8):
+                dm.calc_range_many_dev(rl.RL_METHOD_RM, 300.0, d.data_ptr(), out.data_ptr(), q.shape[0])
+            ctx.set_stream(streams[1 - (k & 1)].cuda_stream)
+            dm.close()  # its casts are on the other stream
+            outs.append(out)
+    finally:
+        torch.cuda.synchronize()
+        ctx.set_stream(None)
+    for k, out in enumerate(outs):
+        assert_bits_equal(out.cpu().numpy()[:3000], want[k % 3], f"map {k}")
