@@ -2,7 +2,10 @@
 // include/rangelib_hip.h.
 //
 // Kernels
-//   k_edt_cols      distance-transform pass 1 (closed form along y, per column)
+//   k_edt_cols8     distance-transform pass 1 (bit scans along y) and the occupancy
+//   k_edt_rows8     bitmap; pass 2 (bounded search) and the compact map: maps of up
+//                   to 4096 x 3966 cells
+//   k_edt_cols      pass 1 (closed form along y, per column) for the other maps
 //   k_edt_init      f = 0 (occupied) / FLT_MAX (free) for the envelope pass
 //   k_edt_envelope  distance-transform lower envelope, one line per lane,
 //                   replicating vendor/distance_transform.h:1054-1096
@@ -241,6 +244,162 @@ __global__ __launch_bounds__(256) void k_edt_rows(const float* __restrict__ g,
       }
     }
     D[(size_t)x * H + y] = do_sqrt ? __builtin_sqrtf(best) : best;
+  }
+}
+
+// The two passes for maps of up to 4096 x RL_EDT_TILE_W cells (height x width),
+// with the compact map and the occupancy bitmap formed on the way: the map is
+// read once, and what goes between the passes is a 16-bit distance per cell.
+// 2048^2 corridor map: k_edt_cols, k_edt_rows, k_build_idx8 and k_build_bits took
+// 42 + 125 + 25 + 10 us, these 16 + 38.
+#define RL_EDT_NONE 32768u  // no obstacle in the column: its square, 2^30, is beyond every sum of squares here
+#define RL_EDT_TILE_W 3966  // 8 rows of 16-bit distances and their ends within 62 KB of LDS
+
+// Pass 1 for the 8 columns x = 8 blockIdx.x ..: each column's cells become bits
+// (a ballot per 64 cells), the nearest obstacle of a cell is found by bit scans
+// in its word and, through a mask of the non-empty words, in the next ones, and
+// the same bits are the bitmap's tiles (null: not wanted).
+__global__ __launch_bounds__(1024) void k_edt_cols8(const uint8_t* __restrict__ occ, uint16_t* __restrict__ g, int W,
+                                                    int H, unsigned long long* __restrict__ bits, int ntx, int nty) {
+  __shared__ unsigned long long word[8][64], any[8];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int x0 = blockIdx.x * 8, nw = (H + 63) >> 6;  // at most 64 words
+  const int nc = min(8, W - x0);
+  {  // two waves per column, 8 words in flight
+    const int u = wave & 7;
+    const uint8_t* col = occ + (size_t)(x0 + min(u, nc - 1)) * H;
+    for (int k0 = wave >> 3; k0 < nw; k0 += 16) {
+      uint8_t c[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) c[q] = col[min((k0 + 2 * q) * 64 + lane, H - 1)];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int k = k0 + 2 * q;
+        const unsigned long long m = __ballot(u < nc && k * 64 + lane < H && c[q] != 0);
+        if (lane == 0 && k < nw) word[u][k] = m;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave < 8) {
+    const unsigned long long m = __ballot(lane < nw && word[wave][lane < nw ? lane : 0] != 0ull);
+    if (lane == 0) any[wave] = m;
+  }
+  __syncthreads();
+  for (int u = 0; u < nc; ++u) {
+    const unsigned long long nz = any[u];
+    uint16_t* gc = g + (size_t)(x0 + u) * H;
+    for (int y = threadIdx.x; y < H; y += 1024) {
+      const int k = y >> 6, b = y & 63;
+      const unsigned long long w = word[u][k];
+      unsigned d = RL_EDT_NONE;
+      const unsigned long long lo = w << (63 - b), hi = w >> b;  // cells up to y, from y on
+      if (lo) {
+        d = (unsigned)__builtin_clzll(lo);
+      } else {
+        const unsigned long long q = nz & ((1ull << k) - 1ull);
+        if (q) {
+          const int j = 63 - __builtin_clzll(q);
+          d = (unsigned)(y - (j * 64 + 63 - __builtin_clzll(word[u][j])));
+        }
+      }
+      if (hi) {
+        d = min(d, (unsigned)__builtin_ctzll(hi));
+      } else {
+        const unsigned long long q = k < 63 ? nz >> (k + 1) : 0ull;
+        if (q) {
+          const int j = k + 1 + __builtin_ctzll(q);
+          d = min(d, (unsigned)(j * 64 + __builtin_ctzll(word[u][j]) - y));
+        }
+      }
+      gc[y] = (uint16_t)d;
+    }
+  }
+  if (!bits) return;
+  for (int ty = threadIdx.x; ty < nty; ty += 1024) {
+    const int k = ty >> 3, sh = (ty & 7) * 8;
+    unsigned long long t = 0;  // cell (8 tx + u, 8 ty + v): bit 8 u + v
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t |= ((word[u][k] >> sh) & 0xffull) << (8 * u);
+    bits[(size_t)blockIdx.x * nty + ty] = t;
+    // transposed: bit 8 v + u (blocks of 4, 2 and 1 swapped across the diagonal)
+    unsigned long long s = (t ^ (t >> 28)) & 0x00000000F0F0F0F0ull;
+    t ^= s ^ (s << 28);
+    s = (t ^ (t >> 14)) & 0x0000CCCC0000CCCCull;
+    t ^= s ^ (s << 14);
+    s = (t ^ (t >> 7)) & 0x00AA00AA00AA00AAull;
+    t ^= s ^ (s << 7);
+    bits[(size_t)ntx * nty + (size_t)ty * ntx + blockIdx.x] = t;
+  }
+}
+
+// Pass 2 for 8 rows: the bounded search of k_edt_rows (same rows, same results,
+// in integers: every sum is below 2^31, and its conversion to float rounds as
+// the float sum does), four distances a step, their candidates beyond the bound
+// being candidates all the same.  A wave takes 8 x 8 cells, one block of the
+// compact map: its 64 codes are 64 consecutive bytes.  Rows are dealt to the
+// XCDs in runs (workgroup b runs on XCD b mod 8), so the lines that neighbouring
+// row groups share stay in one L2.
+__global__ __launch_bounds__(1024) void k_edt_rows8(const uint16_t* __restrict__ g, float* __restrict__ D, int W, int H,
+                                                    int* __restrict__ slow, int* __restrict__ any_slow,
+                                                    const float* __restrict__ lut, uint8_t* __restrict__ idx8, int nby) {
+  extern __shared__ uint16_t s_d[];  // [x + 1][8 rows], a column without obstacles at either end
+  __shared__ uint8_t code_of[1024];  // code of a squared distance below 1024
+  __shared__ int s_bad[8], s_fin[8];
+  const int per = (int)(gridDim.x >> 3);  // gridDim.x: a multiple of 8, at least nby
+  const int by = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (by >= nby) return;  // the same in every thread
+  const int y0 = by * 8, t = threadIdx.x;
+  const int r = t & 7;
+  if (t < 8) s_bad[t] = s_fin[t] = 0;
+  code_of[t] = (uint8_t)RL_IDX8_ESCAPE;
+  if (t < 8) s_d[t] = s_d[(W + 1) * 8 + t] = (uint16_t)RL_EDT_NONE;
+  __syncthreads();
+  if (t < (int)RL_IDX8_ESCAPE) {  // lut[t] = sqrtf of the t-th sum of two squares
+    const int n = (int)(lut[t] * lut[t] + 0.5f);
+    code_of[n] = (uint8_t)t;
+  }
+  bool bad = false, fin = false;
+  for (int x = t >> 3; x < W; x += 128) {
+    const unsigned d = y0 + r < H ? g[(size_t)x * H + y0 + r] : RL_EDT_NONE;
+    if (d != RL_EDT_NONE) {
+      fin = true;
+      bad |= d * d + (unsigned)x * (unsigned)x >= 16777216u;
+    }
+    s_d[(x + 1) * 8 + r] = (uint16_t)d;
+  }
+  if (fin) s_fin[r] = 1;
+  if (bad) s_bad[r] = 1;
+  __syncthreads();
+  if (t < 8 && y0 + t < H) {
+    slow[y0 + t] = s_bad[t];
+    if (s_bad[t]) *any_slow = 1;
+  }
+  const int lane = t & 63, v = lane >> 3, y = y0 + v;
+  const int nbx = (W + 7) >> 3;
+  const bool row = y < H && !s_bad[v], found = s_fin[v] != 0;
+  for (int bx = t >> 6; bx < nbx; bx += 16) {
+    const int x = bx * 8 + (lane & 7);
+    unsigned code = RL_IDX8_ESCAPE;
+    if (row && x < W) {
+      const unsigned own = s_d[(x + 1) * 8 + v];
+      unsigned best = own * own;
+      if (found) {
+        const int dmax = max(x, W - 1 - x);
+        for (int d = 1; d <= dmax && (unsigned)(d * d) < best; d += 4) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int xa = max(x - d - q, -1), xb = min(x + d + q, W);
+            const unsigned a = s_d[(xa + 1) * 8 + v], b = s_d[(xb + 1) * 8 + v], dd = (unsigned)((d + q) * (d + q));
+            best = min(best, min(a * a, b * b) + dd);
+          }
+        }
+      }
+      const bool none = best >= RL_EDT_NONE * RL_EDT_NONE;
+      D[(size_t)x * H + y] = __builtin_sqrtf(none ? FLT_MAX : (float)best);
+      if (best < 1024u) code = code_of[best];
+    }
+    if (idx8) idx8[((size_t)bx * nby + by) * 64 + lane] = (uint8_t)code;
   }
 }
 
@@ -1413,43 +1572,54 @@ int launch_particles(rl_map* m, int method, bool sensor, float max_range, const 
 // tabulated distance (NaN, not sqrtf of a small integer) gets the escape code,
 // so the compact march reads it from the fp32 map and behaves as the fp32
 // march.
-int build_compact(rl_map* m, unsigned flags) {
+int alloc_compact(rl_map* m, unsigned flags) {
   if (flags & RL_MAP_NO_COMPACT) return RL_OK;
-  rl_ctx* c = m->ctx;
-  const int W = m->width, H = m->height;
-  m->nby = (H + 7) / 8;
-  const size_t nbytes = (size_t)((W + 7) / 8) * (size_t)m->nby * 64;
+  m->nby = (m->height + 7) / 8;
+  const size_t nbytes = (size_t)((m->width + 7) / 8) * (size_t)m->nby * 64;
   if (nbytes > 0xFFFFFFFFull) return RL_OK;  // 32-bit offsets only: such maps march the fp32 map
-  if (!m->d_idx8 && c->pool.alloc(&m->d_idx8, nbytes) != hipSuccess) {
+  if (!m->d_idx8 && m->ctx->pool.alloc(&m->d_idx8, nbytes) != hipSuccess) {
     (void)hipGetLastError();
     return fail(RL_ERR_NOMEM, "device allocation of the %zu-byte compact map failed", nbytes);
   }
+  return RL_OK;
+}
+
+int build_compact(rl_map* m, unsigned flags) {
+  rl_ctx* c = m->ctx;
+  TRY(alloc_compact(m, flags));
+  if (!m->d_idx8) return RL_OK;
+  const size_t nbytes = (size_t)((m->width + 7) / 8) * (size_t)m->nby * 64;
   hipLaunchKernelGGL(k_build_idx8, dim3(grid_for((long long)nbytes, 256)), dim3(256), 0, c->stream,
-                     (const float*)m->d_edt, (const float*)c->d_lut, m->d_idx8, W, H, m->nby, nbytes);
+                     (const float*)m->d_edt, (const float*)c->d_lut, m->d_idx8, m->width, m->height, m->nby, nbytes);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(RL_ERR_HIP, "compact map build: %s", hipGetErrorString(e));
   return RL_OK;
 }
 
-// Occupancy bitmap from m->d_occ (both orientations, 16 bytes of padding so
+// Occupancy bitmap of m->d_occ (both orientations, 16 zero bytes of padding so
 // that a window read at the last tile stays in the buffer).  Maps whose bitmap
 // would pass 4 GiB keep walking the byte grid.
-int build_bits(rl_map* m) {
+int alloc_bits(rl_map* m) {
   rl_ctx* c = m->ctx;
-  const int ntx = (m->width + 7) / 8, nty = (m->height + 7) / 8;
-  const size_t nbytes = (size_t)ntx * nty * 16;
+  const size_t nbytes = (size_t)((m->width + 7) / 8) * ((m->height + 7) / 8) * 16;
   if (nbytes + 16 > 0xFFFFFFFFull) return RL_OK;
   if (c->pool.alloc(&m->d_bits, nbytes + 16) != hipSuccess) {
     (void)hipGetLastError();
     return fail(RL_ERR_NOMEM, "device allocation of the %zu-byte occupancy bitmap failed", nbytes + 16);
   }
   m->bits_bytes = (unsigned)nbytes;
-  hipError_t e = hipMemsetAsync(m->d_bits + nbytes, 0, 16, c->stream);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_build_bits, dim3(grid_for((long long)ntx * nty, 256)), dim3(256), 0, c->stream,
-                       (const uint8_t*)m->d_occ, (unsigned long long*)m->d_bits, m->width, m->height, ntx, nty);
-    e = hipGetLastError();
-  }
+  HIP_TRY(hipMemsetAsync(m->d_bits + nbytes, 0, 16, c->stream));
+  return RL_OK;
+}
+
+int build_bits(rl_map* m) {
+  rl_ctx* c = m->ctx;
+  TRY(alloc_bits(m));
+  if (!m->d_bits) return RL_OK;
+  const int ntx = (m->width + 7) / 8, nty = (m->height + 7) / 8;
+  hipLaunchKernelGGL(k_build_bits, dim3(grid_for((long long)ntx * nty, 256)), dim3(256), 0, c->stream,
+                     (const uint8_t*)m->d_occ, (unsigned long long*)m->d_bits, m->width, m->height, ntx, nty);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(RL_ERR_HIP, "occupancy bitmap build: %s", hipGetErrorString(e));
   return RL_OK;
 }
@@ -1464,7 +1634,10 @@ int build_edt(rl_map* m, unsigned flags) {
   const bool cols = H <= 4096 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY);
   // the row search needs EDT_RB rows of the map in LDS (plus its flags) within 64 KiB
   const bool search = (size_t)EDT_RB * W * sizeof(float) + 64 <= 65536 && !(flags & RL_MAP_EDT_ENVELOPE_ONLY);
+  const bool tiled = cols && W <= RL_EDT_TILE_W;  // (and search: 4 W floats fit)
+  void *first = nullptr, *squares = nullptr;  // pool blocks: pass 1's result; g made later
   float* g = nullptr;
+  uint16_t* g16 = nullptr;
   int *v = nullptr, *slow = nullptr;  // slow[y]: row y is left to the envelope
   double* z = nullptr;
   int* any_slow;  // in pinned memory, written by the kernel where a row is
@@ -1482,23 +1655,43 @@ int build_edt(rl_map* m, unsigned flags) {
     return c->pool.alloc(&v, N * sizeof(int)) == hipSuccess &&
            c->pool.alloc(&z, (N + (size_t)W + (size_t)H) * sizeof(double)) == hipSuccess;
   };
+  auto columns = [&] { hipLaunchKernelGGL(k_edt_cols, dim3(W), dim3(256), 0, c->stream, m->d_occ, g, H); };
   auto rows_envelope = [&](const int* only) {
     hipLaunchKernelGGL(k_edt_envelope, dim3(grid_for(H, 64)), dim3(64), 0, c->stream, (const float*)g, m->d_edt, H, W,
                        (long long)H, 1LL, v, z, 1, only);
   };
   do {
-    if (c->pool.alloc(&g, N * sizeof(float)) != hipSuccess || hipMalloc(&slow, (size_t)H * sizeof(int)) != hipSuccess ||
-        (!(cols && search) && !stacks())) {
+    // the rows' marks follow the first pass's result
+    const size_t g_bytes = (N * (tiled ? sizeof(uint16_t) : sizeof(float)) + 15) & ~(size_t)15;
+    char* p = nullptr;
+    if (c->pool.alloc(&p, g_bytes + (size_t)H * sizeof(int)) != hipSuccess) {
       oom();
       break;
     }
+    first = p;
+    slow = (int*)(p + g_bytes);
+    if (tiled)
+      g16 = (uint16_t*)p;
+    else
+      g = (float*)p;
+    if (!(cols && search) && !stacks()) {
+      oom();
+      break;
+    }
+    if (tiled && ((rc = alloc_compact(m, flags)) != RL_OK || (rc = alloc_bits(m)) != RL_OK)) break;
     hipError_t e = hipEventRecord(e0, c->stream);
     if (e != hipSuccess) {
       rc = fail(RL_ERR_HIP, "distance transform: %s", hipGetErrorString(e));
       break;
     }
-    if (cols) {
-      hipLaunchKernelGGL(k_edt_cols, dim3(W), dim3(256), 0, c->stream, m->d_occ, g, H);
+    if (tiled) {
+      const int ntx = (W + 7) / 8, nty = (H + 7) / 8;
+      hipLaunchKernelGGL(k_edt_cols8, dim3((unsigned)ntx), dim3(1024), 0, c->stream, (const uint8_t*)m->d_occ, g16, W, H,
+                         (unsigned long long*)m->d_bits, ntx, nty);
+      hipLaunchKernelGGL(k_edt_rows8, dim3((unsigned)(nty + 7) / 8 * 8), dim3(1024), (size_t)(W + 2) * 16, c->stream,
+                         (const uint16_t*)g16, m->d_edt, W, H, slow, any_slow, (const float*)c->d_lut, m->d_idx8, nty);
+    } else if (cols) {
+      columns();
     } else {
       hipLaunchKernelGGL(k_edt_init, dim3(grid_for((long long)N, 256)), dim3(256), 0, c->stream,
                          m->d_occ, m->d_edt, N);
@@ -1508,21 +1701,23 @@ int build_edt(rl_map* m, unsigned flags) {
     }
     // Pass 2: the bounded search where it is exact, the lower envelope on the
     // rows it marks (or on every row when the envelope is asked for).
-    if (search)
+    if (!tiled && search)
       hipLaunchKernelGGL(k_edt_rows, dim3((H + EDT_RB - 1) / EDT_RB), dim3(256),
                          (size_t)EDT_RB * W * sizeof(float), c->stream, (const float*)g,
                          m->d_edt, W, H, slow, any_slow, 1);
-    else
+    else if (!tiled)
       rows_envelope(nullptr);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
-    if (e == hipSuccess && (rc = build_compact(m, flags)) == RL_OK) rc = build_bits(m);
+    if (e == hipSuccess && !tiled && (rc = build_compact(m, flags)) == RL_OK) rc = build_bits(m);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess && rc == RL_OK && *(volatile int*)any_slow) {
-      if (!v && !stacks()) {
+      if (!g && c->pool.alloc(&squares, N * sizeof(float)) == hipSuccess) g = (float*)squares;
+      if (!g || (!v && !stacks())) {
         oom();
         break;
       }
+      if (tiled) columns();  // the squares that the envelope takes
       rows_envelope(slow);
       e = hipGetLastError();
       if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
@@ -1533,10 +1728,7 @@ int build_edt(rl_map* m, unsigned flags) {
     if (rc == RL_OK) (void)hipEventElapsedTime(&m->edt_ms, e0, e1);
   } while (0);
   (void)hipStreamSynchronize(c->stream);
-  c->pool.release(g, true);
-  c->pool.release(v, true);
-  c->pool.release(z, true);
-  if (slow) (void)hipFree(slow);
+  for (void* p : {first, squares, (void*)v, (void*)z}) c->pool.release(p, true);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return rc;

@@ -597,3 +597,27 @@ def test_map_buffers_reused(ctx):
         ctx.set_stream(None)
     for k, out in enumerate(outs):
         assert_bits_equal(out.cpu().numpy()[:3000], want[k % 3], f"map {k}")
+
+
+@pytest.mark.parametrize("h,w", [(1, 1), (7, 8), (8, 7), (65, 17), (64, 64), (129, 130), (4096, 9), (4097, 9),
+                                 (20, 3966), (20, 3967), (1500, 3900)])
+def test_map_build_tiles(ctx, h, w):
+    """What a map's creation forms together -- distance transform, compact map,
+    occupancy bitmap -- at the edges of its tiles (8 columns, 8 rows, 64-cell
+    words, 4096 rows, 3966 columns; the last size has rows left to the envelope):
+    distances, marches over the compact map and Bresenham walks over the bitmap."""
+    rng = np.random.default_rng(h * 5000 + w)
+    img = (rng.random((h, w)) < (0.02 if h * w < 1e6 else 2e-6)).astype(np.uint8) * np.uint8(200)
+    if h * w < 100:
+        img[0, 0] = 0
+    if h == 1500:
+        img[:] = _points((h, w), [(0, w - 10), (700, 10)])
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    assert_bits_equal(dm.edt(), O.edt(img), "edt")
+    n = 4000
+    q = np.stack([rng.uniform(-1, w + 1, n), rng.uniform(-1, h + 1, n), rng.uniform(0, 2 * math.pi, n)],
+                 1).astype(np.float32)
+    out = np.empty(n, np.float32)
+    for method, kind in ((rl.RL_METHOD_RM, "rm"), (rl.RL_METHOD_BL, "bl")):
+        dm.calc_range_many(method, 300.0, q, out, n)
+        assert_bits_equal(out, O.Oracle(img, 300.0, kind).calc_range_many(q), kind)
