@@ -903,53 +903,98 @@ __global__ __launch_bounds__(256) void k_particles_xcd(MapDev m, TrigDev trig, f
                                  j0, base, boxes + wib * RL_BOX_BYTES, terms + wib * 64, pre);
 }
 
-// GiantLUTCast's table by tiles of RL_GLT_TILE consecutive cells (x-major
-// order, so mostly neighbours along y) and all their bins: a wave marches 4
-// bins' directions from 16 neighbouring cells, rays of similar length, instead
-// of 64 directions from one cell (a wave runs as long as its longest ray).
-// The tile's entries are assembled in LDS in the table's order (cell-major,
-// RL_GLT_TILE * td entries, the launch's dynamic LDS) and stored contiguously.
-// Same values as k_glt_build, entry by entry.  Measured on the 2048^2
-// corridor map with 108 bins: tiles of 4, 8, 16, 32, 64, 128, 256 cells took
-// 4.84, 3.95, 3.69, 3.81, 4.03, 5.18, 11.4 ms (one entry per thread: 5.34 ms);
-// larger tiles hold more LDS per workgroup and leave fewer of them per CU.
-#ifndef RL_GLT_TILE
-#define RL_GLT_TILE 16  // cells per tile of k_glt_build_tiles (a power of two)
-#endif
+// March steps of the cells for the table build, x-major with a row and a column
+// more than the map: steps[x * (H + 1) + y] = max(d * 0.999f, 1.0f) of cell (x, y),
+// +infinity where a march ends (an occupied cell, or off the map).
+__global__ __launch_bounds__(256) void k_glt_steps(const float* __restrict__ edt, int W, int H,
+                                                   float* __restrict__ steps) {
+  const int x = (int)blockIdx.y;
+  const int y = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (y > H) return;
+  float g = INFINITY;
+  if (x < W && y < H) {
+    const float d = edt[(size_t)x * H + y];
+    const float st = d * 0.999f;
+    const float s = (st < 1.0f) ? 1.0f : st;
+    // an infinite distance ends the march past max_range, as any step that long
+    if (!(d <= 0.0f)) g = (s == INFINITY) ? FLT_MAX : s;
+  }
+  steps[(size_t)x * (unsigned)(H + 1) + y] = g;
+}
+
+// GiantLUTCast's table by tiles of 4 x 4 cells and all their bins, a tile per
+// wave: the wave marches 4 bins' directions from the 16 cells, rays of similar
+// length (a wave runs as long as its longest ray; on the 2048^2 corridor map
+// with 108 bins 7.1 reads on average, where a row of 16 cells takes 8.7, 64
+// directions from one cell 15.5, and a ray by itself 3.6).  The tile's entries
+// are assembled in LDS and stored by rows of cells, which are contiguous in the
+// table.  Same values as k_glt_build, entry by entry.
+//
+// The launch is bound by its L1 accesses (1.58 G, one per lane and read: 2.7 ms
+// at one a cycle and CU) and by VALU work (1.06 G, 1.8 ms), so the march reads the cells' steps
+// (k_glt_steps) instead of their codes: a position off the map is clamped to the
+// border of infinite steps, an ending cell's infinite step takes t past
+// max_range, and one comparison per read decides whether the ray goes on (12
+// VALU instructions per read; codes, a step table and separate tests took 22).
+// A lane's rays all start at one cell, whose step is read once.  The float
+// operations and their order are rm_march's.  Measured: 3.69 ms with codes and
+// tiles of a workgroup, 3.44 with steps, 2.91 with a tile per wave (no wave waits
+// for another's rays), 2.59 with 4 x 4 cells; byte codes with a step table in LDS
+// took as long as the steps (2.93, in blocks 2.82).
+#define RL_GLT_TILE 16      // cells of a tile: 4 x 4
 #define RL_GLT_TILE_TD 256  // the largest td built by tiles
-__global__ __launch_bounds__(256) void k_glt_build_tiles(MapDev m, float max_range, int td,
-                                                         const float2* __restrict__ dirs, float limits_div_max,
-                                                         uint16_t* __restrict__ out, long long ncells) {
-  __shared__ float lut[RL_LUT_SIZE];
-  extern __shared__ uint16_t tile[];  // RL_GLT_TILE * td entries
-  stage_lut<RL_METHOD_RM>(m, lut);
-  const long long ntiles = (ncells + RL_GLT_TILE - 1) / RL_GLT_TILE;
-  for (long long t = blockIdx.x; t < ntiles; t += gridDim.x) {  // the same in every thread
-    const long long first = t * RL_GLT_TILE;
-    const int nc = (int)min((long long)RL_GLT_TILE, ncells - first);
-    for (int r = threadIdx.x; r < RL_GLT_TILE * td; r += blockDim.x) {
-      const int c = r & (RL_GLT_TILE - 1), bin = r / RL_GLT_TILE;  // a wave: 64 / RL_GLT_TILE bins
-      if (c >= nc) continue;
-      const long long cell = first + c;
-      const int x = (int)(cell / m.height), y = (int)(cell - (long long)x * m.height);
+__global__ __launch_bounds__(256) void k_glt_build_tiles(const float* __restrict__ steps, int W, int H, float max_range,
+                                                         int td, const float2* __restrict__ dirs, float limits_div_max,
+                                                         uint16_t* __restrict__ out, unsigned ntx, unsigned nty) {
+  extern __shared__ __align__(16) uint16_t tiles[];  // RL_GLT_TILE * td entries per wave
+  const unsigned pitch = 4u * (unsigned)(H + 1);  // bytes; the steps are below 4 GiB (checked by the caller)
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)steps, (short)0, (int)((unsigned)(W + 1) * pitch), 0x00020000);
+  const int lane = threadIdx.x & 63, c = lane & (RL_GLT_TILE - 1);
+  uint16_t* tile = tiles + (threadIdx.x >> 6) * (RL_GLT_TILE * td);
+  const unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6);  // tiles x-major; fewer than 2^27 (steps below 4 GiB)
+  if (t >= ntx * nty) return;  // the same in every lane of the wave; no workgroup barrier below
+  const int x0 = (int)(t / nty) * 4, y0 = (int)(t - (t / nty) * nty) * 4;
+  const int x = x0 + (c >> 2), y = y0 + (c & 3);
+  if (x < W && y < H) {
+    const float fx = (float)x, fy = (float)y;
+    // the first read is at the cell itself, whatever the direction
+    const float g0 = steps[(size_t)x * (unsigned)(H + 1) + y];
+    for (int bin = lane / RL_GLT_TILE; bin < td; bin += 64 / RL_GLT_TILE) {
       const float2 d = dirs[bin];
-      const float fx = (float)x, fy = (float)y;
-      int unused;
-      // the plain march: the table is bound by the work of its many rays, not
-      // by the longest chain, and speculation's extra reads cost more than
-      // they save (2048^2 corridor map, 108 bins, one entry per thread: 5.31 ms
-      // plain, 6.10 ms at width 2 after 8 reads, 5.64-5.78 ms after 16 or 32)
-      float v = (m.idx8 && rl::fast_march_ok(fx, fy, max_range))
-                    ? rl::rm_march_idx8<false, 1>(m, lut, rl::Box{nullptr, 0, 0}, max_range, fx, fy, d.x, d.y,
-                                                  &unused)
-                    : rl::rm_march<false>(m.edt, m.width, m.height, max_range, fx, fy, d.x, d.y, &unused);
+      float s = g0, tc = 0.0f, tn = g0;  // the last step read, its position and the next
+      unsigned px = (unsigned)x, py = (unsigned)y;
+      while (tn < max_range) {
+        tc = tn;
+        px = min((unsigned)(int)(fx + d.x * tc), (unsigned)W);
+        py = min((unsigned)(int)(fy + d.y * tc), (unsigned)H);
+        s = __builtin_bit_cast(float,
+                               __builtin_amdgcn_raw_buffer_load_b32(rsrc, __umul24(px, pitch) + (py << 2), 0, 0));
+        tn = tc + s;
+      }
+      float v = max_range;
+      if (s == INFINITY && px < (unsigned)W && py < (unsigned)H) {
+        const float xd = (float)(int)px - fx;
+        const float yd = (float)(int)py - fy;
+        v = __builtin_sqrtf(xd * xd + yd * yd);
+      }
       v = (v < max_range) ? v : max_range;  // std::min(max_range, r)
       tile[c * td + bin] = (uint16_t)(unsigned)(v * limits_div_max);
     }
-    __syncthreads();
-    uint16_t* dst = out + first * td;
-    for (int e = threadIdx.x; e < nc * td; e += blockDim.x) dst[e] = tile[e];
-    __syncthreads();  // the tile is stored before the next one is assembled
+  }
+  // the wave reads what its other lanes wrote
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int n = min(4, H - y0) * td;  // entries of a row of cells
+  for (int u = 0; u < 4 && x0 + u < W; ++u) {
+    uint16_t* dst = out + ((size_t)(x0 + u) * (unsigned)H + (unsigned)y0) * (unsigned)td;
+    const uint16_t* src = tile + u * 4 * td;  // 8 td bytes each
+    if ((((uintptr_t)dst | (unsigned)(2 * n)) & 7) == 0) {
+      for (int e = lane; e < n / 4; e += 64) ((uint2*)dst)[e] = ((const uint2*)src)[e];
+    } else {
+      for (int e = lane; e < n; e += 64) dst[e] = src[e];
+    }
   }
 }
 
@@ -993,10 +1038,8 @@ __global__ __launch_bounds__(256) void k_glt_build(MapDev m, float max_range, in
     const float2 d = dirs[i];
     const float fx = (float)x, fy = (float)y;
     int unused;
-    // the default speculation: the plain march instantiated here as well (as
-    // k_glt_build_tiles marches) changed the compiler's code for the particle
-    // kernels (k_particles<RM, sensor> 2073 -> 2557 VALU instructions, about
-    // 1% slower); this kernel builds only tables of more than 256 bins
+    // this kernel builds only tables of more than 256 bins and those of maps
+    // whose steps k_glt_build_tiles cannot hold
     float r = (m.idx8 && rl::fast_march_ok(fx, fy, max_range))
                   ? rl::rm_march_idx8<false>(m, lut, rl::Box{nullptr, 0, 0}, max_range, fx, fy, d.x, d.y, &unused)
                   : rl::rm_march<false>(m.edt, m.width, m.height, max_range, fx, fy, d.x, d.y, &unused);
@@ -1998,18 +2041,25 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
   long long blocks = (total + 255) / 256;
   if (blocks > (1LL << 20)) blocks = 1LL << 20;
   float2* dirs = nullptr;
+  // the cells' steps: 32-bit byte offsets, and scratch of 4 bytes a cell
+  const size_t steps_bytes = ((size_t)m->width + 1) * ((size_t)m->height + 1) * sizeof(float);
+  float* steps = nullptr;
+  if (theta_disc <= RL_GLT_TILE_TD && steps_bytes <= 0xFFFFFFFFull &&
+      c->pool.alloc(&steps, steps_bytes) != hipSuccess)
+    (void)hipGetLastError();  // no room: one entry per thread, without them
   hipError_t e = hipMalloc(&dirs, (size_t)theta_disc * sizeof(float2));
   if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_glt_dirs, dim3((unsigned)((theta_disc + 255) / 256)), dim3(256), 0, c->stream, c->trig,
                        theta_disc, step, dirs);
-    const long long ncells = (long long)m->width * m->height;
-    if (theta_disc <= RL_GLT_TILE_TD) {
-      long long tiles = (ncells + RL_GLT_TILE - 1) / RL_GLT_TILE;
-      if (tiles > (1LL << 20)) tiles = 1LL << 20;
-      hipLaunchKernelGGL(k_glt_build_tiles, dim3((unsigned)tiles), dim3(256),
-                         (unsigned)(RL_GLT_TILE * theta_disc * sizeof(uint16_t)), c->stream, m->dev(), max_range,
-                         theta_disc, (const float2*)dirs, limits_div_max, m->d_glt, ncells);
+    if (steps) {
+      hipLaunchKernelGGL(k_glt_steps, dim3((unsigned)grid_for(m->height + 1, 256), (unsigned)(m->width + 1)), dim3(256),
+                         0, c->stream, (const float*)m->d_edt, m->width, m->height, steps);
+      const unsigned ntx = (unsigned)(m->width + 3) / 4, nty = (unsigned)(m->height + 3) / 4;
+      hipLaunchKernelGGL(k_glt_build_tiles, dim3((ntx * nty + 3) / 4), dim3(256),
+                         (unsigned)(4 * RL_GLT_TILE * theta_disc * sizeof(uint16_t)), c->stream, (const float*)steps,
+                         m->width, m->height, max_range, theta_disc, (const float2*)dirs, limits_div_max, m->d_glt, ntx,
+                         nty);
     } else if (total <= 0xFFFFFFFFLL)
       hipLaunchKernelGGL(k_glt_build<false>, dim3((unsigned)blocks), dim3(256), 0, c->stream, m->dev(), max_range,
                          theta_disc, (const float2*)dirs, limits_div_max, m->d_glt, total);
@@ -2022,6 +2072,8 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) (void)hipEventElapsedTime(&m->glt_ms, e0, e1);
   if (dirs) (void)hipFree(dirs);
+  (void)hipStreamSynchronize(c->stream);
+  c->pool.release(steps, true);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (e != hipSuccess) {

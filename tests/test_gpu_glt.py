@@ -168,3 +168,17 @@ def test_glt_special_headings_and_errors(ctx):
     assert np.isnan(out[0]) and np.isnan(out[1]) and np.isnan(out[2])  # NaN / non-terminating headings
     assert_bits_equal(out[3:9], want[3:9], "finite headings")
     assert np.isnan(out[9]) and out[10] == np.float32(R) and out[11] == np.float32(R)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 5), (4, 4), (5, 3), (17, 66), (64, 31)])
+@pytest.mark.parametrize("td,R", [(1, 20.0), (7, 3.5), (16, 1000.0)])
+def test_glt_tiles_ragged(ctx, w, h, td, R):
+    """Whole tables where the 4 x 4 tiles are cut by the map's edges, with rays
+    that leave the map, end at max_range and start in walls, and distances past
+    the compact map's codes."""
+    img = (np.random.default_rng(w * 100 + h).random((h, w)) < 0.05).astype(np.uint8)
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    dm.build_giant_lut(R, td)
+    got, _, _, _ = dm.giant_lut()
+    want = O.Oracle(img, R, "glt", theta_disc=td).glt
+    assert np.array_equal(got, want.reshape(got.shape))
