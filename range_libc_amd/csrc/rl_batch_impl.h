@@ -31,8 +31,14 @@ struct BatchMap {
   float* ranges;
   double* weights;
   int N, M, S;
+  int G;  // particles per wave of k_batch_pool
   int sensor;
 };
+
+// Rays per wave of k_batch_pool at most: with more, the resident waves span so
+// many maps that these fall out of the L2s (16 maps of up to 2048^2, 5.6 M rays:
+// 64, 96, 128, 192, 256, 512 rays 290, 270, 267, 267, 272, 332 us).
+#define RL_BATCH_WAVE_RAYS 128
 
 struct BatchItem {
   int map;    // -1: an empty item (padding of the XCD-affine order)
@@ -77,6 +83,30 @@ __global__ __launch_bounds__(256) void k_batch(const BatchMap* __restrict__ maps
   }
 }
 
+// Ray marching from a pool of rays per wave (pool_particles): an item is the
+// particles that the workgroup's four waves take.
+__global__ __launch_bounds__(256, 7) void k_batch_pool(const BatchMap* __restrict__ maps,
+                                                       const BatchItem* __restrict__ items, int n_items,
+                                                       TrigDev trig) {
+  __shared__ float lut[RL_LUT_SIZE];
+  __shared__ PoolLds pool[4];
+  for (int i = threadIdx.x; i < RL_LUT_SIZE; i += blockDim.x) lut[i] = maps[0].m.steps[i];
+  __syncthreads();
+  const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
+    const BatchItem item = items[it];
+    if (item.map < 0) continue;
+    const BatchMap& bm = maps[item.map];
+    const int first = item.first + wib * bm.G, np = min(bm.G, bm.N - first);
+    if (bm.sensor)
+      pool_particles<POOL_STEP>(bm.m, lut, trig, bm.max_range, bm.ins, bm.angles, bm.obs, bm.table, bm.K, bm.ranges,
+                                bm.weights, first, np, bm.M, pool + wib);
+    else
+      pool_particles<POOL_RANGES>(bm.m, lut, trig, bm.max_range, bm.ins, bm.angles, bm.obs, bm.table, bm.K, bm.ranges,
+                                  bm.weights, first, np, bm.M, pool + wib);
+  }
+}
+
 struct rl_batch {
   rl_ctx* ctx = nullptr;
   int method = RL_METHOD_RM;
@@ -93,6 +123,7 @@ struct rl_batch {
   BatchMap* d_maps = nullptr;
   BatchItem* d_items = nullptr;
   int n_items = 0;
+  bool pooled = false;  // the items are those of k_batch_pool
   size_t cap_maps = 0, cap_items = 0;
 };
 
@@ -105,6 +136,12 @@ int batch_upload(rl_batch* b) {
   std::vector<std::pair<double, BatchItem>> items;
   b->gens.resize(nj);
   for (int i = 0; i < nj; ++i) b->gens[i] = b->jobs[i].map->gen.load();
+  // one kernel for the whole list: pooled when every map's rays could be
+  long long rays = 0;
+  for (const rl_batch_job& j : b->jobs) rays += (long long)j.num_particles * j.num_angles;
+  b->pooled = b->method == RL_METHOD_RM && !b->lds_box;
+  for (const rl_batch_job& j : b->jobs)
+    b->pooled = b->pooled && (j.num_particles == 0 || pool_pays(j.map, rays, j.num_angles));
   for (int i = 0; i < nj; ++i) {
     const rl_batch_job& j = b->jobs[i];
     BatchMap& bm = maps[i];
@@ -123,7 +160,8 @@ int batch_upload(rl_batch* b) {
     int S = segment_size(j.num_angles);
     if (S > b->rays_per_wave) S = b->rays_per_wave;
     bm.S = S;
-    const int chunk = 4 * (64 / S);
+    bm.G = pool_particles_per_wave(std::min(rays, RL_BATCH_WAVE_RAYS * (long long)RL_POOL_RESIDENT), j.num_angles);
+    const int chunk = 4 * (b->pooled ? bm.G : 64 / S);
     const double ray_cost = (double)j.num_angles * (1.0 + b->reads_per_ray[i]);
     for (int f = 0; f < j.num_particles; f += chunk) {
       int cnt = j.num_particles - f < chunk ? j.num_particles - f : chunk;
@@ -232,7 +270,9 @@ int batch_launch_locked(rl_batch* b) {
     grid -= grid % b->xcds;
     if (grid == 0) grid = b->n_items;
   }
-  if (b->method == RL_METHOD_BL)
+  if (b->pooled)
+    hipLaunchKernelGGL(k_batch_pool, dim3(grid), dim3(256), 0, c->stream, b->d_maps, b->d_items, b->n_items, c->trig);
+  else if (b->method == RL_METHOD_BL)
     hipLaunchKernelGGL(k_batch<RL_METHOD_BL>, dim3(grid), dim3(256), 0, c->stream, b->d_maps, b->d_items,
                        b->n_items, c->trig, b->lds_box);
   else if (b->method == RL_METHOD_GLT)

@@ -15,6 +15,9 @@
 //                   repeated-angles frames
 //   k_sensor        eval_sensor_model: one particle per wave segment
 //   k_fused         calc_range_repeat_angles_eval_sensor_model
+//   k_particles     one ray per lane, a particle's beams on a wave segment: ranges
+//                   and weights; k_particles_pool: many rays per lane, for launches
+//                   of more rays than lanes
 //
 // Build: hipcc --offload-arch=gfx950 -O3 -ffp-contract=off (see build.py).
 #include <dlfcn.h>
@@ -849,6 +852,143 @@ __device__ __forceinline__ void particle_beams(const MapDev& m, const float* lut
   if (SENSOR && valid && j0 == 0) weights[p] = w;
 }
 
+// Ray marching over the compact map from a pool of rays per wave (rl::pool_march):
+// the wave's np particles (first, first + 1, ...; none: returns) times their M
+// beams, RL_POOL_RAYS at most at a time.  All lanes form the directions, the pool
+// is marched, then all lanes turn the results into ranges and weights' terms and
+// one lane per particle multiplies these in beam order.  Same operations per ray
+// as particle_beams, so the same bits.  Wave-uniform arguments.
+//
+// OUT selects what is written, as the call it stands for forms it: the ranges
+// (k_particles without a sensor model), ranges and weights (k_particles), or the
+// weights from ranges in grid units (k_fused).
+//
+// LDS: 18.5 KB a workgroup of four waves, so seven fit a compute unit (7168 waves
+// on the chip).
+#define RL_POOL_RAYS 512     // at most this many rays of a wave in LDS, 8 bytes each
+#define RL_POOL_PARTICLES 32 // at most this many particles of a wave
+enum { POOL_RANGES, POOL_STEP, POOL_WEIGHTS };
+struct PoolPose {
+  float x, y, theta, fast;  // grid pose; fast = 0: cast outside the pool
+};
+struct PoolLds {
+  double ray[RL_POOL_RAYS];  // a ray's direction, then its squared range, then its term
+  PoolPose pose[RL_POOL_PARTICLES];
+};
+
+// Particle of ray r < RL_POOL_RAYS among rays of mb beams per particle, inv =
+// 1.0f / mb: exact, as (r + 0.5) / mb is at least 0.5 / mb from a whole number,
+// more than the two roundings move it.
+__device__ __forceinline__ int pool_particle(int r, float inv) { return (int)(((float)r + 0.5f) * inv); }
+
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int OUT>
+__device__ __forceinline__ void pool_particles(const MapDev& m, const float* lut, const TrigDev& trig,
+                                               float max_range, const float* __restrict__ ins,
+                                               const float* __restrict__ angles,
+                                               const float* __restrict__ obs,
+                                               const double* __restrict__ table, int K,
+                                               float* __restrict__ ranges, double* __restrict__ weights,
+                                               int first, int np, int M, PoolLds* shared) {
+  if (np <= 0) return;
+  const int lane = threadIdx.x & 63;
+  RL_LDS PoolPose* pose = (RL_LDS PoolPose*)shared->pose;
+  RL_LDS float2* ray = (RL_LDS float2*)shared->ray;
+  RL_LDS double* term = (RL_LDS double*)shared->ray;
+  const float hi = (float)((double)(float)K - 1.0);
+  wave_lds_sync();  // the wave's reads for the particles before
+  if (lane < np) {
+    const float* in = ins + 3 * (size_t)(first + lane);
+    float gx, gy;
+    rl::to_grid(m.world, in[0], in[1], &gx, &gy);
+    const bool fast = 0.0f < max_range && rl::fast_march_ok(gy, gx, max_range);
+    pose[lane].x = fast ? gy : -1.0f;
+    pose[lane].y = fast ? gx : -1.0f;
+    pose[lane].theta = -in[2] + m.world.rotation_const;
+    pose[lane].fast = fast ? 1.0f : 0.0f;
+  }
+  double w = 1.0;
+  for (int jb = 0; jb < M; jb += RL_POOL_RAYS) {
+    const int mb = min(M - jb, RL_POOL_RAYS), n = np * mb;
+    const float inv = 1.0f / (float)mb;
+    wave_lds_sync();  // the poses; the terms of the beams before have been read
+    for (int r = lane; r < n; r += 64) {
+      const int pi = pool_particle(r, inv);
+      float dx, dy;
+      rl::sincos_libc(pose[pi].theta - angles[jb + r - pi * mb], trig, &dy, &dx);
+      // a NaN direction (NaN or infinite heading) ends at max_range: its first
+      // step leaves the map, and a hit at its origin is not taken
+      const bool nan = dx != dx || dy != dy;
+      ray[r].x = nan ? -4e9f : dx;
+      ray[r].y = nan ? __int_as_float(0x7fc00000) : dy;
+    }
+    wave_lds_sync();
+    rl::pool_march(
+        m, lut, max_range, n,
+        [&](int s, float* x0, float* y0, float* dx, float* dy) {
+          const int pi = pool_particle(s, inv);
+          *x0 = pose[pi].x, *y0 = pose[pi].y;
+          *dx = ray[s].x, *dy = ray[s].y;
+        },
+        [&](int s, float d, bool squared) {
+          const bool nan = ray[s].y != ray[s].y;
+          ray[s].x = nan ? -1.0f : d;
+          if (!squared && !nan) ray[s].y = 2.0f;  // (no direction's value: x is the range itself)
+        });
+    wave_lds_sync();
+    for (int r = lane; r < n; r += 64) {
+      const int pi = pool_particle(r, inv), j = jb + r - pi * mb;
+      float d = ray[r].x;
+      if (ray[r].y != 2.0f) d = d < 0.0f ? max_range : __builtin_sqrtf(d);
+      if (pose[pi].fast == 0.0f) {
+        const float* in = ins + 3 * (size_t)(first + pi);
+        float gx, gy, s, c;
+        rl::to_grid(m.world, in[0], in[1], &gx, &gy);
+        rl::sincos_libc(pose[pi].theta - angles[j], trig, &s, &c);
+        int unused;
+        d = rl::rm_march<false>(m.edt, m.width, m.height, max_range, gy, gx, c, s, &unused);
+      }
+      if (OUT != POOL_WEIGHTS) {
+        d = d * m.world.scale;
+        ranges[(size_t)(first + pi) * M + j] = d;
+      }
+      if (OUT != POOL_RANGES) {
+        const float o = rl::clamp_table(obs[j] * m.world.inv_scale, hi);
+        // (no world scale in the weights-only call, RangeLib.h:602-603)
+        const float dd = rl::clamp_table(OUT == POOL_WEIGHTS ? d : d * m.world.inv_scale, hi);
+        term[r] = rl::glb(table)[(size_t)(int)o * (size_t)K + (size_t)(int)dd];
+      }
+    }
+    if (OUT != POOL_RANGES) {
+      wave_lds_sync();
+      if (lane < np) w = slot_product(w, term + lane * mb, mb);
+    }
+  }
+  if (OUT != POOL_RANGES && lane < np) weights[first + lane] = w;
+}
+
+template <int OUT>
+__global__ __launch_bounds__(256, 7) void k_particles_pool(MapDev m, TrigDev trig, float max_range,
+                                                           const float* __restrict__ ins,
+                                                           const float* __restrict__ angles,
+                                                           const float* __restrict__ obs,
+                                                           const double* __restrict__ table, int K,
+                                                           float* __restrict__ ranges,
+                                                           double* __restrict__ weights, int N, int M, int G) {
+  __shared__ float lut[RL_LUT_SIZE];
+  __shared__ PoolLds pool[4];
+  stage_lut<RL_METHOD_RM>(m, lut);
+  const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int first = ((int)blockIdx.x * 4 + wib) * G;
+  pool_particles<OUT>(m, lut, trig, max_range, ins, angles, obs, table, K, ranges, weights, first, min(G, N - first),
+                      M, pool + wib);
+}
+
 // Particles in input order: wave segment -> particle.
 template <int METHOD, bool SENSOR>
 __global__ __launch_bounds__(256) void k_particles(MapDev m, TrigDev trig, float max_range,
@@ -1523,6 +1663,40 @@ int launch_sensor(rl_map* m, const float* obs, const float* ranges, double* outs
   return RL_OK;
 }
 
+// Rule for the pool of rays per wave (k_particles_pool).  One ray per lane
+// (k_particles) keeps 4096 waves resident, and is the better form while all rays
+// fit them at once: then a launch lasts as long as its longest ray, which a pool
+// starts later (2048^2 corridors, 60 beams: 4000 particles 22.2 us, pooled 25.8;
+// 5000: 29.6, 26.5; 6000: 34.5, 27.8; 40000: 150.6, 67.3).  A wave's rays are
+// cast together from 96 up, and up to what LDS holds as long as the launch still
+// has a wave for each that the chip keeps resident (1531 x 1999, 107 beams,
+// 20011 particles: 128, 256, 384, 512 rays a wave 121, 119, 103, 100 us; 12000:
+// 84, 74, 80, 86).
+#define RL_POOL_MIN_RAYS (4096 * 64)
+#define RL_POOL_RESIDENT 7168  // waves of the pool's kernels that the chip keeps resident
+#define RL_POOL_WAVE_RAYS 96   // rays of a wave at least
+
+bool pool_pays(const rl_map* m, long long rays, int M) {
+  return rays > RL_POOL_MIN_RAYS && M * RL_POOL_PARTICLES >= RL_POOL_WAVE_RAYS && m->d_idx8 && !m->ctx->lds_box;
+}
+
+// Particles of M beams that a wave takes of a launch of `rays` rays.
+int pool_particles_per_wave(long long rays, int M) {
+  const long long want = std::max<long long>(RL_POOL_WAVE_RAYS, rays / RL_POOL_RESIDENT);
+  const long long g = std::min<long long>((want + M - 1) / M, std::min(RL_POOL_RAYS / M, RL_POOL_PARTICLES));
+  return g < 1 ? 1 : (int)g;
+}
+
+template <int OUT>
+void launch_pool(rl_map* m, float max_range, const float* ins, const float* angles, const float* obs, float* ranges,
+                 double* weights, int N, int M) {
+  const int G = pool_particles_per_wave((long long)N * M, M);
+  const unsigned blocks = (unsigned)(((long long)N + 4 * G - 1) / (4 * G));
+  hipLaunchKernelGGL(k_particles_pool<OUT>, dim3(blocks), dim3(256), 0, m->ctx->stream, m->dev(), m->ctx->trig,
+                     max_range, ins, angles, obs, OUT == POOL_RANGES ? nullptr : m->d_table,
+                     OUT == POOL_RANGES ? 1 : m->table_width, ranges, weights, N, M, G);
+}
+
 int launch_fused(rl_map* m, int method, float max_range, const float* ins, const float* angles,
                  const float* obs, double* weights, int N, int M) {
   TRY(check_map(m, method, max_range));
@@ -1531,7 +1705,9 @@ int launch_fused(rl_map* m, int method, float max_range, const float* ins, const
   int S = segment_size(M);
   long long waves = ((long long)N + 64 / S - 1) / (64 / S);
   dim3 grid(grid_for(waves * 64, 256)), block(256);
-  if (method == RL_METHOD_BL)
+  if (method == RL_METHOD_RM && pool_pays(m, (long long)N * M, M))
+    launch_pool<POOL_WEIGHTS>(m, max_range, ins, angles, obs, nullptr, weights, N, M);
+  else if (method == RL_METHOD_BL)
     hipLaunchKernelGGL(k_fused<RL_METHOD_BL>, grid, block, 0, m->ctx->stream, m->dev(), m->ctx->trig,
                        max_range, ins, angles, obs, m->d_table, m->table_width, weights, N, M, S);
   else if (method == RL_METHOD_GLT)
@@ -1581,6 +1757,8 @@ int launch_particles_t(rl_map* m, float max_range, const float* ins, const float
     long long blocks = RL_REGIONS * ((N + per_block - 1) / per_block);
     hipLaunchKernelGGL((k_particles_xcd<METHOD, SENSOR>), dim3((unsigned)blocks), dim3(256), 0, c->stream,
                        m->dev(), c->trig, max_range, ins, angles, obs, table, K, ranges, weights, M, S, sc);
+  } else if (METHOD == RL_METHOD_RM && pool_pays(m, (long long)N * M, M)) {
+    launch_pool<SENSOR ? POOL_STEP : POOL_RANGES>(m, max_range, ins, angles, obs, ranges, weights, N, M);
   } else {
     long long waves = ((long long)N + 64 / S - 1) / (64 / S);
     hipLaunchKernelGGL((k_particles<METHOD, SENSOR>), dim3(grid_for(waves * 64, 256)), dim3(256), 0,
@@ -1926,6 +2104,7 @@ int rl_create(int device, rl_ctx** out) {
       const float st = lut[i] * 0.999f;
       lut[RL_LUT_SIZE + i] = (st < 1.0f) ? 1.0f : st;
     }
+    lut[RL_LUT_SIZE] = INFINITY;  // code 0 ends a march
     if (hipMalloc(&c->d_lut, sizeof(lut)) != hipSuccess ||
         hipMemcpy(c->d_lut, lut, sizeof(lut), hipMemcpyHostToDevice) != hipSuccess) {
       (void)hipGetLastError();

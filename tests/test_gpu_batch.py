@@ -111,6 +111,24 @@ def test_batch_autotune_and_graph_capture():
     ctx.set_stream(None)
 
 
+@pytest.mark.parametrize("order,grid", [(0, 0), (1, 0), (1, 256), (2, 0), (2, 320)])
+def test_batch_pooled(order, grid):
+    """A batch with rays enough to be marched from pools: jobs with and without a
+    sensor model, one particle, more beams than a pool holds."""
+    ctx = rl.Context(0)
+    sizes = [(3000, 60, 500, True), (1, 600, 120, True), (1500, 107, 300, False), (77, 5, 500, True)]
+    specs = [{"kind": "corridor" if i % 2 else "rect_disk", "side": 300 + 77 * i, "map_seed": 60 + i, "particles": n,
+              "beams": m, "max_range": R, "sensor": s, "pose_seed": 70 + i} for i, (n, m, R, s) in enumerate(sizes)]
+    jobs, want, keep = _make_jobs(ctx, specs, 6)
+    b = rl.Batch(ctx)
+    b.set_jobs(jobs)
+    b.set_config(order=order, grid=grid)
+    for _ in range(2):
+        b.launch()
+        ctx.sync()
+        _check(keep, want)
+
+
 def test_batch_rejects_bad_jobs():
     ctx = rl.Context(0)
     b = rl.Batch(ctx)

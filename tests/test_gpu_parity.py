@@ -501,6 +501,47 @@ def test_pf_step_bit_exact(kind, m, corridor_map):
     assert np.array_equal(ww.cpu().numpy(), want_w)
 
 
+@pytest.mark.parametrize("n,m,R,world", [(n, m, R, None) for n, m, R in [(87_500, 3, 500.0), (4370, 60, 500.0), (20_011, 107, 120.0), (700, 512, 500.0),
+                                   (601, 513, 500.0), (253, 1100, 500.0), (4370, 60, 0.0), (4370, 60, 2e9)]] +
+                         [(4370, 61, 500.0, (0.5, 0.3, 1.5, -2.0, float(np.sin(0.3)), float(np.cos(0.3))))])
+def test_pooled_rays(n, m, R, world, rect_map):
+    """Launches whose waves march a pool of rays: edges of the particles and rays of
+    a wave, beams beyond a pool, origins and headings that are not marched, every
+    output, bit for bit."""
+    torch = _torch()
+    ctx = rl.default_context(0)
+    table = W.sensor_table(401)
+    ins = W.world_poses(rect_map, n, seed=41)
+    heads = np.array([np.nan, np.inf, 1e6, 2 * np.pi, -0.0], np.float32)
+    origins = np.array([[100.5, 200.25], [-0.5, 30.0], [30.0, -0.75], [0.0, 0.0], [511.9, 511.9], [512.0, 3.0],
+                        [np.nan, 5.0], [5.0, np.inf], [3e9, 40.0], [250.0, 250.0]], np.float32)
+    odd = np.array([[x, y, h] for x, y in origins for h in heads], np.float32)
+    ins[np.arange(len(odd)) * (n // len(odd))] = odd
+    ang = W.beam_angles(m)
+    orc = O.Oracle(rect_map, R, "rm", world=world) if world else O.Oracle(rect_map, R, "rm")
+    orc.set_sensor_model(table)
+    obs = W.noisy_observation(np.full(m, 60.0, np.float32), seed=42)
+    want_r = orc.numpy_calc_range_angles(ins, ang)
+    want_w = orc.eval_sensor_model(obs, want_r, m, n)
+    dm = rl.DeviceMap(ctx, O.xmajor(rect_map))
+    dm.set_sensor_table(table)
+    if world:
+        dm.set_world(*world)
+    d = {k: torch.from_numpy(v).cuda() for k, v in (("ins", ins), ("ang", ang), ("obs", obs))}
+    rr, r2 = (torch.full((n * m,), -1.0, dtype=torch.float32, device="cuda") for _ in range(2))
+    ww, w2 = (torch.full((n,), -1.0, dtype=torch.float64, device="cuda") for _ in range(2))
+    dm.pf_step_dev(rl.RL_METHOD_RM, R, d["ins"].data_ptr(), d["ang"].data_ptr(), d["obs"].data_ptr(), rr.data_ptr(),
+                   ww.data_ptr(), n, m)
+    dm.numpy_calc_range_angles_dev(rl.RL_METHOD_RM, R, d["ins"].data_ptr(), d["ang"].data_ptr(), r2.data_ptr(), n, m)
+    dm.repeat_angles_eval_sensor_model_dev(rl.RL_METHOD_RM, R, d["ins"].data_ptr(), d["ang"].data_ptr(),
+                                           d["obs"].data_ptr(), w2.data_ptr(), n, m)
+    ctx.sync()
+    assert_bits_equal(rr.cpu().numpy(), want_r, "step ranges")
+    assert_bits_equal(r2.cpu().numpy(), want_r, "ranges")
+    assert np.array_equal(ww.cpu().numpy(), want_w)
+    assert np.array_equal(w2.cpu().numpy(), orc.calc_range_repeat_angles_eval_sensor_model(ins, ang, obs))
+
+
 @pytest.mark.parametrize("xcd,box", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_scheduling_options(xcd, box, corridor_map):
     """XCD-aware scheduling and LDS staging change only where data is read from."""
