@@ -498,35 +498,35 @@ __global__ __launch_bounds__(256) void k_cast(MapDev m, TrigDev trig, float max_
 }
 
 // Regrouping, measured on 1 M Bresenham queries of a 2048^2 corridor map
-// (R = 1000): 256 threads with 1, 2, 4, 6 or 8 rounds between regroupings
-// 149, 134, 127, 129, 129 us; 128 or 512 threads (4 and 2 rounds) 133, 140 us;
-// one walk per lane to its end 133 us.  Each regrouping costs three barriers
-// and the parked state's LDS traffic, and waits for the workgroup's slowest wave.
+// (R = 1000; a walk takes 3.8 rounds in the mean, 5% more than 10): after 3, 5 and
+// then every 8 rounds 119.7 us; 3 and then 6 121.5; 4 and then 8 121.7; every 4
+// 123.6.  (With an earlier round: every 1, 2, 4, 6 or 8 rounds 149, 134, 127, 129,
+// 129 us; 128 or 512 threads 133, 140; one walk per lane to its end 133.)  Each
+// regrouping costs three barriers and the parked state's LDS traffic, and waits for
+// the workgroup's slowest wave; walks that are left late are long.  The rounds
+// bound the kernel (VALU): 44% of their lanes are in use.
 #ifndef RL_BL_WG
 #define RL_BL_WG 256  // threads of a k_cast_bl workgroup, whose walks are regrouped together
-#endif
-#ifndef RL_BL_PHASE
-#define RL_BL_PHASE 4  // rounds of every walk between regroupings (k_cast_bl)
 #endif
 #define RL_BL_PARK 18  // words of a parked walk: rl::BlWalk and its ray
 
 // A walk and its ray parked in slot i of LDS (one array per word, so that
 // consecutive slots are in consecutive banks).
 __device__ __forceinline__ void park_walk(unsigned (*park)[RL_BL_WG], int i, const rl::BlWalk& w, int ray) {
-  park[0][i] = __float_as_uint(w.x), park[1][i] = __float_as_uint(w.y), park[2][i] = __float_as_uint(w.err);
-  park[3][i] = __float_as_uint(w.deltax), park[4][i] = __float_as_uint(w.deltay);
+  park[0][i] = __float_as_uint(w.x), park[1][i] = __float_as_uint(w.y), park[2][i] = __float_as_uint(w.err2);
+  park[3][i] = __float_as_uint(w.deltax), park[4][i] = __float_as_uint(w.deltay2);
   park[5][i] = __float_as_uint(w.xstep), park[6][i] = __float_as_uint(w.ystep);
-  park[7][i] = __float_as_uint(w.limx), park[8][i] = w.limy;
+  park[7][i] = w.limx, park[8][i] = w.limy;
   park[9][i] = __float_as_uint(w.x0), park[10][i] = __float_as_uint(w.y0);
   park[11][i] = w.sx, park[12][i] = w.sy, park[13][i] = (unsigned)w.xend, park[14][i] = (unsigned)w.left;
   park[15][i] = w.bbase, park[16][i] = w.brow, park[17][i] = (unsigned)ray;
 }
 
 __device__ __forceinline__ void unpark_walk(const unsigned (*park)[RL_BL_WG], int i, rl::BlWalk* w, int* ray) {
-  w->x = __uint_as_float(park[0][i]), w->y = __uint_as_float(park[1][i]), w->err = __uint_as_float(park[2][i]);
-  w->deltax = __uint_as_float(park[3][i]), w->deltay = __uint_as_float(park[4][i]);
+  w->x = __uint_as_float(park[0][i]), w->y = __uint_as_float(park[1][i]), w->err2 = __uint_as_float(park[2][i]);
+  w->deltax = __uint_as_float(park[3][i]), w->deltay2 = __uint_as_float(park[4][i]);
   w->xstep = __uint_as_float(park[5][i]), w->ystep = __uint_as_float(park[6][i]);
-  w->limx = __uint_as_float(park[7][i]), w->limy = park[8][i];
+  w->limx = park[7][i], w->limy = park[8][i];
   w->x0 = __uint_as_float(park[9][i]), w->y0 = __uint_as_float(park[10][i]);
   w->sx = park[11][i], w->sy = park[12][i], w->xend = (int)park[13][i], w->left = (int)park[14][i];
   w->bbase = park[15][i], w->brow = park[16][i], *ray = (int)park[17][i];
@@ -534,7 +534,7 @@ __device__ __forceinline__ void unpark_walk(const unsigned (*park)[RL_BL_WG], in
 
 // Bresenham rays (BresenhamsLine::calc_range, RangeLib.h:696-769, one per
 // thread as numpy_calc_range / calc_range_many cast them) over the occupancy
-// bitmap, with the walks of a workgroup regrouped every RL_BL_PHASE rounds:
+// bitmap, with the walks of a workgroup regrouped after some rounds:
 // the walks still running move (through LDS) to the workgroup's first
 // threads, so they fill whole waves and the other waves stop issuing.  Walk
 // lengths vary widely (on corridor maps the longest is ~20x the mean), and
@@ -565,9 +565,10 @@ __global__ __launch_bounds__(RL_BL_WG) void k_cast_bl(MapDev m, TrigDev trig, fl
     live = rl::bl_begin(m, max_range, x, y, s, c, &w, &d);
     if (!live) outs[r] = (FRAME == 0) ? d : d * scale;  // ended before its loop
   }
-  for (;;) {  // ends when no walk of the workgroup is left (the same in every thread)
+  for (int phase = 0;; ++phase) {  // ends when no walk of the workgroup is left (the same in every thread)
+    const int rounds = phase == 0 ? 3 : phase == 1 ? 5 : 8;
 #pragma unroll 1
-    for (int j = 0; j < RL_BL_PHASE; ++j) {
+    for (int j = 0; j < rounds; ++j) {
       if (live) {
         bool hit;
         int unused = 0;

@@ -351,6 +351,31 @@ def test_bresenham_far_origins(ctx, rect_map):
         assert_bits_equal(out, O.Oracle(rect_map, R, "bl").calc_range_many(q), f"R={R}")
 
 
+@pytest.mark.parametrize("R", [1e-40, 0.25, 5.0, 60.0])
+def test_bresenham_signs_and_edges(ctx, R):
+    """Walks from zeros of both signs, the least floats about them, and the map's
+    four edges, on a map that is no whole number of tiles: ranges and step counts
+    equal the oracle's."""
+    torch = _torch()
+    img = (np.random.default_rng(8).random((33, 43)) < 0.04).astype(np.uint8)
+    img[:3, :3] = 0
+    tiny = np.float32(1e-45)
+    xs = np.array([0.0, -0.0, tiny, -tiny, -0.5, 0.5, 7.0, 42.0, 42.75, 43.0, -1.0], np.float32)
+    ys = np.array([0.0, -0.0, tiny, -tiny, -0.5, 0.5, 8.0, 32.0, 32.75, 33.0, -1.0], np.float32)
+    heads = np.concatenate([np.arange(16) * (np.pi / 8), [-0.0, 0.01, np.pi / 4]]).astype(np.float32)
+    q = np.array([[x, y, h] for x in xs for y in ys for h in heads], np.float32)
+    n = q.shape[0]
+    m = rl.DeviceMap(ctx, O.xmajor(img))
+    out = np.empty(n, np.float32)
+    m.calc_range_many(rl.RL_METHOD_BL, R, q, out, n)
+    want, want_cnt = O.Oracle(img, R, "bl").calc_range_many(q, counts=True)
+    assert_bits_equal(out, want, f"R={R}")
+    d_q, cnt = torch.from_numpy(q).cuda(), torch.zeros(n, dtype=torch.int32, device="cuda")
+    m.count_steps_dev(rl.RL_METHOD_BL, rl.RL_FRAME_GRID, R, d_q.data_ptr(), 0, cnt.data_ptr(), n, 1)
+    ctx.sync()
+    assert np.array_equal(cnt.cpu().numpy(), want_cnt)
+
+
 def test_bresenham_rounding_steps(ctx):
     """Bresenham walks whose unit steps round: fractional origins just below a
     power of two (32 ... 512) on the walking axis, within a few units in the
