@@ -418,7 +418,7 @@ def bench_uneven64(args):
         "speedup_vs_per_map": per_map_ms / batch_ms, "autotuned": batch.config(), "autotune_best_ms": tuned_ms,
         "rays": total_rays, "maps": len(jobs), "setup_s": setup_s, "steps": args.steps,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "k_batch<RM>",
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "k_batch<RM>" if batch.config()["lds_box"] else "k_batch_pool",
                      "kernel_ms": batch_ms, "alg_bytes_per_launch": alg, "edt_reads_per_ray": reads / total_rays,
                      "max_reads_per_ray": max_reads},
         "config": {"workload": "uneven64_side256-4096_p500-8000_b30-120_r500"}}
