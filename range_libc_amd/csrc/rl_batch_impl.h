@@ -6,7 +6,8 @@
 // chunk is the particles one 256-thread workgroup casts together (4 waves x
 // 64 / S particles, S = lanes per particle).  k_batch runs a fixed grid whose
 // workgroups stride over the list, so long items placed first (order 1:
-// estimated cost, descending) finish while later short items fill the gaps.
+// estimated cost, descending; in pooled batches only the short ones last) finish
+// while later short items fill the gaps.
 //
 // Tuned per batch by rl_batch_autotune: lanes per particle S (16, 32 or 64,
 // never above the beam count's power of two), LDS staging of the 64x64 cells
@@ -168,8 +169,17 @@ int batch_upload(rl_batch* b) {
       items.push_back({cnt * ray_cost, BatchItem{i, f}});
     }
   }
-  auto by_cost = [](const std::pair<double, BatchItem>& a, const std::pair<double, BatchItem>& z) {
-    return a.first > z.first;
+  // Pooled items are of nearly equal rays, and short beside the launch: what matters
+  // is only that small remainders come last, so costs within a factor of eight of the
+  // largest count as equal and keep the jobs' order.  Sorted by cost, the maps with
+  // the most reads per ray run side by side and those bound by instructions after
+  // them (16 maps of up to 2048^2 258.9 against 235 us, the 64-map batch 0.960
+  // against 0.902 ms).
+  double most = 0.0;
+  for (const auto& it : items) most = std::max(most, it.first);
+  const double small = b->pooled ? most / 8.0 : HUGE_VAL;
+  auto by_cost = [small](const std::pair<double, BatchItem>& a, const std::pair<double, BatchItem>& z) {
+    return std::min(a.first, small) > std::min(z.first, small);
   };
   std::vector<BatchItem> flat;
   if (b->order == 2 && b->xcds > 1) {
