@@ -291,6 +291,18 @@ __device__ __forceinline__ bf16_t f2bf_hw(float v) {
   return v != v ? (bf16_t)0x7fc0 : r;
 }
 
+// Two floats rounded to bf16 (nearest even), v0 in the low half.
+__device__ __forceinline__ unsigned sg_pack2(float v0, float v1) {
+  return (unsigned)__builtin_bit_cast(bf16_t, (__bf16)v0) | ((unsigned)__builtin_bit_cast(bf16_t, (__bf16)v1) << 16);
+}
+
+// A hidden layer's relu, on the sum in fp32: v_maximum3_f32, which keeps NaNs of
+// either sign (biases have them, and the matrix instructions give them: a NaN times a
+// negative weight).
+__device__ __forceinline__ float sg_relu(float v) { return __builtin_elementwise_maximum(v, 0.0f); }
+
+// Conversions that differ from f2bf's, of the features (f2bf_hw) and of a layer's
+// outputs (sg_pack2 of sg_relu; but for a zero's sign and a NaN's).
 __global__ void k_sg_bf16_check(unsigned long long* __restrict__ bad) {
   unsigned long long local = 0;
   const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
@@ -298,21 +310,11 @@ __global__ void k_sg_bf16_check(unsigned long long* __restrict__ bad) {
        u += stride) {
     const float f = __uint_as_float((unsigned)u);
     local += f2bf_hw(f) != f2bf(f) ? 1u : 0u;
+    const unsigned two = sg_pack2(sg_relu(f), sg_relu(f));
+    const bool same = f != f ? bf2f((bf16_t)two) != bf2f((bf16_t)two) : (two & 0xffffu) == f2bf(f <= 0.0f ? 0.0f : f);
+    local += same && two >> 16 == (two & 0xffffu) ? 0u : 1u;
   }
   if (local) atomicAdd(bad, local);
-}
-
-// Two floats rounded to bf16 (nearest even), v0 in the low half.
-__device__ __forceinline__ unsigned sg_pack2(float v0, float v1) {
-  return (unsigned)__builtin_bit_cast(bf16_t, (__bf16)v0) | ((unsigned)__builtin_bit_cast(bf16_t, (__bf16)v1) << 16);
-}
-
-// relu of two bf16: negative values have their sign bit set, so the signed
-// 16-bit maximum with 0 is relu (a NaN of the matrix instructions is positive
-// and stays).
-__device__ __forceinline__ unsigned sg_relu2(unsigned v) {
-  typedef short s2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(s2, v), s2{0, 0}));
 }
 
 // One hidden layer: act (64 x K) -> act (64 x 256), wave w computing columns
@@ -360,8 +362,8 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
 #pragma unroll
     for (int i = 0; i < RT; ++i)
       *(uint2*)(act + (i * 16 + r16) * RL_SG_ACT_PAD + c) =
-          make_uint2(sg_relu2(sg_pack2(acc[i][j][0] + bb[0], acc[i][j][1] + bb[1])),
-                     sg_relu2(sg_pack2(acc[i][j][2] + bb[2], acc[i][j][3] + bb[3])));
+          make_uint2(sg_pack2(sg_relu(acc[i][j][0] + bb[0]), sg_relu(acc[i][j][1] + bb[1])),
+                     sg_pack2(sg_relu(acc[i][j][2] + bb[2]), sg_relu(acc[i][j][3] + bb[3])));
   }
   __syncthreads();
 }

@@ -411,3 +411,34 @@ def test_gradient_row_cuts_vs_cpu(ctx, n):
     for w, b, o, i in S.LAYERS:
         for sl in (slice(w, w + o * i), slice(b, b + o)):
             assert _rel(grad[sl], g16[sl]) <= 1e-2 and _cos(grad[sl], g16[sl]) >= 0.9999
+
+
+@pytest.mark.parametrize("layer", [0, 1, 2])
+@pytest.mark.parametrize("what,bits", [("bias", 0xffc00000), ("bias", 0x7fc00000), ("bias", 0xff800001), ("bias", 0xff800000),
+                                       ("bias", 0x7f800000), ("weight", 0xffc00000), ("weight", 0xff800000)])
+def test_fused_forward_of_nan_and_infinite_parameters(ctx, layer, what, bits):
+    """NaNs of both signs and infinities among a hidden layer's parameters: the fused
+    forward is NaN exactly where the per-layer one is, and the checked cast of a
+    network that says NaN is the exact march."""
+    R, n = 100.0, 100
+    img, g, rays = _map_and_rays(n, seed=5)
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    sg = rl.Surrogate(dm, seed=9)
+    p = sg.params()[0].copy()
+    w, b, o, i = S.LAYERS[layer]
+    p.view(np.uint32)[b + 3 if what == "bias" else w + 3 * i + 5] = bits
+    sg.set_params(p)
+    with np.errstate(invalid="ignore"):
+        fused, layers = sg.forward(rays), sg.forward_layers(rays)
+    assert np.array_equal(np.isnan(fused), np.isnan(layers))
+    finite = ~np.isnan(layers)
+    assert_bits_equal(fused[finite], layers[finite], "fused vs per-layer forward")
+    if np.isnan(p).any():
+        assert np.isnan(fused).all()
+        torch = _torch()
+        ins, ang = torch.from_numpy(W.world_poses(img, n, seed=2)).cuda(), torch.from_numpy(W.beam_angles(7)).cuda()
+        got, want = (torch.zeros(7 * n, dtype=torch.float32, device="cuda") for _ in range(2))
+        sg.calc_range_angles_dev(R, ins.data_ptr(), ang.data_ptr(), got.data_ptr(), n, 7, bound_max=1e9)
+        dm.numpy_calc_range_angles_dev(rl.RL_METHOD_RM, R, ins.data_ptr(), ang.data_ptr(), want.data_ptr(), n, 7)
+        ctx.sync()
+        assert_bits_equal(got.cpu().numpy(), want.cpu().numpy(), "checked cast")
