@@ -297,9 +297,10 @@ RL_HD void sincosf_libc_bm(float h, const Bitmap& bs, const Bitmap& bc, float* s
 }
 
 // Host-side helpers (plain host functions under hipcc).
-// Smallest exponent field among the listed inputs of a bucketed table (RLT_EXP_MAX + 1 if none).
+// Smallest exponent field among the listed inputs of a bucketed table, RLT_EXP_MAX if
+// there are none: the device reads a byte of the bitmap for every input.
 static inline int table_min_exponent(const uint32_t* off, const uint16_t* keys) {
-  int e_min = RLT_EXP_MAX + 1;
+  int e_min = RLT_EXP_MAX;
   for (uint32_t b = 0; b < RLT_NBUCKETS; ++b)
     for (uint32_t i = off[b]; i < off[b + 1]; ++i) {
       uint32_t ab = ((b & ((1u << RLT_SIGN_SHIFT) - 1u)) << RLT_BUCKET_SHIFT) | keys[i];

@@ -18,7 +18,7 @@ import pytest
 
 from oracle import oracle as O
 from range_libc_amd import workloads as W
-from tests.conftest import GOLDEN, assert_bits_equal
+from tests.conftest import GOLDEN, ROOT, assert_bits_equal
 
 FLT_MAX = np.finfo(np.float32).max
 
@@ -335,6 +335,17 @@ def test_trig_table_exhaustive_vs_libc():
     p = subprocess.run([exe, "--verify", table], capture_output=True, text=True, timeout=300)
     assert p.returncode == 0, p.stdout + p.stderr
     assert " 0 mismatches" in p.stdout
+
+
+def test_trig_bitmap_of_few_exceptions(tmp_path):
+    """The device's lookup of exceptions stays in its bitmap for any table, that of a
+    C library without exceptions among them."""
+    exe = str(tmp_path / "trig_bitmap")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-Wno-unknown-pragmas", "-I",
+                    os.path.join(ROOT, "range_libc_amd", "csrc"), os.path.join(ROOT, "tests", "cpp", "trig_bitmap.cpp"),
+                    "-o", exe], check=True, capture_output=True, text=True)
+    p = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert p.returncode == 0, p.stdout + p.stderr
 
 
 # --------------------------------------------------------------------------- live vs the compiled reference
