@@ -1050,8 +1050,8 @@ __global__ __launch_bounds__(256) void k_particles_xcd(MapDev m, TrigDev trig, f
 // +infinity where a march ends (an occupied cell, or off the map).
 __global__ __launch_bounds__(256) void k_glt_steps(const float* __restrict__ edt, int W, int H,
                                                    float* __restrict__ steps) {
-  const int x = (int)blockIdx.y;
-  const int y = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int x = (int)blockIdx.x;  // W + 1 of them: a grid's y has fewer
+  const int y = (int)(blockIdx.y * blockDim.x + threadIdx.x);
   if (y > H) return;
   float g = INFINITY;
   if (x < W && y < H) {
@@ -1094,49 +1094,48 @@ __global__ __launch_bounds__(256) void k_glt_build_tiles(const float* __restrict
       (void*)steps, (short)0, (int)((unsigned)(W + 1) * pitch), 0x00020000);
   const int lane = threadIdx.x & 63, c = lane & (RL_GLT_TILE - 1);
   uint16_t* tile = tiles + (threadIdx.x >> 6) * (RL_GLT_TILE * td);
-  const unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6);  // tiles x-major; fewer than 2^27 (steps below 4 GiB)
-  if (t >= ntx * nty) return;  // the same in every lane of the wave; no workgroup barrier below
-  const int x0 = (int)(t / nty) * 4, y0 = (int)(t - (t / nty) * nty) * 4;
-  const int x = x0 + (c >> 2), y = y0 + (c & 3);
-  if (x < W && y < H) {
-    const float fx = (float)x, fy = (float)y;
-    // the first read is at the cell itself, whatever the direction
-    const float g0 = steps[(size_t)x * (unsigned)(H + 1) + y];
-    for (int bin = lane / RL_GLT_TILE; bin < td; bin += 64 / RL_GLT_TILE) {
-      const float2 d = dirs[bin];
-      float s = g0, tc = 0.0f, tn = g0;  // the last step read, its position and the next
-      unsigned px = (unsigned)x, py = (unsigned)y;
-      while (tn < max_range) {
-        tc = tn;
-        px = min((unsigned)(int)(fx + d.x * tc), (unsigned)W);
-        py = min((unsigned)(int)(fy + d.y * tc), (unsigned)H);
-        s = __builtin_bit_cast(float,
-                               __builtin_amdgcn_raw_buffer_load_b32(rsrc, __umul24(px, pitch) + (py << 2), 0, 0));
-        tn = tc + s;
+  // tiles x-major, fewer than 2^27 (steps below 4 GiB); a wave's loop has no workgroup barrier
+  for (unsigned t = blockIdx.x * 4u + (threadIdx.x >> 6); t < ntx * nty; t += gridDim.x * 4u) {
+    const int x0 = (int)(t / nty) * 4, y0 = (int)(t - (t / nty) * nty) * 4;
+    const int x = x0 + (c >> 2), y = y0 + (c & 3);
+    if (x < W && y < H) {
+      const float fx = (float)x, fy = (float)y;
+      // the first read is at the cell itself, whatever the direction
+      const float g0 = steps[(size_t)x * (unsigned)(H + 1) + y];
+      for (int bin = lane / RL_GLT_TILE; bin < td; bin += 64 / RL_GLT_TILE) {
+        const float2 d = dirs[bin];
+        float s = g0, tc = 0.0f, tn = g0;  // the last step read, its position and the next
+        unsigned px = (unsigned)x, py = (unsigned)y;
+        while (tn < max_range) {
+          tc = tn;
+          px = min((unsigned)(int)(fx + d.x * tc), (unsigned)W);
+          py = min((unsigned)(int)(fy + d.y * tc), (unsigned)H);
+          s = __builtin_bit_cast(float,
+                                 __builtin_amdgcn_raw_buffer_load_b32(rsrc, __umul24(px, pitch) + (py << 2), 0, 0));
+          tn = tc + s;
+        }
+        float v = max_range;
+        if (s == INFINITY && px < (unsigned)W && py < (unsigned)H) {
+          const float xd = (float)(int)px - fx;
+          const float yd = (float)(int)py - fy;
+          v = __builtin_sqrtf(xd * xd + yd * yd);
+        }
+        v = (v < max_range) ? v : max_range;  // std::min(max_range, r)
+        tile[c * td + bin] = (uint16_t)(unsigned)(v * limits_div_max);
       }
-      float v = max_range;
-      if (s == INFINITY && px < (unsigned)W && py < (unsigned)H) {
-        const float xd = (float)(int)px - fx;
-        const float yd = (float)(int)py - fy;
-        v = __builtin_sqrtf(xd * xd + yd * yd);
+    }
+    wave_lds_sync();  // the wave reads what its other lanes wrote
+    const int n = min(4, H - y0) * td;  // entries of a row of cells
+    for (int u = 0; u < 4 && x0 + u < W; ++u) {
+      uint16_t* dst = out + ((size_t)(x0 + u) * (unsigned)H + (unsigned)y0) * (unsigned)td;
+      const uint16_t* src = tile + u * 4 * td;  // 8 td bytes each
+      if ((((uintptr_t)dst | (unsigned)(2 * n)) & 7) == 0) {
+        for (int e = lane; e < n / 4; e += 64) ((uint2*)dst)[e] = ((const uint2*)src)[e];
+      } else {
+        for (int e = lane; e < n; e += 64) dst[e] = src[e];
       }
-      v = (v < max_range) ? v : max_range;  // std::min(max_range, r)
-      tile[c * td + bin] = (uint16_t)(unsigned)(v * limits_div_max);
     }
-  }
-  // the wave reads what its other lanes wrote
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int n = min(4, H - y0) * td;  // entries of a row of cells
-  for (int u = 0; u < 4 && x0 + u < W; ++u) {
-    uint16_t* dst = out + ((size_t)(x0 + u) * (unsigned)H + (unsigned)y0) * (unsigned)td;
-    const uint16_t* src = tile + u * 4 * td;  // 8 td bytes each
-    if ((((uintptr_t)dst | (unsigned)(2 * n)) & 7) == 0) {
-      for (int e = lane; e < n / 4; e += 64) ((uint2*)dst)[e] = ((const uint2*)src)[e];
-    } else {
-      for (int e = lane; e < n; e += 64) dst[e] = src[e];
-    }
+    wave_lds_sync();  // the tile was read before the next one is written
   }
 }
 
@@ -2234,10 +2233,11 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
     hipLaunchKernelGGL(k_glt_dirs, dim3((unsigned)((theta_disc + 255) / 256)), dim3(256), 0, c->stream, c->trig,
                        theta_disc, step, dirs);
     if (steps) {
-      hipLaunchKernelGGL(k_glt_steps, dim3((unsigned)grid_for(m->height + 1, 256), (unsigned)(m->width + 1)), dim3(256),
+      hipLaunchKernelGGL(k_glt_steps, dim3((unsigned)(m->width + 1), (unsigned)grid_for(m->height + 1, 256)), dim3(256),
                          0, c->stream, (const float*)m->d_edt, m->width, m->height, steps);
       const unsigned ntx = (unsigned)(m->width + 3) / 4, nty = (unsigned)(m->height + 3) / 4;
-      hipLaunchKernelGGL(k_glt_build_tiles, dim3((ntx * nty + 3) / 4), dim3(256),
+      // (a grid's threads stay below 2^32: up to 2^20 workgroups, their waves striding)
+      hipLaunchKernelGGL(k_glt_build_tiles, dim3(std::min((ntx * nty + 3) / 4, 1u << 20)), dim3(256),
                          (unsigned)(4 * RL_GLT_TILE * theta_disc * sizeof(uint16_t)), c->stream, (const float*)steps,
                          m->width, m->height, max_range, theta_disc, (const float2*)dirs, limits_div_max, m->d_glt, ntx,
                          nty);

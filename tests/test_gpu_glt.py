@@ -182,3 +182,22 @@ def test_glt_tiles_ragged(ctx, w, h, td, R):
     got, _, _, _ = dm.giant_lut()
     want = O.Oracle(img, R, "glt", theta_disc=td).glt
     assert np.array_equal(got, want.reshape(got.shape))
+
+
+def test_glt_largest_step_map(ctx):
+    """A map whose steps just fit their 4 GiB, with more 4 x 4 tiles than a launch has
+    waves and the most columns: one heading along x, every distance 1.5 but at some
+    walls."""
+    w, h, R = 65535, 16382, 3.0
+    edt = np.full((w, h), 1.5, np.float32)
+    walls = [(2, 0), (300, 16381), (32768, 8191), (65532, 3), (65534, 0), (65534, 16381)]
+    for x, y in walls:
+        edt[x, y] = 0.0
+    dm = rl.DeviceMap(ctx, np.zeros((w, h), np.uint8), edt_xmajor=edt)
+    del edt
+    dm.build_giant_lut(R, 1)
+    table = dm.giant_lut()[0].reshape(w, h)
+    want = {(x - d, y): np.uint16(np.float32(d) * (np.float32(65535) / np.float32(R))) for x, y in walls for d in range(3)}
+    assert np.count_nonzero(table != 65535) == len(want)
+    for at, v in want.items():
+        assert table[at] == v, at
