@@ -223,24 +223,24 @@ __global__ __launch_bounds__(256) void k_cddt_compact(long long nb, const long l
                                                       const float* __restrict__ vals, const uint8_t* __restrict__ used,
                                                       int mode, const long long* __restrict__ new_start,
                                                       long long* __restrict__ kept, float* __restrict__ out) {
-  const long long b = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  if (b >= nb) return;
-  const long long s = start[b], e = start[b + 1];
-  long long o = COPY ? new_start[b] : 0;
-  for (long long j0 = s; j0 < e; j0 += 64) {
-    const long long j = j0 + lane;
-    bool keep = false;
-    float v = 0.0f;
-    if (j < e) {
-      v = vals[j];
-      keep = mode == 0 ? (j == s || v != vals[j - 1]) : used[j] != 0;
+  for (long long b = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); b < nb; b += (long long)gridDim.x * 4) {
+    const long long s = start[b], e = start[b + 1];
+    long long o = COPY ? new_start[b] : 0;
+    for (long long j0 = s; j0 < e; j0 += 64) {
+      const long long j = j0 + lane;
+      bool keep = false;
+      float v = 0.0f;
+      if (j < e) {
+        v = vals[j];
+        keep = mode == 0 ? (j == s || v != vals[j - 1]) : used[j] != 0;
+      }
+      const unsigned long long m = __ballot(keep);
+      if (COPY && keep) out[o + __popcll(m & ((1ull << lane) - 1ull))] = v;
+      o += __popcll(m);
     }
-    const unsigned long long m = __ballot(keep);
-    if (COPY && keep) out[o + __popcll(m & ((1ull << lane) - 1ull))] = v;
-    o += __popcll(m);
+    if (!COPY && lane == 0) kept[b] = o;
   }
-  if (!COPY && lane == 0) kept[b] = o;
 }
 
 // 5. Prune marks (RangeLib.h:1172-1275).  In the reference every free cell looks
@@ -479,6 +479,10 @@ int cddt_read(rl_map* m, const long long* d, long long* out) {
   return RL_OK;
 }
 
+// One wave per bin, striding from 2^20 workgroups on (a grid's threads stay below
+// 2^32; 65536 headings of a 1200^2 map have 10^8 bins).
+dim3 cddt_compact_grid(long long nb) { return dim3((unsigned)std::min<long long>((nb + 3) / 4, 1 << 20)); }
+
 // Keeps the entries selected by `mode` (see k_cddt_compact): new start and
 // values.  kept: the bins' numbers of entries to keep (nb + 1, the last 0).
 int cddt_compact(rl_map* m, int mode, const uint8_t* used, const DevBuf& kept) {
@@ -492,7 +496,7 @@ int cddt_compact(rl_map* m, int mode, const uint8_t* used, const DevBuf& kept) {
   long long total = 0;
   TRY(cddt_read(m, nstart.as<long long>() + nb, &total));
   TRY(nvals.alloc((size_t)total * sizeof(float)));
-  hipLaunchKernelGGL(k_cddt_compact<true>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
+  hipLaunchKernelGGL(k_cddt_compact<true>, cddt_compact_grid(nb), dim3(256), 0, st, nb,
                      (const long long*)m->cddt_start, (const float*)m->cddt_vals, used, mode, (const long long*)nstart.p,
                      (long long*)nullptr, nvals.as<float>());
   HIP_TRY(hipGetLastError());
@@ -607,7 +611,7 @@ int cddt_build_locked(rl_map* m, int td) {
   m->cddt_nv = total;
   // drop duplicates
   TRY(cddt_counts(m, &kept));
-  hipLaunchKernelGGL(k_cddt_compact<false>, dim3((unsigned)grid_for(nb, 4)), dim3(256), 0, st, nb,
+  hipLaunchKernelGGL(k_cddt_compact<false>, cddt_compact_grid(nb), dim3(256), 0, st, nb,
                      (const long long*)m->cddt_start, (const float*)m->cddt_vals, (const uint8_t*)nullptr, 0,
                      (const long long*)nullptr, kept.as<long long>(), (float*)nullptr);
   HIP_TRY(hipGetLastError());

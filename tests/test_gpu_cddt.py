@@ -230,3 +230,15 @@ def test_cddt_tables_equal_oracle(ctx, name, td):
         assert np.array_equal(got["widths"], want["widths"])
         assert np.array_equal(got["start"], want["start"]), "pruned" if prune else "full"
         assert_bits_equal(got["vals"], want["vals"], "pruned" if prune else "full")
+
+
+def test_cddt_bins_beyond_a_grid(ctx):
+    """As many headings as are accepted, on a map with more bins than a launch of one
+    wave each may have (2^26), all empty: every range is max_range."""
+    dm = rl.DeviceMap(ctx, np.zeros((1200, 1100), np.uint8))
+    dm.build_cddt(65536)
+    dm.prune_cddt(50.0)
+    q = W.grid_poses(np.zeros((1100, 1200), np.uint8), 500, seed=3)
+    out = np.zeros(500, np.float32)
+    dm.calc_range_many(rl.RL_METHOD_CDDT, 50.0, q, out, 500)
+    assert_bits_equal(out, np.full(500, 50.0, np.float32), "empty tables")
