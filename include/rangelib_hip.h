@@ -103,6 +103,12 @@ int rl_sync(rl_ctx* ctx);
  * CMakeLists.txt:13-14). */
 #define RL_OPT_XCD_SCHED 1          /* 1: bucket particles by map region per XCD (default 0) */
 #define RL_OPT_LDS_BOX 2            /* 1: stage 64x64 cells around a particle in LDS (default 0) */
+/* Bytes of device memory of destroyed maps and of table builds that the context
+ * keeps for the next ones (default 512 MiB).  Setting it gives back what is kept
+ * beyond it at once: 0 keeps nothing.  The context's own allocations take kept
+ * memory back by themselves when the device has no other; those of other
+ * libraries cannot. */
+#define RL_OPT_IDLE_BYTES 3
 int rl_set_option(rl_ctx* ctx, int option, long long value);
 
 /* --- maps ----------------------------------------------------------------- */

@@ -25,6 +25,7 @@ RL_MAP_EDT_ENVELOPE_ONLY = 1
 RL_MAP_NO_COMPACT = 2
 RL_OPT_XCD_SCHED = 1
 RL_OPT_LDS_BOX = 2
+RL_OPT_IDLE_BYTES = 3
 
 _vp = C.c_void_p
 _fp = C.POINTER(C.c_float)

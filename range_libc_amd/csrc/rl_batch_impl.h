@@ -223,7 +223,7 @@ int batch_upload(rl_batch* b) {
   if (b->cap_maps < maps.size()) {
     if (b->d_maps) HIP_TRY(hipFree(b->d_maps));
     b->d_maps = nullptr;
-    if (hipMalloc(&b->d_maps, maps.size() * sizeof(BatchMap)) != hipSuccess) {
+    if (c->pool.alloc_plain(&b->d_maps, maps.size() * sizeof(BatchMap)) != hipSuccess) {
       (void)hipGetLastError();
       b->cap_maps = 0;
       return fail(RL_ERR_NOMEM, "batch descriptor allocation failed");
@@ -233,7 +233,7 @@ int batch_upload(rl_batch* b) {
   if (b->cap_items < flat.size()) {
     if (b->d_items) HIP_TRY(hipFree(b->d_items));
     b->d_items = nullptr;
-    if (hipMalloc(&b->d_items, flat.size() * sizeof(BatchItem)) != hipSuccess) {
+    if (c->pool.alloc_plain(&b->d_items, flat.size() * sizeof(BatchItem)) != hipSuccess) {
       (void)hipGetLastError();
       b->cap_items = 0;
       return fail(RL_ERR_NOMEM, "batch work-list allocation failed");

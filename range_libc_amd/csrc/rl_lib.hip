@@ -1401,12 +1401,14 @@ int segment_size(int m) {
 // are let go: hipFree of a block above 16 MB takes 0.22 ms and up (0.9 ms seen
 // for the next hipMalloc after it), and replacing a 2048^2 map spent 0.6 of its
 // 1.04 ms there.  Blocks below RL_POOL_MIN go to the allocator directly (under a
-// microsecond).  At most RL_POOL_BYTES are kept idle, and given back with the
-// context.  A block that other streams may still be reading (a map's buffers:
-// their addresses are handed out) is reused only after the device was waited
-// for, as hipFree would have.
+// microsecond).  At most `limit` bytes (RL_OPT_IDLE_BYTES) are kept idle.  They are
+// given back with the context, when the limit is lowered, and when any allocation of
+// the context runs out of memory.  A block that other streams may still be reading (a
+// map's buffers: their addresses are handed out) is reused only after the device was
+// waited for, as hipFree would have.  No exception leaves it: a block that cannot be
+// recorded is not kept.
 #define RL_POOL_MIN (1u << 20)
-#define RL_POOL_BYTES (512u << 20)  // the buffers of a CDDT build of a 2048^2 map are 0.4 GB
+#define RL_POOL_BYTES (512u << 20)  // the default limit; the buffers of a CDDT build of a 2048^2 map are 0.4 GB
 struct DevPool {
   struct Block {
     void* p;
@@ -1414,14 +1416,33 @@ struct DevPool {
     bool idle;  // no work uses it any more
   };
   std::mutex mu;
-  std::vector<Block> kept;
+  std::vector<Block> kept;  // oldest first
   std::unordered_map<void*, size_t> live;  // capacities of the blocks handed out
-  size_t held = 0;
+  size_t held = 0, limit = RL_POOL_BYTES;
+
+  // A block from the allocator; out of memory with blocks kept, these are given back first.
+  hipError_t fresh(void** out, size_t bytes) {  // mu held
+    const hipError_t e = hipMalloc(out, bytes);
+    if (e != hipErrorOutOfMemory || kept.empty()) return e;
+    (void)hipGetLastError();
+    trim(0);
+    return hipMalloc(out, bytes);
+  }
+
+  // hipMalloc / hipFree, for buffers that live as long as their owner.
+  template <class T>
+  hipError_t alloc_plain(T** out, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu);
+    void* p = nullptr;
+    const hipError_t e = fresh(&p, bytes);
+    *out = e == hipSuccess ? (T*)p : nullptr;
+    return e;
+  }
 
   template <class T>
   hipError_t alloc(T** out, size_t bytes) {
+    if (bytes < RL_POOL_MIN) return alloc_plain(out, bytes ? bytes : 16);
     *out = nullptr;
-    if (bytes < RL_POOL_MIN) return hipMalloc((void**)out, bytes ? bytes : 16);
     const size_t cap = (bytes + (2u << 20) - 1) & ~(size_t)((2u << 20) - 1);
     std::lock_guard<std::mutex> lk(mu);
     size_t best = kept.size();
@@ -1438,19 +1459,14 @@ struct DevPool {
       const Block b = kept[best];
       kept.erase(kept.begin() + (long)best);
       held -= b.cap;
-      live[b.p] = b.cap;
+      record(b.p, b.cap);
       *out = (T*)b.p;
       return hipSuccess;
     }
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, cap);
-    if (e != hipSuccess && !kept.empty()) {  // out of memory with blocks kept: give them back first
-      (void)hipGetLastError();
-      drop();
-      e = hipMalloc(&p, cap);
-    }
+    const hipError_t e = fresh(&p, cap);
     if (e != hipSuccess) return e;
-    live[p] = cap;
+    record(p, cap);
     *out = (T*)p;
     return hipSuccess;
   }
@@ -1463,19 +1479,43 @@ struct DevPool {
     if (it != live.end()) {
       const size_t cap = it->second;
       live.erase(it);
-      if (held + cap <= RL_POOL_BYTES) {
-        kept.push_back(Block{p, cap, idle});
-        held += cap;
-        return;
-      }
+      if (held + cap <= limit && keep(Block{p, cap, idle})) return;
     }
     (void)hipFree(p);
   }
 
-  void drop() {  // mu held, or the last user
-    for (const Block& b : kept) (void)hipFree(b.p);
-    kept.clear();
-    held = 0;
+  void set_limit(size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu);
+    limit = bytes;
+    trim(limit);
+  }
+
+  // Gives blocks back, oldest first, until at most `bytes` are kept.
+  void trim(size_t bytes) {  // mu held, or the last user
+    size_t n = 0;
+    for (; n < kept.size() && held > bytes; ++n) {
+      (void)hipFree(kept[n].p);
+      held -= kept[n].cap;
+    }
+    kept.erase(kept.begin(), kept.begin() + (long)n);
+  }
+
+ private:
+  void record(void* p, size_t cap) {
+    try {
+      live[p] = cap;
+    } catch (const std::bad_alloc&) {  // release() will free it
+    }
+  }
+
+  bool keep(const Block& b) {
+    try {
+      kept.push_back(b);
+    } catch (const std::bad_alloc&) {
+      return false;
+    }
+    held += b.cap;
+    return true;
   }
 };
 
@@ -1521,7 +1561,7 @@ struct rl_ctx {
       stage[slot] = nullptr;
       stage_cap[slot] = 0;
       size_t cap = bytes + bytes / 4;
-      if (hipMalloc(&stage[slot], cap) != hipSuccess) {
+      if (pool.alloc_plain(&stage[slot], cap) != hipSuccess) {
         (void)hipGetLastError();
         return fail(RL_ERR_NOMEM, "hipMalloc of %zu staging bytes failed", cap);
       }
@@ -1731,9 +1771,8 @@ int ensure_sched(rl_map* m, int n) {
   m->d_sched = nullptr;
   m->sched_cap = 0;
   size_t cap = (size_t)n + (size_t)n / 4 + 64;
-  if (hipMalloc(&m->d_sched, (cap + 4 * RL_REGIONS) * sizeof(int)) != hipSuccess) {
+  if (m->ctx->pool.alloc_plain(&m->d_sched, (cap + 4 * RL_REGIONS) * sizeof(int)) != hipSuccess) {
     (void)hipGetLastError();
-    m->d_sched = nullptr;
     return fail(RL_ERR_NOMEM, "hipMalloc of the scheduling buffer failed (inside graph capture, "
                               "make one uncaptured call of this size first)");
   }
@@ -2122,7 +2161,7 @@ int rl_destroy(rl_ctx* c) {
   if (c->refs.fetch_sub(1) != 1) return RL_OK;  // maps or batches still hold it
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  c->pool.drop();
+  c->pool.trim(0);
   for (int i = 0; i < 6; ++i)
     if (c->stage[i]) (void)hipFree(c->stage[i]);
   if (c->pin) (void)hipHostFree(c->pin);
@@ -2227,7 +2266,7 @@ int rl_map_build_giant_lut(rl_map* m, float max_range, int theta_disc) {
   if (theta_disc <= RL_GLT_TILE_TD && steps_bytes <= 0xFFFFFFFFull &&
       c->pool.alloc(&steps, steps_bytes) != hipSuccess)
     (void)hipGetLastError();  // no room: one entry per thread, without them
-  hipError_t e = hipMalloc(&dirs, (size_t)theta_disc * sizeof(float2));
+  hipError_t e = c->pool.alloc_plain(&dirs, (size_t)theta_disc * sizeof(float2));
   if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_glt_dirs, dim3((unsigned)((theta_disc + 255) / 256)), dim3(256), 0, c->stream, c->trig,
@@ -2356,9 +2395,8 @@ int rl_map_set_sensor_table(rl_map* m, const double* table, int k) {
     m->d_table = nullptr;
   }
   size_t bytes = (size_t)k * k * sizeof(double);
-  if (hipMalloc(&m->d_table, bytes) != hipSuccess) {
+  if (m->ctx->pool.alloc_plain(&m->d_table, bytes) != hipSuccess) {
     (void)hipGetLastError();
-    m->d_table = nullptr;
     return fail(RL_ERR_NOMEM, "hipMalloc of a %dx%d sensor table failed", k, k);
   }
   HIP_TRY(hipMemcpyAsync(m->d_table, table, bytes, hipMemcpyHostToDevice, m->ctx->stream));
@@ -2631,6 +2669,10 @@ int rl_set_option(rl_ctx* c, int option, long long value) {
     c->xcd_sched = value != 0;
   } else if (option == RL_OPT_LDS_BOX) {
     c->lds_box = value != 0;
+  } else if (option == RL_OPT_IDLE_BYTES) {
+    CHECK_ARG(value >= 0, "RL_OPT_IDLE_BYTES must be >= 0");
+    TRY(use_device(c));
+    c->pool.set_limit((size_t)value);
   } else {
     return fail(RL_ERR_ARG, "unknown option %d", option);
   }

@@ -703,10 +703,9 @@ void sg_free(rl_surrogate* s) {
 }
 
 template <typename T>
-int sg_alloc(T** p, size_t count) {
-  if (hipMalloc((void**)p, count * sizeof(T)) != hipSuccess) {
+int sg_alloc(rl_ctx* c, T** p, size_t count) {
+  if (c->pool.alloc_plain(p, count * sizeof(T)) != hipSuccess) {
     (void)hipGetLastError();
-    *p = nullptr;
     return fail(RL_ERR_NOMEM, "surrogate: device allocation of %zu bytes failed", count * sizeof(T));
   }
   return RL_OK;
@@ -714,10 +713,10 @@ int sg_alloc(T** p, size_t count) {
 
 // Frees *p and allocates count elements.
 template <typename T>
-int sg_regrow(T** p, size_t count) {
+int sg_regrow(rl_ctx* c, T** p, size_t count) {
   if (*p) (void)hipFree(*p);
   *p = nullptr;
-  return sg_alloc(p, count);
+  return sg_alloc(c, p, count);
 }
 
 // Ray buffers for n rays.
@@ -726,10 +725,10 @@ int sg_reserve(rl_surrogate* s, int n) {
   HIP_TRY(hipStreamSynchronize(s->map->ctx->stream));
   s->cap = 0;
   size_t c = (size_t)n;
-  TRY(sg_regrow(&s->d_rays, c));
-  TRY(sg_regrow(&s->d_out, c * RL_SG_OUT));
-  TRY(sg_regrow(&s->d_poses, c * 3));
-  TRY(sg_regrow(&s->d_target, c));
+  TRY(sg_regrow(s->map->ctx, &s->d_rays, c));
+  TRY(sg_regrow(s->map->ctx, &s->d_out, c * RL_SG_OUT));
+  TRY(sg_regrow(s->map->ctx, &s->d_poses, c * 3));
+  TRY(sg_regrow(s->map->ctx, &s->d_target, c));
   s->cap = n;
   return RL_OK;
 }
@@ -743,14 +742,14 @@ int sg_reserve_train(rl_surrogate* s, int n, size_t partials) {
     const size_t ld = ((size_t)n + 63) / 64 * 64;
     // every minibatch of up to n rays is cut into at most this many slices
     const size_t slices = std::min<size_t>(RL_SG_MAX_SPLIT, ((size_t)n + 1023) / 1024);
-    TRY(sg_regrow(&s->d_t, SgT::N * ld));
-    TRY(sg_regrow(&s->d_split, slices * RL_SGT_PART));
-    TRY(sg_regrow(&s->d_bsplit, (size_t)256 * RL_SGT_BIAS));
+    TRY(sg_regrow(s->map->ctx, &s->d_t, SgT::N * ld));
+    TRY(sg_regrow(s->map->ctx, &s->d_split, slices * RL_SGT_PART));
+    TRY(sg_regrow(s->map->ctx, &s->d_bsplit, (size_t)256 * RL_SGT_BIAS));
     s->tcap = n;
   }
   if (s->pcap < partials) {
     s->pcap = 0;
-    TRY(sg_regrow(&s->d_partial, partials));
+    TRY(sg_regrow(s->map->ctx, &s->d_partial, partials));
     s->pcap = partials;
   }
   return RL_OK;
@@ -792,7 +791,7 @@ int sg_forward_layers(rl_surrogate* s, int n) {
   const int w_off[4] = {SgLayout::W1, SgLayout::W2, SgLayout::W3, SgLayout::W4};
   const int b_off[4] = {SgLayout::B1, SgLayout::B2, SgLayout::B3, SgLayout::B4};
   int rc = RL_OK;
-  for (int l = 0; l < 4 && rc == RL_OK; ++l) rc = sg_alloc(&act[l], (size_t)n * fin[l]);
+  for (int l = 0; l < 4 && rc == RL_OK; ++l) rc = sg_alloc(m->ctx, &act[l], (size_t)n * fin[l]);
   if (rc == RL_OK) {
     hipLaunchKernelGGL(k_sg_features, dim3(grid_for(n, 256)), dim3(256), 0, st, (const float4*)s->d_rays,
                        (const float*)s->d_freq, 1.0f / (float)m->width, 1.0f / (float)m->height, act[0], n);
@@ -904,11 +903,11 @@ int rl_surrogate_create(rl_map* map, unsigned seed, rl_surrogate** out) {
   s->map = map;
   map->refs.fetch_add(1);
   int rc = RL_OK;
-  if ((rc = sg_alloc(&s->d_p, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_m1, RL_SG_NPARAM)) ||
-      (rc = sg_alloc(&s->d_m2, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_g, RL_SG_NPARAM)) ||
-      (rc = sg_alloc(&s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(&s->d_pf, SgFrag::N)) ||
-      (rc = sg_alloc(&s->d_freq, RL_SG_NF * 4)) ||
-      (rc = sg_alloc(&s->d_stats, 5))) {
+  if ((rc = sg_alloc(map->ctx, &s->d_p, RL_SG_NPARAM)) || (rc = sg_alloc(map->ctx, &s->d_m1, RL_SG_NPARAM)) ||
+      (rc = sg_alloc(map->ctx, &s->d_m2, RL_SG_NPARAM)) || (rc = sg_alloc(map->ctx, &s->d_g, RL_SG_NPARAM)) ||
+      (rc = sg_alloc(map->ctx, &s->d_pb, RL_SG_NPARAM)) || (rc = sg_alloc(map->ctx, &s->d_pf, SgFrag::N)) ||
+      (rc = sg_alloc(map->ctx, &s->d_freq, RL_SG_NF * 4)) ||
+      (rc = sg_alloc(map->ctx, &s->d_stats, 5))) {
     sg_free(s);
     delete s;
     map->refs.fetch_sub(1);  // cannot reach zero: the caller holds the map
@@ -1188,8 +1187,8 @@ static int debug_gemm(rl_ctx* c, const uint16_t* A, const uint16_t* B, float* C,
   bf16_t *dA = nullptr, *dB = nullptr;
   float* dC = nullptr;
   int rc = RL_OK;
-  if ((rc = sg_alloc(&dA, (size_t)M * K)) || (rc = sg_alloc(&dB, (size_t)K * N)) ||
-      (rc = sg_alloc(&dC, (size_t)M * N))) {
+  if ((rc = sg_alloc(c, &dA, (size_t)M * K)) || (rc = sg_alloc(c, &dB, (size_t)K * N)) ||
+      (rc = sg_alloc(c, &dC, (size_t)M * N))) {
     if (dA) (void)hipFree(dA);
     if (dB) (void)hipFree(dB);
     return rc;

@@ -665,6 +665,57 @@ def test_map_buffers_reused(ctx):
         assert_bits_equal(out.cpu().numpy()[:3000], want[k % 3], f"map {k}")
 
 
+def test_idle_device_memory_is_given_back():
+    """Memory of closed maps that the context keeps comes back when the limit is
+    lowered, when another allocation of the context fails, and with the context; maps
+    made in kept memory and after are as any."""
+    torch = _torch()
+    img = W.rect_disk_map(4000, seed=1)
+    occ = O.xmajor(img)
+    kept = 64 << 20  # the distance map alone
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    def closed_map(c):
+        rl.DeviceMap(c, occ).close()
+
+    c = rl.Context(0)
+    c.set_option(rl._lib.RL_OPT_IDLE_BYTES, 0)
+    closed_map(c)
+    before = free()
+    closed_map(c)
+    assert before - free() < kept // 2  # nothing is kept
+    c.set_option(rl._lib.RL_OPT_IDLE_BYTES, 1 << 30)
+    closed_map(c)
+    assert before - free() > kept // 2
+    c.set_option(rl._lib.RL_OPT_IDLE_BYTES, 0)
+    assert before - free() < kept // 2
+    c.set_option(rl._lib.RL_OPT_IDLE_BYTES, 1 << 30)
+    small = rl.DeviceMap(c, np.zeros((8, 8), np.uint8))
+    sg = rl.Surrogate(small, seed=1)
+    closed_map(c)
+    assert before - free() > kept // 2
+    n = 100_000_000  # 373 GB of training matrices
+    with pytest.raises(rl.RangeLibError):
+        sg.gradient(10.0, np.zeros((n, 4), np.float32), np.zeros(n, np.float32))
+    sg.close()
+    assert before - free() < kept // 2
+    with pytest.raises(rl.RangeLibError):
+        c.set_option(rl._lib.RL_OPT_IDLE_BYTES, -1)
+    dm = rl.DeviceMap(c, occ)
+    q = W.grid_poses(img, 1000, seed=2)
+    out = np.zeros(1000, np.float32)
+    dm.calc_range_many(rl.RL_METHOD_RM, 300.0, q, out, 1000)
+    assert_bits_equal(out, O.Oracle(img, 300.0, "rm").calc_range_many(q), "after")
+    dm.close()
+    small.close()
+    del dm, small, sg
+    c.close()
+    assert before - free() < kept // 2
+
+
 @pytest.mark.parametrize("h,w", [(1, 1), (7, 8), (8, 7), (65, 17), (64, 64), (129, 130), (4096, 9), (4097, 9),
                                  (20, 3966), (20, 3967), (1500, 3900)])
 def test_map_build_tiles(ctx, h, w):
