@@ -1601,6 +1601,7 @@ struct rl_map {
   float *cddt_trans = nullptr, *cddt_cos = nullptr, *cddt_sin = nullptr, *cddt_vals = nullptr;
   long long *cddt_bin_off = nullptr, *cddt_start = nullptr;
   int cddt_td = 0, cddt_nang = 0;
+  bool cddt_solid = false;  // mostly solid blocks (see there)
   long long cddt_nb = 0, cddt_nv = 0;
   float cddt_td_div_2pi = 0.0f, cddt_ms = 0.0f;
 

@@ -242,3 +242,34 @@ def test_cddt_bins_beyond_a_grid(ctx):
     out = np.zeros(500, np.float32)
     dm.calc_range_many(rl.RL_METHOD_CDDT, 50.0, q, out, 500)
     assert_bits_equal(out, np.full(500, 50.0, np.float32), "empty tables")
+
+
+def _block_map(name):
+    if name == "half":
+        img = np.zeros((203, 310), np.uint8)
+        img[:, 140:] = 1
+    elif name == "stripes":
+        img = (np.arange(317)[:, None] % 61 < 40).astype(np.uint8) * np.ones((1, 258), np.uint8)
+    elif name == "rooms":
+        img = np.ones((301, 290), np.uint8)
+        for y, x, h, w in ((0, 0, 9, 7), (290, 5, 11, 3), (7, 280, 1, 10), (120, 130, 40, 8), (200, 250, 3, 40)):
+            img[y:y + h, x:x + w] = 0
+    else:  # one free cell in the middle of a solid map
+        img = np.ones((161, 250), np.uint8)
+        img[80, 131] = 0
+    return img
+
+
+@pytest.mark.parametrize("td", [1, 2, 8, 61])
+@pytest.mark.parametrize("name", ["half", "stripes", "rooms", "lone"])
+def test_cddt_prune_through_blocks(ctx, name, td):
+    """Pruned tables of maps whose walks cross solid tiles, more and fewer than eight in
+    a row, and tiles that the map's edge cuts: against the oracle."""
+    img = _block_map(name)
+    for im in (img, np.ascontiguousarray(img.T)):
+        dm = rl.DeviceMap(ctx, O.xmajor(im))
+        dm.build_cddt(td)
+        dm.prune_cddt(50.0)
+        got, want = dm.cddt_tables(), O.Oracle(im, 50.0, "cddt", theta_disc=td, prune=True).cddt_tables()
+        assert np.array_equal(got["start"], want["start"])
+        assert_bits_equal(got["vals"], want["vals"], "pruned")
