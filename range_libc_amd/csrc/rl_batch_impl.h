@@ -137,12 +137,13 @@ int batch_upload(rl_batch* b) {
   std::vector<std::pair<double, BatchItem>> items;
   b->gens.resize(nj);
   for (int i = 0; i < nj; ++i) b->gens[i] = b->jobs[i].map->gen.load();
-  // one kernel for the whole list: pooled when every map's rays could be
+  // one kernel for the whole list: pooled when every map's rays can be and one ray per
+  // lane would not be resident at once
   long long rays = 0;
   for (const rl_batch_job& j : b->jobs) rays += (long long)j.num_particles * j.num_angles;
-  b->pooled = b->method == RL_METHOD_RM && !b->lds_box;
+  b->pooled = b->method == RL_METHOD_RM && !b->lds_box && rays > RL_POOL_MIN_RAYS;
   for (const rl_batch_job& j : b->jobs)
-    b->pooled = b->pooled && (j.num_particles == 0 || pool_pays(j.map, rays, j.num_angles));
+    b->pooled = b->pooled && (j.num_particles == 0 || pool_fits(j.map, j.num_angles));
   for (int i = 0; i < nj; ++i) {
     const rl_batch_job& j = b->jobs[i];
     BatchMap& bm = maps[i];

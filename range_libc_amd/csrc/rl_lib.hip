@@ -1706,24 +1706,52 @@ int launch_sensor(rl_map* m, const float* obs, const float* ranges, double* outs
 }
 
 // Rule for the pool of rays per wave (k_particles_pool).  One ray per lane
-// (k_particles) keeps 4096 waves resident, and is the better form while all rays
+// (k_particles, k_fused) keeps 4096 waves resident that form ranges and weights, 5120
+// that form weights and 7168 that form ranges, and is the better form while all rays
 // fit them at once: then a launch lasts as long as its longest ray, which a pool
-// starts later (2048^2 corridors, 60 beams: 4000 particles 22.2 us, pooled 25.8;
-// 5000: 29.6, 26.5; 6000: 34.5, 27.8; 40000: 150.6, 67.3).  A wave's rays are
-// cast together from 96 up, and up to what LDS holds as long as the launch still
-// has a wave for each that the chip keeps resident (1531 x 1999, 107 beams,
-// 20011 particles: 128, 256, 384, 512 rays a wave 121, 119, 103, 100 us; 12000:
-// 84, 74, 80, 86).
+// starts later.  Time of the pool over that of one ray per lane, over five maps with
+// short and long rays, 32 and 60 beams a particle:
+//   rays (thousands)     262          350          400          600
+//   ranges and weights   0.85 - 1.06  0.81 - 0.96  0.80 - 0.97  0.66 - 0.92
+//   ranges               1.02 - 1.12  1.03 - 1.11  0.88 - 1.03  0.85 - 1.09
+//   weights              0.59 - 1.15  0.60 - 1.00  0.61 - 1.00  0.56 - 1.06
+// so the line is at 4096 full waves, at 6144 waves of up to 64 beams for ranges alone
+// (above 64 a wave casts a particle's beams in several rounds, the last not full: the
+// pool's 0.69 to 0.96 at 262 thousand, 100 and 200 beams).  k_fused's rays of one long
+// map keep a wave each to their end, which is why weights gain at any size there (36 ->
+// 22 us) and the line is not at its 5120 waves (short rays at 300 thousand, 11 -> 12 us).
+// A particle of more beams than a pool holds is marched pool by pool, each with the
+// tail of its last rays: 600 beams 0.79 - 1.10, 1100 0.85 - 1.15, 2000 0.91 - 1.23.
+//
+// A wave's rays are cast together from 96 up, and up to what LDS holds as long as the
+// launch still has a wave for each that the chip keeps resident (1531 x 1999, 107
+// beams, 20011 particles: 128, 256, 384, 512 rays a wave 121, 119, 103, 100 us; 12000:
+// 84, 74, 80, 86), and at most 64 (or one particle's) while the resident waves hold the
+// launch so (4 beams, ranges and weights of 262 thousand rays 1.04 - 1.16 of one ray per
+// lane with 96, 0.87 - 1.02 with 64).
 #define RL_POOL_MIN_RAYS (4096 * 64)
 #define RL_POOL_RESIDENT 7168  // waves of the pool's kernels that the chip keeps resident
-#define RL_POOL_WAVE_RAYS 96   // rays of a wave at least
+#define RL_POOL_WAVE_RAYS 96   // rays of a wave at least, past 64 a wave
+#define RL_POOL_MAX_BEAMS 1024
 
-bool pool_pays(const rl_map* m, long long rays, int M) {
-  return rays > RL_POOL_MIN_RAYS && M * RL_POOL_PARTICLES >= RL_POOL_WAVE_RAYS && m->d_idx8 && !m->ctx->lds_box;
+// Whether rays of M beams per particle can be marched from pools (beams are counted in
+// int, a pool beyond the last).
+bool pool_fits(const rl_map* m, int M) {
+  return M >= (RL_POOL_WAVE_RAYS + RL_POOL_PARTICLES - 1) / RL_POOL_PARTICLES && M <= 1 << 20 && m->d_idx8 &&
+         !m->ctx->lds_box;
+}
+
+// Whether a launch of N particles of M beams is cast from pools; ranges: it forms ranges alone.
+bool pool_pays(const rl_map* m, int N, int M, bool ranges) {
+  if ((long long)N * M <= RL_POOL_MIN_RAYS || M > RL_POOL_MAX_BEAMS || !pool_fits(m, M)) return false;
+  const int per_wave = 64 / segment_size(M);
+  return !ranges || M > 64 || N / per_wave >= 6144;
 }
 
 // Particles of M beams that a wave takes of a launch of `rays` rays.
 int pool_particles_per_wave(long long rays, int M) {
+  const int one = std::max(1, std::min(64 / M, RL_POOL_PARTICLES));  // of at most 64 rays
+  if (rays / M <= (long long)one * RL_POOL_RESIDENT) return one;
   const long long want = std::max<long long>(RL_POOL_WAVE_RAYS, rays / RL_POOL_RESIDENT);
   const long long g = std::min<long long>((want + M - 1) / M, std::min(RL_POOL_RAYS / M, RL_POOL_PARTICLES));
   return g < 1 ? 1 : (int)g;
@@ -1747,7 +1775,7 @@ int launch_fused(rl_map* m, int method, float max_range, const float* ins, const
   int S = segment_size(M);
   long long waves = ((long long)N + 64 / S - 1) / (64 / S);
   dim3 grid(grid_for(waves * 64, 256)), block(256);
-  if (method == RL_METHOD_RM && pool_pays(m, (long long)N * M, M))
+  if (method == RL_METHOD_RM && pool_pays(m, N, M, false))
     launch_pool<POOL_WEIGHTS>(m, max_range, ins, angles, obs, nullptr, weights, N, M);
   else if (method == RL_METHOD_BL)
     hipLaunchKernelGGL(k_fused<RL_METHOD_BL>, grid, block, 0, m->ctx->stream, m->dev(), m->ctx->trig,
@@ -1798,7 +1826,7 @@ int launch_particles_t(rl_map* m, float max_range, const float* ins, const float
     long long blocks = RL_REGIONS * ((N + per_block - 1) / per_block);
     hipLaunchKernelGGL((k_particles_xcd<METHOD, SENSOR>), dim3((unsigned)blocks), dim3(256), 0, c->stream,
                        m->dev(), c->trig, max_range, ins, angles, obs, table, K, ranges, weights, M, S, sc);
-  } else if (METHOD == RL_METHOD_RM && pool_pays(m, (long long)N * M, M)) {
+  } else if (METHOD == RL_METHOD_RM && pool_pays(m, N, M, !SENSOR)) {
     launch_pool<SENSOR ? POOL_STEP : POOL_RANGES>(m, max_range, ins, angles, obs, ranges, weights, N, M);
   } else {
     long long waves = ((long long)N + 64 / S - 1) / (64 / S);

@@ -567,6 +567,14 @@ def test_pooled_rays(n, m, R, world, rect_map):
     assert np.array_equal(w2.cpu().numpy(), orc.calc_range_repeat_angles_eval_sensor_model(ins, ang, obs))
 
 
+@pytest.mark.parametrize("n,m", [(98_303, 3), (98_304, 3), (29_200, 9), (43_100, 9), (13_000, 21), (6143, 60), (6144, 60),
+                                 (7168, 60), (7169, 60), (6150, 64), (4100, 65), (257, 1024), (257, 1025)])
+def test_pooled_rays_at_the_rules_lines(n, m, rect_map):
+    """Both sides of the lines between one ray per lane and pools of up to 64 rays, of
+    96 and more, and of a particle's beams."""
+    test_pooled_rays(n, m, 300.0, None, rect_map)
+
+
 @pytest.mark.parametrize("xcd,box", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_scheduling_options(xcd, box, corridor_map):
     """XCD-aware scheduling and LDS staging change only where data is read from."""
