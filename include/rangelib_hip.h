@@ -334,9 +334,12 @@ int rl_debug_chase_dev(rl_ctx* ctx, const unsigned* d_next, int steps, long long
 /* C = A * B through the surrogate's bf16 matrix-core GEMM (host row-major
  * matrices of bf16 bit patterns; fp32 result). */
 int rl_debug_gemm_bf16(rl_ctx* ctx, const uint16_t* A, const uint16_t* B, float* C, int M, int N, int K);
-/* rl_surrogate_forward through the per-layer kernels that training uses
+/* rl_surrogate_forward through plain per-layer kernels, kept for comparison
  * (rl_surrogate_forward itself runs one fused kernel with the same outputs). */
 int rl_debug_surrogate_forward_layers(rl_surrogate* s, const float* rays4, int n, float* out);
+/* The hidden layers' activations of n rays, 3 x n x 256 bf16 bit patterns (host):
+ * the training pass's, or the per-layer kernels'. */
+int rl_debug_surrogate_hidden(rl_surrogate* s, const float* rays4, int n, int training, uint16_t* hidden);
 /* Number of float bit patterns (of all 2^32) on which the fused surrogate
  * kernel's bf16 conversion differs from the per-layer kernels' (expected 0). */
 int rl_debug_bf16_check(rl_ctx* ctx, unsigned long long* mismatches);

@@ -99,6 +99,7 @@ SIGNATURES = {
     "rl_surrogate_set_params": [_vp, _vp, _vp],
     "rl_surrogate_forward": [_vp, _vp, C.c_int, _vp],
     "rl_debug_surrogate_forward_layers": [_vp, _vp, C.c_int, _vp],
+    "rl_debug_surrogate_hidden": [_vp, _vp, C.c_int, C.c_int, _vp],
     "rl_debug_bf16_check": [_vp, _vp],
     "rl_surrogate_gradient": [_vp, C.c_float, _vp, _vp, C.c_int, _fp, _vp, _vp],
     "rl_surrogate_step": [_vp, C.c_float],
@@ -511,10 +512,18 @@ class Surrogate:
         return out
 
     def forward_layers(self, rays4: np.ndarray) -> np.ndarray:
-        """forward() through the per-layer kernels that training uses (test hook)."""
+        """forward() through plain per-layer kernels, kept for comparison (test hook)."""
         r = np.ascontiguousarray(rays4, np.float32).reshape(-1, 4)
         out = np.empty((r.shape[0], 2), np.float32)
         check(lib().rl_debug_surrogate_forward_layers(self.handle, ptr(r), r.shape[0], ptr(out)))
+        return out
+
+    def hidden(self, rays4: np.ndarray, training: bool) -> np.ndarray:
+        """Hidden activations (3, n, 256), bf16 bit patterns, of the training pass or of
+        the per-layer kernels (test hook)."""
+        r = np.ascontiguousarray(rays4, np.float32).reshape(-1, 4)
+        out = np.empty((3, r.shape[0], 256), np.uint16)
+        check(lib().rl_debug_surrogate_hidden(self.handle, ptr(r), r.shape[0], int(training), ptr(out)))
         return out
 
     def gradient(self, max_range: float, rays4: np.ndarray, targets: np.ndarray):

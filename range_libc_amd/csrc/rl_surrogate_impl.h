@@ -101,7 +101,8 @@ struct SgFrag {
 // GEMM: C(m, n) = sum_k A(m, k) * B(k, n), bf16 operands, fp32 accumulation.
 // A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn] (any
 // transposition).  Epilogue: + bias[n], relu, then store fp32 and/or bf16.
-// Serves the per-layer forward pass (the heads) and the GEMM hooks.
+// Serves the per-layer forward pass (the heads) and the GEMM hooks, which are test
+// hooks only, as are k_gemm_bf16_nt and k_sg_features.
 // Tile 64 x 64 per 256-thread workgroup, each wave 32 x 32 (2 x 2 MFMA tiles
 // of 16 x 16), k in steps of 32 through LDS.
 struct GemmArgs {
@@ -780,9 +781,11 @@ GemmArgs gemm_args() {
   return g;
 }
 
-// Forward pass of n rays already in d_rays, layer by layer, into d_out: the
-// plain form that k_sg_infer is compared with (its buffers live for the call).
-int sg_forward_layers(rl_surrogate* s, int n) {
+// Forward pass of n rays already in d_rays, layer by layer, into d_out, and the hidden
+// layers' activations (3 x n x 256, host, optional): the plain form that k_sg_infer and
+// k_sg_fwd_bwd are compared with, reached by the debug entry points only (its buffers
+// live for the call).
+int sg_forward_layers(rl_surrogate* s, int n, bf16_t* hidden) {
   rl_map* m = s->map;
   hipStream_t st = m->ctx->stream;
   bf16_t* act[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -818,6 +821,10 @@ int sg_forward_layers(rl_surrogate* s, int n) {
       g.C = s->d_out;
     rc = sg_gemm(st, g);
   }
+  for (int l = 1; hidden && l < 4 && rc == RL_OK; ++l)
+    if (hipMemcpyAsync(hidden + (size_t)(l - 1) * n * RL_SG_H, act[l], (size_t)n * RL_SG_H * sizeof(bf16_t),
+                       hipMemcpyDeviceToHost, st) != hipSuccess)
+      rc = fail(RL_ERR_HIP, "surrogate layers failed");
   if (rc == RL_OK && hipStreamSynchronize(st) != hipSuccess) rc = fail(RL_ERR_HIP, "surrogate layers failed");
   for (bf16_t* a : act)
     if (a) (void)hipFree(a);
@@ -1008,7 +1015,7 @@ static int surrogate_forward(rl_surrogate* s, const float* rays4, int n, float* 
   TRY(sg_reserve(s, n));
   hipStream_t st = s->map->ctx->stream;
   HIP_TRY(hipMemcpyAsync(s->d_rays, rays4, (size_t)n * 16, hipMemcpyHostToDevice, st));
-  TRY(layers ? sg_forward_layers(s, n) : sg_infer(s, n));
+  TRY(layers ? sg_forward_layers(s, n, nullptr) : sg_infer(s, n));
   HIP_TRY(hipMemcpyAsync(out, s->d_out, (size_t)n * 8, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   return RL_OK;
@@ -1145,10 +1152,34 @@ int rl_debug_gemm_bf16(rl_ctx* c, const uint16_t* A, const uint16_t* B, float* C
   return debug_gemm(c, A, B, C, M, N, K, false);
 }
 
-// rl_surrogate_forward through the per-layer kernels the training uses (test
-// hook for the fused inference kernel).
+// rl_surrogate_forward through the per-layer kernels, which serve these debug entry
+// points only (test hook for the fused inference kernel).
 int rl_debug_surrogate_forward_layers(rl_surrogate* s, const float* rays4, int n, float* out) {
   return surrogate_forward(s, rays4, n, out, true);
+}
+
+// Hidden activations (3 x n x 256 bf16 bit patterns) of the training pass, or of the
+// per-layer kernels (test hook for the training kernel's forward).
+int rl_debug_surrogate_hidden(rl_surrogate* s, const float* rays4, int n, int training, uint16_t* hidden) {
+  CHECK_ARG(s && rays4 && hidden && n > 0, "bad argument");
+  if (training) {
+    const std::vector<float> zeros((size_t)n, 0.0f);
+    TRY(rl_surrogate_gradient(s, 1.0f, rays4, zeros.data(), n, nullptr, nullptr, nullptr));
+  }
+  std::lock_guard<std::mutex> lk(s->map->ctx->mu);
+  TRY(use_device(s->map->ctx));
+  hipStream_t st = s->map->ctx->stream;
+  if (!training) {
+    TRY(sg_reserve(s, n));
+    HIP_TRY(hipMemcpyAsync(s->d_rays, rays4, (size_t)n * 16, hipMemcpyHostToDevice, st));
+    return sg_forward_layers(s, n, hidden);
+  }
+  const size_t ld = ((size_t)n + 63) / 64 * 64;
+  for (int l = 0; l < 3; ++l)
+    HIP_TRY(hipMemcpyAsync(hidden + (size_t)l * n * RL_SG_H, s->d_t + (SgT::A1 + l * RL_SG_H) * ld,
+                           (size_t)n * RL_SG_H * sizeof(bf16_t), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  return RL_OK;
 }
 
 // Mismatches between the fused kernel's bf16 conversion and f2bf over all

@@ -442,3 +442,19 @@ def test_fused_forward_of_nan_and_infinite_parameters(ctx, layer, what, bits):
         dm.numpy_calc_range_angles_dev(rl.RL_METHOD_RM, R, ins.data_ptr(), ang.data_ptr(), want.data_ptr(), n, 7)
         ctx.sync()
         assert_bits_equal(got.cpu().numpy(), want.cpu().numpy(), "checked cast")
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 777])
+def test_training_forward_equals_layers(ctx, n):
+    """The training pass's hidden activations are bitwise the per-layer kernels', whose
+    outputs the fused inference has: what is trained is what infers."""
+    img, g, rays = _map_and_rays(n, seed=7)
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    sg = rl.Surrogate(dm, seed=4)
+    p = sg.params()[0].copy()
+    rng = np.random.default_rng(n)
+    for w, b, o, i in S.LAYERS:
+        p[b:b + o] = rng.uniform(-0.5, 0.5, o)
+    sg.set_params(p)
+    assert np.array_equal(sg.hidden(rays, training=True), sg.hidden(rays, training=False))
+    assert_bits_equal(sg.forward(rays), sg.forward_layers(rays), "fused vs per-layer forward")
