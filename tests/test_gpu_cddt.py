@@ -273,3 +273,22 @@ def test_cddt_prune_through_blocks(ctx, name, td):
         got, want = dm.cddt_tables(), O.Oracle(im, 50.0, "cddt", theta_disc=td, prune=True).cddt_tables()
         assert np.array_equal(got["start"], want["start"])
         assert_bits_equal(got["vals"], want["vals"], "pruned")
+
+
+@pytest.mark.parametrize("td", [1, 2, 4, 7])
+@pytest.mark.parametrize("w,h", [(12, 16384), (12, 16385), (17000, 12), (12, 17000)])
+def test_cddt_bins_beyond_lds(ctx, w, h, td):
+    """Maps whose widest angle has as many bins as the LDS counters hold, and more,
+    whose entries are counted in memory: whole tables, full and pruned, against the
+    oracle."""
+    img = (np.random.default_rng(w + h).random((h, w)) < 0.01).astype(np.uint8)
+    img[h // 3:h // 3 + 9, :] = 1
+    dm = rl.DeviceMap(ctx, O.xmajor(img))
+    dm.build_cddt(td)
+    for prune in (False, True):
+        if prune:
+            dm.prune_cddt(50.0)
+        got, want = dm.cddt_tables(), O.Oracle(img, 50.0, "cddt", theta_disc=td, prune=prune).cddt_tables()
+        assert np.array_equal(got["widths"], want["widths"])
+        assert np.array_equal(got["start"], want["start"]), "pruned" if prune else "full"
+        assert_bits_equal(got["vals"], want["vals"], "pruned" if prune else "full")
