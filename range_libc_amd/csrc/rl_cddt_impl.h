@@ -346,12 +346,6 @@ __global__ __launch_bounds__(256) void k_cddt_prune_mark(const uint8_t* __restri
     for (int q = q0 >> 3; q <= q1 >> 3; ++q) t &= row0[(size_t)(p0 >> 3) * (unsigned)nt + q];
     return t == ~0ull;
   };
-  // orders a wave's LDS accesses
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
   __shared__ int sel[4][8];
   int* slot = sel[threadIdx.x >> 6];
   long long cnt = 0;
@@ -378,10 +372,10 @@ __global__ __launch_bounds__(256) void k_cddt_prune_mark(const uint8_t* __restri
       if (!lm) break;
       const int rank = __popcll(lm & ((1ull << lane) - 1ull)), grp = lane >> 3;
       if (left && rank < 8) slot[rank] = lane;
-      wave_sync();
+      wave_lds_sync();
       const bool helps = grp < __popcll(lm);
       const int owner = helps ? slot[grp] : lane;
-      wave_sync();  // read before the next round's writes
+      wave_lds_sync();  // read before the next round's writes
       const float olo = __shfl(lo, owner), ohi = __shfl(hi, owner);
       int op = __shfl(p, owner);
       const int op1 = __shfl(p1, owner);

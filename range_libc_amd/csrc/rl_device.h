@@ -549,9 +549,11 @@ __device__ __forceinline__ float rm_cast_idx8(const MapDev& m, const float* lut,
 // resource, which gives code 0, whose infinite step takes t past max_range as a
 // long step does, and one comparison decides whether the ray goes on.  A lane
 // whose ray has ended reads its last cell again and stays; once RL_POOL_REFILL
-// lanes have ended they are finished and refilled together.  The rays then left
-// are marched one per lane with speculation (rm_march_idx8_t), the last of them
-// by the whole wave.  Positions and float operations are those of the plain march.
+// lanes have ended they are finished and refilled together.  The rounds end with a
+// refill, which leaves no ended ray in a lane (so no lane goes on with a hit's code 0).
+// The rays then left are marched one per lane with speculation (rm_march_idx8_t), the
+// last of them by the whole wave.  Positions and float operations are those of the
+// plain march.
 #define RL_POOL_REFILL 8  // 4, 8, 12, 16: within 1% of each other
 template <class Fetch, class Finish>
 __device__ __forceinline__ void pool_march(const MapDev& m, const float* lut, float max_range, int n,

@@ -883,6 +883,7 @@ struct PoolLds {
 // more than the two roundings move it.
 __device__ __forceinline__ int pool_particle(int r, float inv) { return (int)(((float)r + 0.5f) * inv); }
 
+// Orders a wave's LDS accesses.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -103,11 +103,6 @@ __device__ __forceinline__ void sgt_mul(SgAcc& acc, const bf16_t* act, const sg_
     }
 }
 
-// Two floats rounded to bf16 (nearest even), v0 in the low half.
-__device__ __forceinline__ unsigned sgt_pack(float v0, float v1) {
-  return (unsigned)__builtin_bit_cast(bf16_t, (__bf16)v0) | ((unsigned)__builtin_bit_cast(bf16_t, (__bf16)v1) << 16);
-}
-
 // Forward epilogue: bias, relu, bf16 into the LDS tile; bit 8 i + 4 j + q of
 // the result is set where the rounded value is positive.
 __device__ __forceinline__ unsigned sgt_out_fwd(const SgAcc& acc, bf16_t* act, const float* sb, int wave, int lane) {
@@ -126,7 +121,7 @@ __device__ __forceinline__ unsigned sgt_out_fwd(const SgAcc& acc, bf16_t* act, c
         // values up to 2^-134 round to zero
         pos |= v[q] > 0x1p-134f ? 1u << (8 * i + 4 * j + q) : 0u;
       }
-      *(uint2*)(act + (i * 16 + (lane & 15)) * RL_SG_ACT_PAD + c) = make_uint2(sgt_pack(v[0], v[1]), sgt_pack(v[2], v[3]));
+      *(uint2*)(act + (i * 16 + (lane & 15)) * RL_SG_ACT_PAD + c) = make_uint2(sg_pack2(v[0], v[1]), sg_pack2(v[2], v[3]));
     }
   }
   return pos;
@@ -145,7 +140,7 @@ __device__ __forceinline__ void sgt_out_bwd(const SgAcc& acc, unsigned pos, bf16
         const int keep = (int)(pos << (31 - (8 * i + 4 * j + q))) >> 31;  // the bit over the whole word
         v[q] = __int_as_float(__float_as_int(acc[i][j][q]) & keep);
       }
-      *(uint2*)(act + (i * 16 + (lane & 15)) * RL_SG_ACT_PAD + c) = make_uint2(sgt_pack(v[0], v[1]), sgt_pack(v[2], v[3]));
+      *(uint2*)(act + (i * 16 + (lane & 15)) * RL_SG_ACT_PAD + c) = make_uint2(sg_pack2(v[0], v[1]), sg_pack2(v[2], v[3]));
     }
   }
 }
