@@ -6,12 +6,12 @@
 //   1. per-angle constants (one thread per angle, the library's sinf/cosf);
 //   2. edge cells (occupied with a free 8-neighbour, OMap::make_edge_map);
 //   3. every (edge cell, angle < td/2) pair projects the cell centre into the
-//      bins its footprint covers: a counting pass (atomics), an exclusive scan
-//      into bin offsets, and a filling pass;
+//      bins its footprint covers: a counting pass (in LDS, in memory for the widest
+//      maps), an exclusive scan into bin offsets, and a filling pass;
 //   4. each bin sorted (segmented bitonic sort, rl_scan_sort.h) and its
 //      duplicates dropped;
-//   5. prune: every free cell marks the entries a query from it can return,
-//      unmarked entries are dropped.
+//   5. prune: the entries that a query from some free cell can return are found by
+//      intervals between entries, the others are dropped.
 // The result equals the reference's compressed_lut bin for bin: the order in
 // which entries arrive does not matter after sorting and deduplication.
 

@@ -1073,8 +1073,9 @@ __global__ __launch_bounds__(256) void k_glt_steps(const float* __restrict__ edt
 // are assembled in LDS and stored by rows of cells, which are contiguous in the
 // table.  Same values as k_glt_build, entry by entry.
 //
-// The launch is bound by its L1 accesses (1.58 G, one per lane and read: 2.7 ms
-// at one a cycle and CU) and by VALU work (1.06 G, 1.8 ms), so the march reads the cells' steps
+// The launch's reads and its VALU instructions take about as long as it does (texture
+// addressing busy 74% of it, 1.08 G instructions 1.76 of 2.57 ms; waves wait on reads 78%
+// of their time, though 94% of 1.58 G hit the L1), so the march reads the cells' steps
 // (k_glt_steps) instead of their codes: a position off the map is clamped to the
 // border of infinite steps, an ending cell's infinite step takes t past
 // max_range, and one comparison per read decides whether the ray goes on (12

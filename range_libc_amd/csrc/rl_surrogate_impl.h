@@ -10,8 +10,8 @@
 //   a1 = relu(W1 phi + b1), a2 = relu(W2 a1 + b2), a3 = relu(W3 a2 + b3)   (256 wide)
 //   o  = W4 a3 + b4,  range = R * o[0],  error bound = exp(o[1]) cells
 // Weights are stored in fp32 (master copy, Adam) and bf16 (MFMA operands);
-// products accumulate in fp32 (v_mfma_f32_16x16x32_bf16 for the 256-wide
-// layers, v_mfma_f32_16x16x16_bf16 elsewhere).
+// products accumulate in fp32 (v_mfma_f32_16x16x32_bf16; the general GEMM of the test
+// hooks takes v_mfma_f32_16x16x16_bf16).
 //
 // Loss per ray: Huber (delta 1 cell) on range - marched range, plus the
 // pinball loss at quantile 0.95 between the bound and the observed absolute
@@ -36,9 +36,10 @@
 // Rejected candidates and the other rays are marched from the origin (exact).
 // Accepted ranges can still differ from the exact march where its phase picks
 // a cell that no probe picked; the error is measured against the marcher.
-// Reads: every read of both steps and of the fallback march is counted, and
-// the dependent rounds of the path (one for the certificate, the longest
-// probe, the fallback march) separately.
+// Reads: every sample of the certificate, read of the probes and read of the
+// fallback march is counted, and the dependent rounds of the path (those of the
+// certificate, the longest probe, the fallback march) separately.  The certificate
+// counts as a whole: where a sample fails, those of the rounds after it are not read.
 
 #define RL_SG_F 64    // Fourier features
 #define RL_SG_NF 32   // frequencies
@@ -279,8 +280,9 @@ __global__ void k_sg_features(const float4* __restrict__ rays, const float* __re
 // of k_sg_features followed by the per-layer GEMMs: the same feature
 // expression, the same matrix instructions over k in the same ascending order
 // from zero accumulators (16x16x32, whose bits are those of the two 16x16x16
-// instructions of k_gemm_bf16), the same bias / relu / bf16 epilogue.  Each row's outputs depend on that row alone, so the
-// rows past n (zero features) are computed and never stored.
+// instructions of k_gemm_bf16), the same bias / relu / bf16 epilogue (but for the sign
+// of a zero and of a NaN).  Each row's outputs depend on that row alone, so the rows
+// past n (zero features) are computed and never stored.
 #define RL_SG_TM 64
 #define RL_SG_ACT_PAD (RL_SG_H + 8)  // row stride in elements: 16-byte reads of 16 rows spread over the banks
 
@@ -373,9 +375,10 @@ __device__ __forceinline__ void sg_hidden_layer(bf16_t* act, const bf16_t* __res
 // the weights in SgFrag order;
 // out: n x 2 fp32.  Launched with ceil(n / 64) workgroups of 256 threads.
 // Register use is held to 128 so that four waves share each SIMD (three: 91 us
-// for 240,000 rays, four: 81; 128 rays per workgroup: 107).  81 us are 0.88
-// PFLOP/s; a 8192^3 bf16 product reaches 1.19 on this card.  Without the weight
-// loads it takes 72 us, without the features 78.
+// for 240,000 rays, four: 81; 128 rays per workgroup: 107).  With relu in fp32, which
+// keeps NaNs, it takes 83: 0.86 PFLOP/s, the matrix cores busy 46% and LDS 50% of it; a
+// 8192^3 bf16 product reaches 1.19 on this card.  (Of the 81 us, without the weight
+// loads 72, without the features 78.)
 __global__ __launch_bounds__(256, 4) void k_sg_infer(const float4* __restrict__ rays, const float* __restrict__ freq,
                                                   float inv_w, float inv_h, const bf16_t* __restrict__ P,
                                                   const bf16_t* __restrict__ F, const float* __restrict__ Pf,
@@ -757,7 +760,7 @@ int sg_reserve_train(rl_surrogate* s, int n, size_t partials) {
 }
 
 // The NT kernel applies when both operands are K-contiguous with 16-byte
-// aligned rows, the output is dense row-major and nothing is masked.
+// aligned rows and the output is dense row-major.
 bool nt_ok(const GemmArgs& g) {
   return g.sak == 1 && g.sbk == 1 && g.sam == g.K && g.sbn == g.K && g.K % 32 == 0 && g.N % 128 == 0 &&
          g.scn == 1 && g.scm == g.N && ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;
@@ -1112,7 +1115,8 @@ int rl_surrogate_train(rl_surrogate* s, float max_range, long long n_pairs, int 
 // Checked surrogate cast of a particle batch (numpy_calc_range_angles
 // semantics for inputs and outputs; ranges approximate, see file comment).
 // stats (host, 5 entries): fallbacks (bound), fallbacks (check), rays finished
-// from the surrogate's start point, distance-map reads, dependent read rounds.
+// from the surrogate's start point, distance-map reads, dependent read rounds (as
+// counted there).
 int rl_surrogate_calc_range_angles_dev(rl_surrogate* s, float max_range, const float* d_ins,
                                        const float* d_angles, float* d_ranges, int N, int M, float bound_max,
                                        unsigned* stats) {

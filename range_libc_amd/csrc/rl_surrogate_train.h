@@ -16,7 +16,8 @@
 // turn, and do not depend on which operand comes first: no difference in
 // 512,000 random tiles over 14 binades); weight gradients in slices of
 // sg_split(n).kchunk rows, added in slice order; bias gradients row by row in
-// chunks of sg_split(n).cchunk rows, added in chunk order.
+// chunks of sg_split(n).cchunk rows, added in chunk order; the loss in a tree over each
+// workgroup's 64 rays, whose sums the host adds in order.
 
 #define RL_SGT_ROWS 64    // rays per workgroup of k_sg_fwd_bwd
 #define RL_SGT_RT (RL_SGT_ROWS / 16)
