@@ -927,8 +927,10 @@ __device__ __forceinline__ void pool_particles(const MapDev& m, const float* lut
       // a NaN direction (NaN or infinite heading) ends at max_range: its first
       // step leaves the map, and a hit at its origin is not taken
       const bool nan = dx != dx || dy != dy;
-      ray[r].x = nan ? -4e9f : dx;
-      ray[r].y = nan ? __int_as_float(0x7fc00000) : dy;
+      // (of a heading beyond the reduction's range they may be infinite, and 0 * dx at
+      // the origin a NaN: any direction of 4e9 leaves the map with its first step)
+      ray[r].x = nan ? -4e9f : __builtin_amdgcn_fmed3f(dx, -4e9f, 4e9f);
+      ray[r].y = nan ? __int_as_float(0x7fc00000) : __builtin_amdgcn_fmed3f(dy, -4e9f, 4e9f);
     }
     wave_lds_sync();
     rl::pool_march(

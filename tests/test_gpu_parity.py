@@ -575,6 +575,37 @@ def test_pooled_rays_at_the_rules_lines(n, m, rect_map):
     test_pooled_rays(n, m, 300.0, None, rect_map)
 
 
+@pytest.mark.parametrize("n,m", [(6500, 60), (20_000, 60), (2000, 200)])
+def test_pooled_rays_of_huge_headings(n, m, rect_map):
+    """Headings past any reduction, whose direction is not finite: a ray that starts on
+    an occupied cell ends there and one that starts off the map at max_range, whatever
+    its heading, from pools as one ray per lane."""
+    torch = _torch()
+    ctx = rl.default_context(0)
+    R = 300.0
+    ins = W.world_poses(rect_map, n, seed=5)
+    y, x = np.nonzero(rect_map)
+    k = np.arange(0, n, 7)
+    at = np.random.default_rng(3).integers(0, x.size, k.size)
+    ins[k, 0], ins[k, 1] = y[at] + 0.75, x[at] + 0.25
+    ins[k[::5], 1] = -3.5
+    ins[k, 2] = np.resize(np.array([3e38, -3e38, 1e30, -1e25, 1e20, 3.4e38], np.float32), k.size)
+    ang = W.beam_angles(m)
+    dm = rl.DeviceMap(ctx, O.xmajor(rect_map))
+    d = [torch.from_numpy(v).cuda() for v in (ins, ang)]
+    out = torch.zeros(n * m, dtype=torch.float32, device="cuda")
+    dm.numpy_calc_range_angles_dev(rl.RL_METHOD_RM, R, d[0].data_ptr(), d[1].data_ptr(), out.data_ptr(), n, m)
+    one = torch.zeros_like(out)
+    for a in range(0, n, 3000):  # launches of one ray per lane
+        c = min(3000, n - a)
+        dm.numpy_calc_range_angles_dev(rl.RL_METHOD_RM, R, d[0][a:].data_ptr(), d[1].data_ptr(), one[a * m:].data_ptr(), c, m)
+    ctx.sync()
+    want = O.Oracle(rect_map, R, "rm").numpy_calc_range_angles(ins, ang).reshape(n, m)
+    got = out.cpu().numpy().reshape(n, m)
+    assert_bits_equal(got[k], want[k], "huge headings")
+    assert_bits_equal(got, one.cpu().numpy().reshape(n, m), "pools and one ray per lane")
+
+
 @pytest.mark.parametrize("xcd,box", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_scheduling_options(xcd, box, corridor_map):
     """XCD-aware scheduling and LDS staging change only where data is read from."""
